@@ -306,6 +306,42 @@ def test_quantize_bit_exact_f32(dev, oracle, bits):
     assert np.array_equal(from_dev_bf16(bi2), oracle.f32_to_bf16(rb2))
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("gs", [32, 64, 128])
+@pytest.mark.parametrize("bits", [2, 4, 8])
+def test_quantize_edges_bit_exact(dev, oracle, dtype, bits, gs):
+    """Groups that decide a code on a half step, constant, tiny (the scale's floor), huge and one-sided groups, over
+    a count of 8-value chunks that ends inside a workgroup: codes, scales and biases equal the oracle's.  The same
+    values with NaN and infinities among them, from an address that the wide loads cannot take, equal the aligned
+    call's bits."""
+    import torch
+
+    rng = np.random.default_rng(bits * gs + len(dtype))
+    N, K = 37, 3 * 128
+    wf = (rng.standard_normal((N, K)) * 0.02).astype(np.float32)
+    wf[0:4] = np.round(rng.uniform(-7, 8, (4, K))) * 0.5  # multiples of half a step
+    wf[0:4, ::gs] = 2.0**bits - 1.0
+    wf[4] = 0.0
+    wf[5] = 0.25
+    wf[6] = -0.25
+    wf[7] *= 1e-9
+    wf[8] *= 1e34
+    wf[9] = np.abs(wf[9]) + 0.1
+    wf[10] = -np.abs(wf[10]) - 0.1
+    wt = torch.from_numpy(wf).to(torch.bfloat16 if dtype == "bf16" else torch.float32)
+    wq, sc, bi = ops.quantize(wt.to(dev), gs, bits)
+    rq, rs, rb = oracle.quantize_f32(wt.float().numpy(), gs, bits)
+    assert np.array_equal(wq.cpu().numpy().view(np.uint32), rq)
+    assert torch.equal(sc.cpu(), torch.from_numpy(rs).to(wt.dtype))
+    assert torch.equal(bi.cpu(), torch.from_numpy(rb).to(wt.dtype))
+    wt[11, 5], wt[12, 9], wt[13, 70] = float("nan"), float("inf"), float("-inf")
+    buf = torch.empty(N * K + 1, dtype=wt.dtype, device=dev)
+    off = buf[1:].view(N, K)  # one element past a 16-byte boundary
+    off.copy_(wt)
+    for a, b in zip(ops.quantize(wt.to(dev), gs, bits), ops.quantize(off, gs, bits)):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
 def test_quantize_then_matmul_smoke(dev):
     """smoke.rs:19-40 with our ops: quantize -> quantized_matmul vs dequantize -> matmul (max |d| < 0.1)."""
     import torch
