@@ -110,11 +110,14 @@ LISAQ_API int lisaq_quantized_matmul(void* stream, const void* x, const uint32_t
  * the matvec arithmetic (f32, per-group scale*sum(x*q) + bias*sum(x),
  * QM:767-830, 996-1088), larger M the matmul arithmetic (weights rounded to T
  * from an f32 fma, f32 accumulation, QM:585-703, 1208-1326); y rounded to T
- * once.  Those paths use no workspace: the matvec one wave per output row
- * (x staged in LDS for f32 and from four rows on; f16 with 4-bit codes
- * through dot instructions), the matmul on the matrix cores for
- * bf16/f16 (64 x 64 or 128 x 128 tiles; x 16-byte aligned, else and for f32
- * 64 x 64 f32-FMA tiles). */
+ * once.  The matvec: one wave per output row (x staged in LDS for f32 and
+ * from four rows on; f16 with 4-bit codes through dot instructions).  The
+ * matmul: the bf16 2/4-bit matmul's kernel for bf16 and f16 where K is a
+ * multiple of 64 and of two groups and the tensors are aligned for it (x and w
+ * 16 bytes, the others 4), which splits K in a workspace of
+ * lisaq_quantized_matmul_workspace bytes (256-byte aligned; without it the
+ * call runs unsplit); else matrix-core tiles of 64 x 64 or 128 x 128 (x
+ * 16-byte aligned) and, for f32, 64 x 64 f32-FMA tiles, without a workspace. */
 LISAQ_API int lisaq_quantized_matmul_typed(void* stream, const void* x, const uint32_t* w, const void* scales,
                                            const void* biases, void* y, int64_t M, int64_t N, int64_t K,
                                            int transpose, int group_size, int bits, int dtype, void* workspace,

@@ -151,7 +151,8 @@ static int run_qmv(hipStream_t st, const QmvConfig& c, const void* x, const uint
 }
 
 static int run_qmm(hipStream_t st, const void* x, const uint32_t* w, const void* s, const void* b, void* y,
-                   int64_t M, int64_t N, int64_t K, int gs, int bits, void* ws, size_t ws_bytes) {
+                   int64_t M, int64_t N, int64_t K, int gs, int bits, void* ws, size_t ws_bytes,
+                   int ct = LISAQ_DTYPE_BF16) {
   LISAQ_REQUIRE(K % 64 == 0, LISAQ_EUNSUPPORTED, "qmm: K=%lld must be a multiple of 64", (long long)K);
   const QmmConfig c = qmm_config(M, N, K, gs, bits);
   QmmParams p{};
@@ -166,7 +167,7 @@ static int run_qmm(hipStream_t st, const void* x, const uint32_t* w, const void*
   p.K = (int)K;
   p.G = (int)(K / gs);
   if (ws) LISAQ_REQUIRE(aligned(ws, 256), LISAQ_EINVAL_LAYOUT, "qmm: workspace must be 256-byte aligned");
-  return qmm_launch(st, c, p, bits, gs, c.grid, 1, ws, ws_bytes);
+  return qmm_launch(st, c, p, bits, gs, c.grid, 1, ws, ws_bytes, ct);
 }
 
 // Gather workspace layout: [counts 256 B][matvec table 0][matvec table 1]
@@ -618,10 +619,20 @@ int lisaq_quantized_matmul_typed(void* stream, const void* x, const uint32_t* w,
   LISAQ_REQUIRE(x && w && s && y, LISAQ_EINVAL_LAYOUT, "quantized_matmul_typed: null tensor pointer");
   LISAQ_REQUIRE(aligned(x, el) && aligned(y, el) && aligned(s, el) && aligned(b, el) && aligned(w, 4),
                 LISAQ_EINVAL_LAYOUT, "quantized_matmul_typed: misaligned tensor");
-  (void)ws;
-  (void)ws_bytes;
-  return launch_typed_mm((hipStream_t)stream, M < lisaq_qmv_batch_limit(K, N), x, w, s, b, y, M, N, K, gs, bits,
-                         dtype);
+  const bool matvec = M < lisaq_qmv_batch_limit(K, N);
+  // f16 and 8-bit matmuls on the bf16 matmul's kernel (measured, f16 4-bit
+  // 1000 x 5120 x 5120: 217 us on qmm_typed_mfma_kernel, 69 us here).  Its
+  // scale/bias copies are 16 bytes of a row at dword granularity, so rows of
+  // an even number of groups from a dword on; other rows and addresses, and
+  // sizes past its 32-bit offsets, stay on the kernels of qtyped.hip.
+  if (!matvec && dtype != LISAQ_DTYPE_F32 && K % 64 == 0 && K / gs % 2 == 0 && aligned(x, 16) && aligned(w, 16) &&
+      aligned(s, 4) && aligned(b, 4) && aligned(y, 4) && M * K < ((int64_t)1 << 31) &&
+      N * K * bits / 8 < ((int64_t)1 << 32)) {
+    const bool room = ws != nullptr && aligned(ws, 256);
+    return run_qmm((hipStream_t)stream, x, w, s, b, y, M, N, K, gs, bits, room ? ws : nullptr, room ? ws_bytes : 0,
+                   dtype);
+  }
+  return launch_typed_mm((hipStream_t)stream, matvec, x, w, s, b, y, M, N, K, gs, bits, dtype);
 }
 
 int lisaq_quantized_matmul_noalloc(void* stream, const void* x, const uint32_t* w, const void* s, const void* b,

@@ -34,9 +34,10 @@ struct QmmConfig {
 
 QmmConfig qmm_config(int64_t M, int64_t N, int64_t K, int gs, int bits, bool allow_split = true);
 // Enqueue.  A plain launch whose config splits K uses ws (>= c.ws_bytes) for
-// the partials, or runs unsplit when ws is missing or too small.
+// the partials, or runs unsplit when ws is missing or too small.  ct: compute
+// type, LISAQ_DTYPE_BF16 or LISAQ_DTYPE_F16.
 int qmm_launch(hipStream_t stream, const QmmConfig& c, QmmParams p, int bits, int gs, int grid_x,
-               int grid_y, void* ws = nullptr, size_t ws_bytes = 0);
+               int grid_y, void* ws = nullptr, size_t ws_bytes = 0, int ct = LISAQ_DTYPE_BF16);
 
 // Gate|up matmul of the MoE prefill: tile-table launch of `grid` workgroups,
 // y = SwiGLU(x . gate^T, x . up^T) over 128-column output tiles of 128 rows,

@@ -6,9 +6,10 @@
 
 namespace lisaq {
 
-// Remainder tiles of a hybrid launch: y = bf16(sum over the S parts), parts
+// Remainder tiles of a hybrid launch: y = T(sum over the S parts), parts
 // added in order; unit (r, s) holds tile full_tiles + r's [BM][BN] partial.
 // Four consecutive columns per thread (16-byte part loads).
+template <int CT>
 __global__ __launch_bounds__(256) void qmm_hybrid_reduce_kernel(const float* __restrict__ part,
                                                                 uint16_t* __restrict__ y, int M, int N, int BM,
                                                                 int BN, int gn, int full_tiles, int S,
@@ -32,22 +33,22 @@ __global__ __launch_bounds__(256) void qmm_hybrid_reduce_kernel(const float* __r
   }
   uint16_t* dst = y + (int64_t)m * N + n;
   if (n + 3 < N && (N & 3) == 0) {
-    *reinterpret_cast<u32x2*>(dst) = u32x2{pack_bf2(v[0], v[1]),
-                                           pack_bf2(v[2], v[3])};
+    *reinterpret_cast<u32x2*>(dst) = u32x2{Ct<CT>::pk(v[0], v[1]), Ct<CT>::pk(v[2], v[3])};
   } else {
     for (int c = 0; c < 4; ++c)
-      if (n + c < N) dst[c] = f2bf(v[c]);
+      if (n + c < N) dst[c] = Ct<CT>::one(v[c]);
   }
 }
 
-// y = bf16(sum over the splits of the f32 partials), splits added in order.
+// y = T(sum over the splits of the f32 partials), splits added in order.
+template <int CT>
 __global__ __launch_bounds__(256) void qmm_split_reduce_kernel(const float* __restrict__ part,
                                                                uint16_t* __restrict__ y, int64_t MN, int S) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i >= MN) return;
   float v = part[i];
   for (int s = 1; s < S; ++s) v += part[(int64_t)s * MN + i];
-  y[i] = f2bf(v);
+  y[i] = Ct<CT>::one(v);
 }
 
 // ---------------------------------------------------------------------------
@@ -61,6 +62,7 @@ QmmConfig qmm_config(int64_t M, int64_t N, int64_t K, int gs, int bits, bool all
     const int64_t gn = (N + 255) / 256;
     int64_t best = -1;
     for (int mt : {8, 6, 4}) {
+      if (mt == 8 && bits == 8) continue;  // (its LDS ring does not fit)
       const int64_t tiles = gn * ((M + 32 * mt - 1) / (32 * mt));
       const int64_t cost = (tiles + 255) / 256 * 32 * mt;
       if (best < 0 || cost < best) {
@@ -77,7 +79,7 @@ QmmConfig qmm_config(int64_t M, int64_t N, int64_t K, int gs, int bits, bool all
   bool hybrid = false;
   {
     const int64_t t8 = ((N + 255) / 256) * ((M + 255) / 256);
-    if (allow_split && tune_int("LISAQ_QMM_HYBRID", 1) && t8 >= 256 && t8 % 256 != 0 && nk >= 16) {
+    if (allow_split && tune_int("LISAQ_QMM_HYBRID", 1) && t8 >= 256 && t8 % 256 != 0 && nk >= 16 && bits != 8) {
       c.MT = 8;
       hybrid = true;
     }
@@ -131,25 +133,31 @@ QmmConfig qmm_config(int64_t M, int64_t N, int64_t K, int gs, int bits, bool all
   }
   c.ws_bytes = c.S > 1 ? (size_t)c.S * M * N * 4 : 0;
   (void)gs;
-  (void)bits;
   return c;
 }
 
 template <bool SPLIT>
-static qmm_fn qmm_pick(const QmmConfig& c, int bits, int gs, int* lds) {
-  if (bits == 4) return qmm_get<4, SPLIT>(gs, c.MT, lds);
-  if (bits == 2) return qmm_get<2, SPLIT>(gs, c.MT, lds);
+static qmm_fn qmm_pick(const QmmConfig& c, int bits, int gs, int ct, int* lds) {
+  if (ct == kCtBf16) {
+    if (bits == 4) return qmm_get<4, SPLIT>(gs, c.MT, lds);
+    if (bits == 2) return qmm_get<2, SPLIT>(gs, c.MT, lds);
+    if (bits == 8) return qmm_get<8, SPLIT>(gs, c.MT, lds);
+  } else if (ct == kCtF16) {
+    if (bits == 4) return qmm_get<4, SPLIT, kCtF16>(gs, c.MT, lds);
+    if (bits == 2) return qmm_get<2, SPLIT, kCtF16>(gs, c.MT, lds);
+    if (bits == 8) return qmm_get<8, SPLIT, kCtF16>(gs, c.MT, lds);
+  }
   return nullptr;
 }
 
 int qmm_launch(hipStream_t stream, const QmmConfig& c, QmmParams p, int bits, int gs, int grid_x,
-               int grid_y, void* ws, size_t ws_bytes) {
+               int grid_y, void* ws, size_t ws_bytes, int ct) {
   // split over K only for plain launches with room for the partials (else the
   // configuration without any split)
   const bool split = !p.tiles && c.S > 1 && ws != nullptr && ws_bytes >= c.ws_bytes;
   if (!p.tiles && c.S > 1 && !split) {
     const QmmConfig c1 = qmm_config(p.M, p.N, p.K, gs, bits, false);
-    return qmm_launch(stream, c1, p, bits, gs, c1.grid, grid_y, nullptr, 0);
+    return qmm_launch(stream, c1, p, bits, gs, c1.grid, grid_y, nullptr, 0, ct);
   }
   LISAQ_REQUIRE((int64_t)p.M * p.K < ((int64_t)1 << 31), LISAQ_EINVAL_SHAPE, "qmm: x larger than 2^31 elements");
   LISAQ_REQUIRE((int64_t)p.N * p.K * bits / 8 < ((int64_t)1 << 32), LISAQ_EINVAL_SHAPE,
@@ -160,7 +168,7 @@ int qmm_launch(hipStream_t stream, const QmmConfig& c, QmmParams p, int bits, in
     return set_error(LISAQ_EUNSUPPORTED, "qmm: split over K with %d-row tiles (%s layout) is not built", 32 * c.MT,
                      c.full_tiles > 0 ? "hybrid" : "per-part");
   int lds = 0;
-  qmm_fn fn = split ? qmm_pick<true>(c, bits, gs, &lds) : qmm_pick<false>(c, bits, gs, &lds);
+  qmm_fn fn = split ? qmm_pick<true>(c, bits, gs, ct, &lds) : qmm_pick<false>(c, bits, gs, ct, &lds);
   if (!fn) return set_error(LISAQ_EUNSUPPORTED, "qmm: bits=%d group_size=%d not supported", bits, gs);
   if (int rc = allow_dyn_lds((const void*)fn, lds, "qmm")) return rc;
   p.ksplit = split ? c.S : 1;
@@ -172,12 +180,12 @@ int qmm_launch(hipStream_t stream, const QmmConfig& c, QmmParams p, int bits, in
   if (rc || !split) return rc;
   if (c.full_tiles > 0) {
     const int64_t count4 = (int64_t)(grid_x - c.full_tiles) * c.BM * c.BN / 4;
-    hipLaunchKernelGGL(qmm_hybrid_reduce_kernel, dim3((unsigned)((count4 + 255) / 256)), dim3(256), 0, stream,
+    hipLaunchKernelGGL(ct == kCtF16 ? qmm_hybrid_reduce_kernel<kCtF16> : qmm_hybrid_reduce_kernel<kCtBf16>, dim3((unsigned)((count4 + 255) / 256)), dim3(256), 0, stream,
                        (const float*)p.partial, p.y, p.M, p.N, c.BM, c.BN, c.grid_n, c.full_tiles, c.S, count4);
     return check_launch("qmm_hybrid_reduce");
   }
   const int64_t MN = (int64_t)p.M * p.N;
-  hipLaunchKernelGGL(qmm_split_reduce_kernel, dim3((unsigned)((MN + 255) / 256)), dim3(256), 0, stream,
+  hipLaunchKernelGGL(ct == kCtF16 ? qmm_split_reduce_kernel<kCtF16> : qmm_split_reduce_kernel<kCtBf16>, dim3((unsigned)((MN + 255) / 256)), dim3(256), 0, stream,
                      (const float*)p.partial, p.y, MN, c.S);
   return check_launch("qmm_split_reduce");
 }

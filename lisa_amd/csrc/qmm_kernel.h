@@ -18,6 +18,10 @@
 //    with the group's scale/bias, v_cvt_pk_bf16_f32.
 //  * The next K-step's x tile and W words are fetched while the current one
 //    runs on the matrix cores.
+// Compute types: bf16 and f16 (CT), 2-, 4- and 8-bit codes.  f16 weights are one
+// v_fma_mixlo/mixhi_f16 per code after the unpack, bf16 ones an fma and half
+// a pack: f16 4-bit 1000 x 5120 x 5120 takes 69 us (758 TFLOP/s; on the
+// separate 64 x 64 typed tiles 217 us), bf16 8-bit 73 us.
 #pragma once
 #include "lisaq_common.h"
 #include "qmm.h"
@@ -35,11 +39,6 @@ __device__ __forceinline__ uint32_t pk_bf16(float a, float b) {
   return __builtin_bit_cast(uint32_t, v);
 }
 
-// Byte I of a word as f32: one v_cvt_f32_ubyte<I>.
-template <int I>
-__device__ __forceinline__ float ubyte_f32(uint32_t v) {
-  return (float)((v >> (8 * I)) & 0xFFu);
-}
 // A word of masked codes made opaque to the optimizer, which would otherwise
 // fold the mask into each byte extraction (v_bfe + v_cvt_f32_ubyte0 instead
 // of one v_cvt_f32_ubyte<I>).
@@ -49,13 +48,44 @@ __device__ __forceinline__ uint32_t opaque(uint32_t v) {
 }
 
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
+
+// Compute type of a matmul (x, scales, biases, the rounded weights and y):
+// bf16 or f16, both on v_mfma_f32_32x32x16 with f32 accumulators.
+constexpr int kCtBf16 = LISAQ_DTYPE_BF16, kCtF16 = LISAQ_DTYPE_F16;
+template <int CT>
+struct Ct;
+template <>
+struct Ct<kCtBf16> {
+  static __device__ __forceinline__ float f(uint16_t h) { return bf2f(h); }
+  static __device__ __forceinline__ uint32_t pk(float a, float b) { return pk_bf16(a, b); }
+  static __device__ __forceinline__ uint16_t one(float v) { return f2bf(v); }
+  static __device__ __forceinline__ f32x16 mfma(u32x4 a, u32x4 b, f32x16 c) {
+    return mfma32x32x16(as_bf16x8(a), as_bf16x8(b), c);
+  }
+};
+template <>
+struct Ct<kCtF16> {
+  static __device__ __forceinline__ float f(uint16_t h) { return (float)__builtin_bit_cast(_Float16, h); }
+  static __device__ __forceinline__ uint32_t pk(float a, float b) {
+    return __builtin_bit_cast(uint32_t, f16x2_t{(_Float16)a, (_Float16)b});
+  }
+  static __device__ __forceinline__ uint16_t one(float v) { return __builtin_bit_cast(uint16_t, (_Float16)v); }
+  static __device__ __forceinline__ f32x16 mfma(u32x4 a, u32x4 b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c,
+                                                  0, 0, 0);
+  }
+};
+
 // Two weights bf16(fma(s, q, b)) from a register whose halves hold the two
 // codes as f16 denormals (value q * 2^-24): with s24 = s * 2^24 (exact),
 // v_fma_mix_f32 forms s24 * (q * 2^-24) + b, whose product equals s * q
 // exactly, so each result is fmaf(s, q, b) bit for bit (|s| < 2^104).
+// (f16 weights: the fma and its rounding are one v_fma_mixlo/mixhi_f16 each.)
+template <int CT = kCtBf16>
 __device__ __forceinline__ uint32_t deq_pair(uint32_t pair, float s24, float b) {
   const f16x2_t hv = __builtin_bit_cast(f16x2_t, pair);
-  return pk_bf16(fmaf(s24, (float)hv[0], b), fmaf(s24, (float)hv[1], b));
+  return Ct<CT>::pk(fmaf(s24, (float)hv[0], b), fmaf(s24, (float)hv[1], b));
 }
 // The two codes in byte I of lo and byte I of hi, each into one half.
 template <int I>
@@ -63,30 +93,10 @@ __device__ __forceinline__ uint32_t pair_bytes(uint32_t lo, uint32_t hi) {
   return __builtin_amdgcn_perm(hi, lo, (0x0Cu << 24) | ((4u + I) << 16) | (0x0Cu << 8) | (uint32_t)I);
 }
 
-// Dequantize the 8 codes of one u32 (4-bit) into 4 bf16x2 in natural K order.
-__device__ __forceinline__ void deq4(uint32_t w, float s, float b, uint32_t* o) {
-  const uint32_t lo = opaque(w & 0x0F0F0F0Fu);         // codes 0,2,4,6
-  const uint32_t hi = opaque((w >> 4) & 0x0F0F0F0Fu);  // codes 1,3,5,7
-  o[0] = pk_bf16(fmaf(s, ubyte_f32<0>(lo), b), fmaf(s, ubyte_f32<0>(hi), b));
-  o[1] = pk_bf16(fmaf(s, ubyte_f32<1>(lo), b), fmaf(s, ubyte_f32<1>(hi), b));
-  o[2] = pk_bf16(fmaf(s, ubyte_f32<2>(lo), b), fmaf(s, ubyte_f32<2>(hi), b));
-  o[3] = pk_bf16(fmaf(s, ubyte_f32<3>(lo), b), fmaf(s, ubyte_f32<3>(hi), b));
-}
-
-// Dequantize the 16 codes of one u32 (2-bit) into 8 bf16x2 in natural K order.
-__device__ __forceinline__ void deq2(uint32_t w, float s, float b, uint32_t* o) {
-  const uint32_t c0 = opaque(w & 0x03030303u);         // codes 0,4,8,12
-  const uint32_t c1 = opaque((w >> 2) & 0x03030303u);  // codes 1,5,9,13
-  const uint32_t c2 = opaque((w >> 4) & 0x03030303u);  // codes 2,6,10,14
-  const uint32_t c3 = opaque((w >> 6) & 0x03030303u);  // codes 3,7,11,15
-  o[0] = pk_bf16(fmaf(s, ubyte_f32<0>(c0), b), fmaf(s, ubyte_f32<0>(c1), b));
-  o[1] = pk_bf16(fmaf(s, ubyte_f32<0>(c2), b), fmaf(s, ubyte_f32<0>(c3), b));
-  o[2] = pk_bf16(fmaf(s, ubyte_f32<1>(c0), b), fmaf(s, ubyte_f32<1>(c1), b));
-  o[3] = pk_bf16(fmaf(s, ubyte_f32<1>(c2), b), fmaf(s, ubyte_f32<1>(c3), b));
-  o[4] = pk_bf16(fmaf(s, ubyte_f32<2>(c0), b), fmaf(s, ubyte_f32<2>(c1), b));
-  o[5] = pk_bf16(fmaf(s, ubyte_f32<2>(c2), b), fmaf(s, ubyte_f32<2>(c3), b));
-  o[6] = pk_bf16(fmaf(s, ubyte_f32<3>(c0), b), fmaf(s, ubyte_f32<3>(c1), b));
-  o[7] = pk_bf16(fmaf(s, ubyte_f32<3>(c2), b), fmaf(s, ubyte_f32<3>(c3), b));
+// Codes 2 I and 2 I + 1 of a word of 8-bit codes, each into one half.
+template <int I>
+__device__ __forceinline__ uint32_t pair_code8(uint32_t w) {
+  return __builtin_amdgcn_perm(0u, w, (0x0Cu << 24) | ((2u * I + 1u) << 16) | (0x0Cu << 8) | (2u * I));
 }
 
 template <typename F, int... I>
@@ -128,6 +138,12 @@ __device__ __forceinline__ int w_swz(int row) { return ((row >> 2) ^ (row >> 3))
 // on 8 distinct 16-byte groups of a 128-byte line and any 16 on 16 distinct
 // groups of a 256-byte line.
 __device__ __forceinline__ int w_swz2(int row) { return ((row >> 1) ^ (row >> 3)) & 3; }
+// 8-bit codes: 128 bytes per row and pair, eight chunks, swizzled as the x
+// rows (which have the same length).
+template <int BITS>
+__device__ __forceinline__ int w_chunk_swz(int row) {
+  return BITS == 8 ? x_swz(row) : BITS == 4 ? w_swz2(row) : 0;
+}
 
 // 16 / 4 / 2 bytes per lane from global memory straight into LDS (lane l
 // writes lds + size*l; lds must be wave-uniform).
@@ -217,10 +233,12 @@ struct QmmLds {
 //
 // WM: waves along M (WN x WM waves, each MT x 32 rows by NT x 32 columns).
 template <int BITS, int GS, int MT, int NT, int WN, bool SPLIT, bool GU = false, int NB = 3, bool SKIP = GU,
-          int WM = 1>
+          int WM = 1, int CT = kCtBf16>
 __global__ __launch_bounds__(64 * WN * WM) void qmm_kernel(QmmParams p) {
   using G = MGeo<BITS>;
+  using C = Ct<CT>;
   using L = QmmLds<BITS, GS, MT, NT, WN, NB, WM>;
+  static_assert(!GU || CT == kCtBf16, "SwiGLU epilogue: bf16 only");
   static_assert(WM == 1 || (!GU && !SKIP), "waves along M: plain tiles only");
   static_assert(NB == 3, "ring depth");
   constexpr int BM = L::BM;
@@ -370,9 +388,8 @@ __global__ __launch_bounds__(64 * WN * WM) void qmm_kernel(QmmParams p) {
     if (GU && rr >= BN / 2) rr -= BN / 2;
     int n = nt0 + rr;
     n = n < p.N ? n : p.N - 1;
-    // 4-bit: physical chunk (off / 16) % 4 of the row holds logical chunk
-    // physical ^ w_swz2(row)
-    const int lb = BITS == 4 ? (off % WROW) ^ (w_swz2(row) << 4) : off % WROW;
+    // physical chunk off / 16 of the row holds logical chunk physical ^ swizzle
+    const int lb = (off % WROW) ^ (w_chunk_swz<BITS>(row) << 4);
     wvo[i] = (uint32_t)n * rowbytes + (uint32_t)lb;
   }
   // scales / biases: blocks of 8 groups (SBK = GS / 8 K-steps), 16 bytes of
@@ -431,10 +448,11 @@ __global__ __launch_bounds__(64 * WN * WM) void qmm_kernel(QmmParams p) {
   };
 
   // ---- one K-step's W of this lane (LDS stage): packed words, scale, bias
-  typedef typename std::conditional<G::WPL == 4, u32x4, u32x2>::type WV;
+  constexpr int WCH = BITS == 8 ? 2 : 1;  // reads of a lane's 32 codes: 16 bytes each (2-bit: 8)
+  typedef typename std::conditional<BITS == 2, u32x2, u32x4>::type WV;
   struct WLane {
-    WV w[NT];
-    uint16_t s[NT], b[NT];  // raw bf16 bits (converted where used)
+    WV w[NT][WCH];
+    uint16_t s[NT], b[NT];  // raw bits of the compute type (converted where used)
   };
   // W of local step kl (clamped to the last step) from its pair buffer
   auto read_w = [&](int kl, WLane& o) {
@@ -449,22 +467,48 @@ __global__ __launch_bounds__(64 * WN * WM) void qmm_kernel(QmmParams p) {
       const int r = (wn * NT + nt) * 32 + col;
       o.s[nt] = *reinterpret_cast<const uint16_t*>(sbb + r * 16);
       o.b[nt] = *reinterpret_cast<const uint16_t*>(sbb + L::SBA + r * 16);
-      const int pc = BITS == 4 ? (2 * e + h) ^ w_swz2(r) : 2 * e + h;  // physical chunk (2-bit: 8 bytes)
-      o.w[nt] = *reinterpret_cast<const WV*>(st + r * WROW + pc * (4 * G::WPL));
+#pragma unroll
+      for (int q = 0; q < WCH; ++q) {
+        const int pc = (WCH * (2 * e + h) + q) ^ w_chunk_swz<BITS>(r);  // physical chunk (2-bit: 8 bytes)
+        o.w[nt][q] = *reinterpret_cast<const WV*>(st + r * WROW + pc * (int)sizeof(WV));
+      }
     }
   };
   // s, b as f32 for one column tile of a W lane
-  auto sf = [&](const WLane& r, int nt) { return bf2f(r.s[nt]); };
-  auto bf = [&](const WLane& r, int nt) { return bf2f(r.b[nt]); };
-  // dequantize all words of a W lane into B operands [nt][16] bf16x2
+  auto sf = [&](const WLane& r, int nt) { return C::f(r.s[nt]); };
+  auto bf = [&](const WLane& r, int nt) { return C::f(r.b[nt]); };
+  // word dw of a lane's codes
+  auto word = [&](const WLane& r, int nt, int dw) -> uint32_t {
+    return BITS == 8 ? r.w[nt][dw >> 2][dw & 3] : r.w[nt][0][dw];
+  };
+  // dequantize all words of a W lane into B operands [nt][16] pairs
   auto dequant_all = [&](const WLane& r, uint32_t (*bop)[16]) {
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
+    for (int nt = 0; nt < NT; ++nt) {
+      const float s24 = sf(r, nt) * 16777216.0f, b_ = bf(r, nt);
+      static_for<G::WPL>([&](auto WI_) {
+        constexpr int jw = decltype(WI_)::value;
+        const uint32_t wv = word(r, nt, jw);
+        if constexpr (BITS == 8) {
+          bop[nt][jw * 2] = deq_pair<CT>(pair_code8<0>(wv), s24, b_);
+          bop[nt][jw * 2 + 1] = deq_pair<CT>(pair_code8<1>(wv), s24, b_);
+        } else if constexpr (BITS == 4) {
+          const uint32_t lo = opaque(wv & 0x0F0F0F0Fu), hi = opaque((wv >> 4) & 0x0F0F0F0Fu);
+          static_for<4>([&](auto PI) {
+            constexpr int d = decltype(PI)::value;
+            bop[nt][jw * 4 + d] = deq_pair<CT>(pair_bytes<d>(lo, hi), s24, b_);
+          });
+        } else {
+          uint32_t c[4];
 #pragma unroll
-      for (int jw = 0; jw < G::WPL; ++jw) {
-        if (BITS == 4) deq4(r.w[nt][jw], sf(r, nt), bf(r, nt), &bop[nt][jw * 4]);
-        else deq2(r.w[nt][jw], sf(r, nt), bf(r, nt), &bop[nt][jw * 8]);
-      }
+          for (int q = 0; q < 4; ++q) c[q] = opaque((wv >> (2 * q)) & 0x03030303u);
+          static_for<8>([&](auto PI) {
+            constexpr int d = decltype(PI)::value, m = d / 2, e = (d % 2) * 2;
+            bop[nt][jw * 8 + d] = deq_pair<CT>(pair_bytes<m>(c[e], c[e + 1]), s24, b_);
+          });
+        }
+      });
+    }
   };
 
   f32x16 acc[MT][NT];
@@ -536,7 +580,7 @@ __global__ __launch_bounds__(64 * WN * WM) void qmm_kernel(QmmParams p) {
   // Odd (local) steps also copy a W pair.
   constexpr int NMF = MT * NT;
   constexpr int SLOTS = 4 * NMF;
-  constexpr int PPW = BITS == 4 ? 4 : 8;             // dequant pieces per packed word
+  constexpr int PPW = 16 / BITS;                     // dequant pieces (pairs) per packed word
   constexpr int NPIECE = NT * G::WPL * PPW;          // dequant pieces per step
   static_assert(XI + WI <= 3 * NMF, "slot plan");  // (short tiles: several dequant pieces per slot)
   int xs = 0;  // x stage of step k
@@ -578,7 +622,7 @@ __global__ __launch_bounds__(64 * WN * WM) void qmm_kernel(QmmParams p) {
         const u32x4 bw = u32x4{bcur[nt][4 * j], bcur[nt][4 * j + 1], bcur[nt][4 * j + 2], bcur[nt][4 * j + 3]};
         // W as the row operand, x as the column operand: the accumulator is
         // y^T, so a lane holds runs of 4 consecutive outputs of one row
-        acc[mt][nt] = mfma32x32x16(as_bf16x8(bw), as_bf16x8(aw), acc[mt][nt]);
+        acc[mt][nt] = C::mfma(bw, aw, acc[mt][nt]);
       }
       __builtin_amdgcn_sched_barrier(0);
       // the W words of the step after next, first thing after the barrier (the
@@ -618,9 +662,11 @@ __global__ __launch_bounds__(64 * WN * WM) void qmm_kernel(QmmParams p) {
         constexpr int d = decltype(DI)::value;
         if constexpr (d * SLOTS / NPIECE == sl) {
           constexpr int dnt = d / (G::WPL * PPW), dw = d / PPW % G::WPL, dp = d % PPW;
-          const uint32_t wv = wn.w[dnt][dw];
+          const uint32_t wv = word(wn, dnt, dw);
           const float s_ = sf(wn, dnt), b_ = bf(wn, dnt);
-          if constexpr (BITS == 4) {
+          if constexpr (BITS == 8) {
+            bnxt[dnt][dw * 2 + dp] = opaque(deq_pair<CT>(pair_code8<dp>(wv), s_ * 16777216.0f, b_));
+          } else if constexpr (BITS == 4) {
             if constexpr (dp == 0) {
               lo[dnt][dw] = opaque(wv & 0x0F0F0F0Fu);
               hi[dnt][dw] = opaque((wv >> 4) & 0x0F0F0F0Fu);
@@ -630,14 +676,14 @@ __global__ __launch_bounds__(64 * WN * WM) void qmm_kernel(QmmParams p) {
             // (opaque: pinned to its slot -- a branch later in the step, such
             // as the conditional wait, otherwise lets the compiler sink the
             // pieces together next to it, out from under the matrix work)
-            bnxt[dnt][dw * 4 + dp] = opaque(deq_pair(pair_bytes<dp>(lo[dnt][dw], hi[dnt][dw]), s_ * 16777216.0f, b_));
+            bnxt[dnt][dw * 4 + dp] = opaque(deq_pair<CT>(pair_bytes<dp>(lo[dnt][dw], hi[dnt][dw]), s_ * 16777216.0f, b_));
           } else {
             if constexpr (dp == 0) {
 #pragma unroll
               for (int c = 0; c < 4; ++c) c4[dnt][dw][c] = opaque((wv >> (2 * c)) & 0x03030303u);
             }
             constexpr int m = dp / 2, e = (dp % 2) * 2;
-            bnxt[dnt][dw * 8 + dp] = opaque(deq_pair(pair_bytes<m>(c4[dnt][dw][e], c4[dnt][dw][e + 1]), s_ * 16777216.0f, b_));
+            bnxt[dnt][dw * 8 + dp] = opaque(deq_pair<CT>(pair_bytes<m>(c4[dnt][dw][e], c4[dnt][dw][e + 1]), s_ * 16777216.0f, b_));
           }
         }
       });
@@ -769,7 +815,7 @@ __global__ __launch_bounds__(64 * WN * WM) void qmm_kernel(QmmParams p) {
                 const f32x16& a = acc[mt][nt];
                 const int c = (wn * NT + nt) * 32 + 8 * g + 4 * h;
                 *reinterpret_cast<u32x2*>(ex + ((mt - hp * MTP) * 32 + col) * XSn + c) =
-                    u32x2{pk_bf16(a[4 * g], a[4 * g + 1]), pk_bf16(a[4 * g + 2], a[4 * g + 3])};
+                    u32x2{C::pk(a[4 * g], a[4 * g + 1]), C::pk(a[4 * g + 2], a[4 * g + 3])};
               }
         }
         wait_lgkm0();
@@ -789,9 +835,9 @@ __global__ __launch_bounds__(64 * WN * WM) void qmm_kernel(QmmParams p) {
   }
   if (whole) {
     store([&](int m, int n, float v0, float v1, float v2, float v3) {
-            *reinterpret_cast<u32x2*>(y + (int64_t)m * p.N + n) = u32x2{pk_bf16(v0, v1), pk_bf16(v2, v3)};
+            *reinterpret_cast<u32x2*>(y + (int64_t)m * p.N + n) = u32x2{C::pk(v0, v1), C::pk(v2, v3)};
           },
-          [&](int m, int n, float v) { y[(int64_t)m * p.N + n] = f2bf(v); });
+          [&](int m, int n, float v) { y[(int64_t)m * p.N + n] = C::one(v); });
   } else if constexpr (SPLIT) {
     if (unit >= 0) {
       // compact partial of one unit: [BM][BN] f32 at unit * BM * BN
@@ -812,37 +858,30 @@ __global__ __launch_bounds__(64 * WN * WM) void qmm_kernel(QmmParams p) {
 
 typedef void (*qmm_fn)(QmmParams);
 
-// Kernel of one (bits, split) quarter: qmm_k<bits>_<split>.hip instantiate the
+// Kernel of one (bits, split, compute type): qmm_k<bits>_<split>.hip (bf16) and
+// qmm_t<type><bits>.hip instantiate the
 // tile heights MT = 4, 6, 8 and group sizes 32, 64, 128 (eight waves, NT = 1),
-// so the four quarters compile in parallel.  *lds = dynamic LDS bytes.
-template <int BITS, bool SPLIT>
+// so the units compile in parallel.  *lds = dynamic LDS bytes.
+template <int BITS, bool SPLIT, int CT = kCtBf16>
 qmm_fn qmm_get(int gs, int MT, int* lds);
 
-template <int BITS, bool SPLIT>
+template <int BITS, bool SPLIT, int CT = kCtBf16>
 qmm_fn qmm_get_impl(int gs, int MT, int* lds) {
   auto one = [&](auto mt) -> qmm_fn {
     constexpr int M_ = decltype(mt)::value;
     *lds = QmmLds<BITS, 64, M_, 1, 8>::TOTAL;  // (group-size independent)
-    if (gs == 32) return qmm_kernel<BITS, 32, M_, 1, 8, SPLIT>;
-    if (gs == 64) return qmm_kernel<BITS, 64, M_, 1, 8, SPLIT>;
-    if (gs == 128) return qmm_kernel<BITS, 128, M_, 1, 8, SPLIT>;
+    if (gs == 32) return qmm_kernel<BITS, 32, M_, 1, 8, SPLIT, false, 3, false, 1, CT>;
+    if (gs == 64) return qmm_kernel<BITS, 64, M_, 1, 8, SPLIT, false, 3, false, 1, CT>;
+    if (gs == 128) return qmm_kernel<BITS, 128, M_, 1, 8, SPLIT, false, 3, false, 1, CT>;
     return nullptr;
   };
   // split launches exist in two layouts only: per-part partials [S][M][N]
   // with 128-row tiles (small grids) and the hybrid compact layout with
   // 256-row tiles; no other tile height is built with split output
-#ifdef LISAQ_TUNING
-  // 256 x 256 tiles as 2 x 4 waves of 128 rows x 64 columns (halves the x
-  // tile's LDS reads, doubles the dequantization per wave)
-  if (MT == 8 && tune_int("LISAQ_QMM_WM", 1) == 2) {
-    *lds = QmmLds<BITS, 64, 4, 2, 4, 3, 2>::TOTAL;
-    if (gs == 32) return qmm_kernel<BITS, 32, 4, 2, 4, SPLIT, false, 3, false, 2>;
-    if (gs == 64) return qmm_kernel<BITS, 64, 4, 2, 4, SPLIT, false, 3, false, 2>;
-    if (gs == 128) return qmm_kernel<BITS, 128, 4, 2, 4, SPLIT, false, 3, false, 2>;
-    return nullptr;
+  // (8-bit codes: the ring of 256-row tiles takes 176 KB)
+  if constexpr (BITS != 8) {
+    if (MT == 8) return one(std::integral_constant<int, 8>{});
   }
-#endif
-  if (MT == 8) return one(std::integral_constant<int, 8>{});
   if constexpr (!SPLIT) {
     if (MT == 6) return one(std::integral_constant<int, 6>{});
   }

@@ -1,0 +1,17 @@
+// Instantiations of the qmm kernel for f16 and 8-bit codes, with and without
+// split-K partial output (the kernel is in qmm_kernel.h).
+#include "qmm_kernel.h"
+
+namespace lisaq {
+
+template <>
+qmm_fn qmm_get<8, false, kCtF16>(int gs, int MT, int* lds) {
+  return qmm_get_impl<8, false, kCtF16>(gs, MT, lds);
+}
+
+template <>
+qmm_fn qmm_get<8, true, kCtF16>(int gs, int MT, int* lds) {
+  return qmm_get_impl<8, true, kCtF16>(gs, MT, lds);
+}
+
+}  // namespace lisaq

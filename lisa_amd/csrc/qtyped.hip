@@ -12,10 +12,10 @@
 //    :585-703): every weight dequantized to T, w = T(scale * q + bias) from an
 //    f32 fma, then y = x . w^T with f32 accumulation, rounded to T once.
 //
-// Kernels: one wave per output row for the matvec; for the matmul the matrix
-// cores with bf16/f16 (below), else 64 x 64 register-tiled f32 FMA -- correct
-// for every dtype and width, not tuned further; the bf16 2/4-bit shapes the
-// engine runs take the tuned kernels instead.
+// Kernels: one wave per output row for the matvec; for the matmul of the
+// problems that the bf16 2/4-bit matmul's kernel does not take in their type
+// (f32, rows of an odd number of groups, addresses off its alignment) the
+// matrix cores with bf16/f16 (below), else 64 x 64 register-tiled f32 FMA.
 #include "lisaq_common.h"
 #include "qmv.h"
 

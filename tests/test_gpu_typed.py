@@ -116,3 +116,35 @@ def test_quantized_matmul_typed_wide_tiles(dev, oracle, dtype, bits):
     got = y.float().cpu().numpy()
     _close(got, oracle.qmm_typed(xf, w, sf, bf, gs, bits, dtype), dtype, f"{dtype} bits={bits} wide tiles")
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("dtype,bits", [("f16", 4), ("f16", 2), ("f16", 8), ("bf16", 8)])
+@pytest.mark.parametrize("M,N,K,gs", [
+    (25, 8, 2176, 64),       # the matmul's first row count, one 8-column tile edge, 34 K-steps (34 groups a row)
+    (33, 777, 64, 32),       # one K-step, odd N (single stores)
+    (130, 300, 1024, 128),   # two row tiles, N a multiple of 4 only; split over K
+    (257, 1000, 4608, 64),   # rows past 256, split over K
+    (700, 4100, 512, 64),    # several column tiles, the last partial
+    (1300, 12288, 1152, 64), # more than one round of tiles: 256-row tiles with the last round split (2 and 4 bits)
+])
+def test_typed_matmul_matrix_core_tiles(dev, oracle, dtype, bits, M, N, K, gs):
+    """The 16-bit typed matmuls on the bf16 matmul's kernel: every tile height and split, at the edges of tiles,
+    against float64 products of the weights rounded to the compute dtype; the same bits on a repeat."""
+    import torch
+
+    rng = np.random.default_rng(M + N + K + bits)
+    w, s, b = np_linear(rng, N, K, bits, gs, s_std=0.02 if bits < 8 else 0.002)
+    sf = oracle._round_to(bf16_bits_to_f32(s), dtype)
+    bf = oracle._round_to(bf16_bits_to_f32(b), dtype)
+    xf = oracle._round_to(rng.standard_normal((M, K)).astype(np.float32), dtype)
+    args = (_tensor(xf, dtype, dev), to_dev_u32(w, dev), _tensor(sf, dtype, dev), _tensor(bf, dtype, dev))
+    assert M >= ops.qmv_batch_limit(K, N)
+    run = lambda: ops._mm_typed(*args, True, gs, bits, args[0].dtype)
+    got = run()
+    q = np.stack([(w >> np.uint32(bits * j)) & np.uint32(2**bits - 1) for j in range(32 // bits)], -1).reshape(N, K)
+    wd = oracle._round_to(np.repeat(sf, gs, 1) * q.astype(np.float32) + np.repeat(bf, gs, 1), dtype)
+    rows = np.unique(np.concatenate([np.arange(min(M, 5)), rng.integers(0, M, 40), [M - 1]]))
+    ref = xf[rows].astype(np.float64) @ wd.astype(np.float64).T
+    _close(got.float().cpu().numpy()[rows], ref, dtype, f"{dtype} bits={bits} {M}x{N}x{K}")
+    for _ in range(2):
+        assert torch.equal(got, run())
