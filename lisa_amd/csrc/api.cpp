@@ -274,7 +274,7 @@ static GatherLayout gather_layout(int64_t R, int64_t N, int64_t K, int E, int gs
     c.off = o;
     o += up256((size_t)c.cap * 16);
   }
-  L.mc = qmm_config(L.limit, N, K, gs, bits);
+  L.mc = qmm_config(L.limit, N, K, gs, bits, true, /*rows_ok=*/false);
   {
     const int mt = tall ? kTallBM / 32 : tune_int("LISAQ_GATHER_MT", L.mc.MT);
     if (mt == 4 || mt == 6 || mt == 8 || mt == kTallBM / 32) {

@@ -28,11 +28,13 @@ struct QmmConfig {
   int MT, NT, WN, BM, BN, grid_n, grid_m;  // WN: waves along N (4 or 8), NT = 8 / WN
   int grid;  // workgroups of a plain (no tile table) launch: grid_n * grid_m
   int S;            // K splits of a plain launch (1: none)
+  bool rows;        // the few-rows kernel (qmm_rows.h): one tile of all rows
   int full_tiles;   // with S > 1: whole tiles before the split remainder (0: every tile split)
   size_t ws_bytes;  // workspace for the split partials (0 when S == 1)
 };
 
-QmmConfig qmm_config(int64_t M, int64_t N, int64_t K, int gs, int bits, bool allow_split = true);
+// rows_ok: small M may take the few-rows kernel (plain launches only)
+QmmConfig qmm_config(int64_t M, int64_t N, int64_t K, int gs, int bits, bool allow_split = true, bool rows_ok = true);
 // Enqueue.  A plain launch whose config splits K uses ws (>= c.ws_bytes) for
 // the partials, or runs unsplit when ws is missing or too small.  ct: compute
 // type, LISAQ_DTYPE_BF16 or LISAQ_DTYPE_F16.

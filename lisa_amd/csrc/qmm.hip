@@ -1,7 +1,7 @@
 // Prefill matmul (qmm): host side -- tile configuration, kernel choice and
 // launch, and the reduction of split-K partials.  The kernel (its design and
 // arithmetic contract) is in qmm_kernel.h; qmm_k{4,2}_{p,s}.hip instantiate it.
-#include "qmm_kernel.h"
+#include "qmm_rows.h"
 #include <cstdlib>
 
 namespace lisaq {
@@ -40,20 +40,83 @@ __global__ __launch_bounds__(256) void qmm_hybrid_reduce_kernel(const float* __r
   }
 }
 
-// y = T(sum over the splits of the f32 partials), splits added in order.
+// y = T(sum over the splits of the f32 partials), splits added in order.  Four
+// outputs per thread, the loads of eight splits in flight at once, one wave per
+// workgroup: the launch is latency (M * N is small where K is split).
 template <int CT>
-__global__ __launch_bounds__(256) void qmm_split_reduce_kernel(const float* __restrict__ part,
-                                                               uint16_t* __restrict__ y, int64_t MN, int S) {
-  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i >= MN) return;
-  float v = part[i];
-  for (int s = 1; s < S; ++s) v += part[(int64_t)s * MN + i];
-  y[i] = Ct<CT>::one(v);
+__global__ __launch_bounds__(64) void qmm_split_reduce_kernel(const float* __restrict__ part,
+                                                              uint16_t* __restrict__ y, int64_t MN, int S) {
+  if ((MN & 3) == 0) {
+    const int64_t i = (blockIdx.x * (int64_t)64 + threadIdx.x) * 4;
+    if (i >= MN) return;
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < S; s0 += 8) {
+      f32x4 t[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        t[e] = *reinterpret_cast<const f32x4*>(part + (int64_t)(s0 + e < S ? s0 + e : S - 1) * MN + i);
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (s0 + e < S) v = s0 + e == 0 ? t[e] : v + t[e];
+    }
+    *reinterpret_cast<u32x2*>(y + i) = u32x2{Ct<CT>::pk(v[0], v[1]), Ct<CT>::pk(v[2], v[3])};
+    return;
+  }
+  // (M * N not a multiple of 4: single values, 64 apart)
+  const int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x;
+  float v[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < S; s0 += 4) {
+    float t[4][4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        t[e][c] = part[(int64_t)(s0 + e < S ? s0 + e : S - 1) * MN + (i + 64 * c < MN ? i + 64 * c : MN - 1)];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        if (s0 + e < S) v[c] = s0 + e == 0 ? t[e][c] : v[c] + t[e][c];
+  }
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+    if (i + 64 * c < MN) y[i + 64 * c] = Ct<CT>::one(v[c]);
 }
 
 // ---------------------------------------------------------------------------
-QmmConfig qmm_config(int64_t M, int64_t N, int64_t K, int gs, int bits, bool allow_split) {
+QmmConfig qmm_config(int64_t M, int64_t N, int64_t K, int gs, int bits, bool allow_split, bool rows_ok) {
   QmmConfig c{};
+  const int nk = (int)(K / 64);
+  const int split_forced = path_int("LISAQ_QMM_SPLIT", 0);  // (tests)
+  // At most 64 rows (batched decode, short prompts): the few-rows kernel, one
+  // tile of all rows, K split over workgroups up to one round of 256 (its LDS
+  // ring takes a compute unit) into parts of at least two chunks.  65-128
+  // rows stay on 128-row tiles: the same kernel with 96 and 128 rows took
+  // 35.9 and 42.6 us at 17408 x 5120, those 38.0 and 40.6.  Its scale blocks
+  // start on a dword, so rows of an even number of groups; 2 bits in groups of
+  // 32 from 33 rows on need more LDS than there is.
+  if (rows_ok && split_forced == 0 && M <= tune_int("LISAQ_QMM_ROWS", 64) && K / gs % 2 == 0 && N * (K / gs) >= 8 &&
+      !(bits == 2 && gs == 32 && M > 32)) {
+    c.rows = true;
+    c.MT = M <= 32 ? 1 : 2;
+    c.NT = 1;
+    c.WN = 16;
+    c.BM = 32 * c.MT;
+    c.BN = 256;
+    c.grid = c.grid_n = (int)((N + 255) / 256);
+    c.grid_m = 1;
+    c.S = 1;
+    const int ks = rows_chunk_steps(bits, gs, c.MT), nc = (nk + ks - 1) / ks;
+    if (allow_split && c.grid <= 128) {
+      int S = 256 / c.grid;
+      if (S > 16) S = 16;
+      if (S > nc / 2) S = nc / 2 > 0 ? nc / 2 : 1;
+      const int per = (nc + S - 1) / S;
+      c.S = (nc + per - 1) / per;  // every part non-empty
+    }
+    c.ws_bytes = c.S > 1 ? (size_t)c.S * M * N * 4 : 0;
+    return c;
+  }
   // Row tile: 128, 192 or 256 rows (MT 32-row tiles), the one with the least
   // (rounds of 256 workgroups) x (rows per tile), i.e. the least matrix-core
   // time including the last, partly filled round; ties go to the taller tile
@@ -75,7 +138,6 @@ QmmConfig qmm_config(int64_t M, int64_t N, int64_t K, int gs, int bits, bool all
   // the remainder (measured: a 256-row tile takes about the time of a
   // 192-row one, the dequantized W operands serving more rows), and the
   // remainder tiles split over K into a full last round (see below).
-  const int nk = (int)(K / 64);
   bool hybrid = false;
   {
     const int64_t t8 = ((N + 255) / 256) * ((M + 255) / 256);
@@ -124,7 +186,7 @@ QmmConfig qmm_config(int64_t M, int64_t N, int64_t K, int gs, int bits, bool all
   // with 128-row tiles only -- the tile height the small-grid rule above
   // always picks and the split tests cover
   {
-    const int v = path_int("LISAQ_QMM_SPLIT", 0);
+    const int v = split_forced;
     if (v >= 1 && v <= nk && allow_split && c.MT == 4) c.S = v;
   }
   if (c.S > 1) {
@@ -134,6 +196,19 @@ QmmConfig qmm_config(int64_t M, int64_t N, int64_t K, int gs, int bits, bool all
   c.ws_bytes = c.S > 1 ? (size_t)c.S * M * N * 4 : 0;
   (void)gs;
   return c;
+}
+
+static qmm_fn rows_pick(const QmmConfig& c, int bits, int gs, int ct, int* lds) {
+  if (ct == kCtBf16) {
+    if (bits == 4) return qmm_rows_get<4, kCtBf16>(gs, c.MT, lds);
+    if (bits == 2) return qmm_rows_get<2, kCtBf16>(gs, c.MT, lds);
+    if (bits == 8) return qmm_rows_get<8, kCtBf16>(gs, c.MT, lds);
+  } else if (ct == kCtF16) {
+    if (bits == 4) return qmm_rows_get<4, kCtF16>(gs, c.MT, lds);
+    if (bits == 2) return qmm_rows_get<2, kCtF16>(gs, c.MT, lds);
+    if (bits == 8) return qmm_rows_get<8, kCtF16>(gs, c.MT, lds);
+  }
+  return nullptr;
 }
 
 template <bool SPLIT>
@@ -164,11 +239,11 @@ int qmm_launch(hipStream_t stream, const QmmConfig& c, QmmParams p, int bits, in
                 "qmm: one weight matrix larger than 4 GiB");
   // the two split layouts: per-part [S][M][N] partials with 128-row tiles,
   // hybrid compact parts with 256-row tiles
-  if (split && !((c.full_tiles == 0 && c.MT == 4) || (c.full_tiles > 0 && c.MT == 8)))
+  if (split && !c.rows && !((c.full_tiles == 0 && c.MT == 4) || (c.full_tiles > 0 && c.MT == 8)))
     return set_error(LISAQ_EUNSUPPORTED, "qmm: split over K with %d-row tiles (%s layout) is not built", 32 * c.MT,
                      c.full_tiles > 0 ? "hybrid" : "per-part");
   int lds = 0;
-  qmm_fn fn = split ? qmm_pick<true>(c, bits, gs, ct, &lds) : qmm_pick<false>(c, bits, gs, ct, &lds);
+  qmm_fn fn = c.rows ? rows_pick(c, bits, gs, ct, &lds) : split ? qmm_pick<true>(c, bits, gs, ct, &lds) : qmm_pick<false>(c, bits, gs, ct, &lds);
   if (!fn) return set_error(LISAQ_EUNSUPPORTED, "qmm: bits=%d group_size=%d not supported", bits, gs);
   if (int rc = allow_dyn_lds((const void*)fn, lds, "qmm")) return rc;
   p.ksplit = split ? c.S : 1;
@@ -185,7 +260,7 @@ int qmm_launch(hipStream_t stream, const QmmConfig& c, QmmParams p, int bits, in
     return check_launch("qmm_hybrid_reduce");
   }
   const int64_t MN = (int64_t)p.M * p.N;
-  hipLaunchKernelGGL(ct == kCtF16 ? qmm_split_reduce_kernel<kCtF16> : qmm_split_reduce_kernel<kCtBf16>, dim3((unsigned)((MN + 255) / 256)), dim3(256), 0, stream,
+  hipLaunchKernelGGL(ct == kCtF16 ? qmm_split_reduce_kernel<kCtF16> : qmm_split_reduce_kernel<kCtBf16>, dim3((unsigned)((MN + 255) / 256)), dim3(64), 0, stream,
                      (const float*)p.partial, p.y, MN, c.S);
   return check_launch("qmm_split_reduce");
 }

@@ -109,6 +109,29 @@ __device__ __forceinline__ void static_for(F&& f) {
   static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
+// All codes of a word as pairs of weights in natural K order (16 / words-per-32-codes of them).
+template <int BITS, int CT>
+__device__ __forceinline__ void deq_word(uint32_t wv, float s24, float b, uint32_t* o) {
+  if constexpr (BITS == 8) {
+    o[0] = deq_pair<CT>(pair_code8<0>(wv), s24, b);
+    o[1] = deq_pair<CT>(pair_code8<1>(wv), s24, b);
+  } else if constexpr (BITS == 4) {
+    const uint32_t lo = opaque(wv & 0x0F0F0F0Fu), hi = opaque((wv >> 4) & 0x0F0F0F0Fu);
+    static_for<4>([&](auto PI) {
+      constexpr int d = decltype(PI)::value;
+      o[d] = deq_pair<CT>(pair_bytes<d>(lo, hi), s24, b);
+    });
+  } else {
+    uint32_t c[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) c[q] = opaque((wv >> (2 * q)) & 0x03030303u);
+    static_for<8>([&](auto PI) {
+      constexpr int d = decltype(PI)::value, m = d / 2, e = (d % 2) * 2;
+      o[d] = deq_pair<CT>(pair_bytes<m>(c[e], c[e + 1]), s24, b);
+    });
+  }
+}
+
 template <int BITS>
 struct MGeo {
   static constexpr int PACK = 32 / BITS;
@@ -488,25 +511,7 @@ __global__ __launch_bounds__(64 * WN * WM) void qmm_kernel(QmmParams p) {
       const float s24 = sf(r, nt) * 16777216.0f, b_ = bf(r, nt);
       static_for<G::WPL>([&](auto WI_) {
         constexpr int jw = decltype(WI_)::value;
-        const uint32_t wv = word(r, nt, jw);
-        if constexpr (BITS == 8) {
-          bop[nt][jw * 2] = deq_pair<CT>(pair_code8<0>(wv), s24, b_);
-          bop[nt][jw * 2 + 1] = deq_pair<CT>(pair_code8<1>(wv), s24, b_);
-        } else if constexpr (BITS == 4) {
-          const uint32_t lo = opaque(wv & 0x0F0F0F0Fu), hi = opaque((wv >> 4) & 0x0F0F0F0Fu);
-          static_for<4>([&](auto PI) {
-            constexpr int d = decltype(PI)::value;
-            bop[nt][jw * 4 + d] = deq_pair<CT>(pair_bytes<d>(lo, hi), s24, b_);
-          });
-        } else {
-          uint32_t c[4];
-#pragma unroll
-          for (int q = 0; q < 4; ++q) c[q] = opaque((wv >> (2 * q)) & 0x03030303u);
-          static_for<8>([&](auto PI) {
-            constexpr int d = decltype(PI)::value, m = d / 2, e = (d % 2) * 2;
-            bop[nt][jw * 8 + d] = deq_pair<CT>(pair_bytes<m>(c[e], c[e + 1]), s24, b_);
-          });
-        }
+        deq_word<BITS, CT>(word(r, nt, jw), s24, b_, &bop[nt][jw * (16 / G::WPL)]);
       });
     }
   };

@@ -1,0 +1,16 @@
+// Instantiations of the few-rows matmul (the kernel is in qmm_rows.h).
+#include "qmm_rows.h"
+
+namespace lisaq {
+
+template <>
+qmm_fn qmm_rows_get<2, kCtF16>(int gs, int MT, int* lds) {
+  return qmm_rows_get_impl<2, kCtF16>(gs, MT, lds);
+}
+
+template <>
+qmm_fn qmm_rows_get<8, kCtF16>(int gs, int MT, int* lds) {
+  return qmm_rows_get_impl<8, kCtF16>(gs, MT, lds);
+}
+
+}  // namespace lisaq

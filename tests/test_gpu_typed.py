@@ -148,3 +148,34 @@ def test_typed_matmul_matrix_core_tiles(dev, oracle, dtype, bits, M, N, K, gs):
     _close(got.float().cpu().numpy()[rows], ref, dtype, f"{dtype} bits={bits} {M}x{N}x{K}")
     for _ in range(2):
         assert torch.equal(got, run())
+
+
+@pytest.mark.parametrize("dtype,bits", [("bf16", 4), ("bf16", 2), ("bf16", 8), ("f16", 4), ("f16", 2), ("f16", 8)])
+@pytest.mark.parametrize("M,N,K,gs", [
+    (33, 8, 128, 64),        # one chunk, a part of a column group
+    (34, 40, 192, 32),       # a chunk that ends partway (three K-steps of 64), 6 groups a row
+    (32, 2051, 1408, 64),    # all 32 rows, odd N (single stores), 22 K-steps: parts ending partway
+    (64, 260, 4224, 64),     # all 64 rows, K parts, 66 groups a row (scale blocks past the last row's end)
+    (40, 5120, 2560, 128),   # 20 scale groups of 128 a row
+    (13, 4100, 5120, 64),    # the fewest rows, several column tiles
+    (17, 33000, 512, 64),    # more column tiles than half the compute units: no split
+])
+def test_few_rows_matmul(dev, oracle, dtype, bits, M, N, K, gs):
+    """The matmul of at most 64 rows at the edges of its chunks, column groups, scale blocks and K parts, against
+    float64 products of the rounded weights; the same bits on a repeat."""
+    import torch
+
+    rng = np.random.default_rng(M + N + K + bits)
+    w, s, b = np_linear(rng, N, K, bits, gs, s_std=0.02 if bits < 8 else 0.002)
+    sf = oracle._round_to(bf16_bits_to_f32(s), dtype)
+    bf = oracle._round_to(bf16_bits_to_f32(b), dtype)
+    xf = oracle._round_to(rng.standard_normal((M, K)).astype(np.float32), dtype)
+    args = (_tensor(xf, dtype, dev), to_dev_u32(w, dev), _tensor(sf, dtype, dev), _tensor(bf, dtype, dev))
+    assert M >= ops.qmv_batch_limit(K, N)
+    run = lambda: ops.quantized_matmul(*args, True, gs, bits)
+    got = run()
+    q = np.stack([(w >> np.uint32(bits * j)) & np.uint32(2**bits - 1) for j in range(32 // bits)], -1).reshape(N, K)
+    wd = oracle._round_to(np.repeat(sf, gs, 1) * q.astype(np.float32) + np.repeat(bf, gs, 1), dtype)
+    ref = xf.astype(np.float64) @ wd.astype(np.float64).T
+    _close(got.float().cpu().numpy(), ref, dtype, f"{dtype} bits={bits} {M}x{N}x{K}")
+    assert torch.equal(got, run())
