@@ -97,6 +97,23 @@ def load() -> ctypes.CDLL:
     return _lib
 
 
+_native = None
+
+
+def native():
+    """The native call path of ``ops`` (``_pyops.so``, csrc/pyops.cpp), over the same liblisaq.so."""
+    global _native
+    if _native is None:
+        load()
+        try:
+            from . import _pyops
+        except ImportError as e:
+            raise RuntimeError("_pyops.so missing or not loadable; build it with "
+                               "`python -c 'import __graft_entry__ as g; g.build()'`") from e
+        _native = _pyops
+    return _native
+
+
 def check(rc: int) -> None:
     if rc != OK:
         raise LisaqError(rc, load().lisaq_last_error().decode(errors="replace"))

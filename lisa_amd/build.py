@@ -1,4 +1,5 @@
-"""Builds liblisaq.so (all HIP kernels + the C ABI) in-tree for gfx950.
+"""Builds liblisaq.so (all HIP kernels + the C ABI) and _pyops.so (the native
+call path of ops.py over it) in-tree for gfx950.
 
 Each source is compiled to an object in parallel with hipcc, then linked into
 ``lisa_amd/liblisaq.so``.  Compilation always runs (the driver's "does it
@@ -10,11 +11,13 @@ import concurrent.futures as cf
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 ROOT = os.path.dirname(HERE)
 OUT = os.path.join(HERE, "liblisaq.so")
+PYOPS = os.path.join(HERE, "_pyops.so")
 OBJ = os.path.join(ROOT, "_build", "lisaq")
 SOURCES = ["qmv.hip", "qmv16.hip", "qmvt.hip", "qmvd.hip", "qmvp.hip", "qmvw.hip", "qmvs.hip", "qmm.hip", "qmm_k4_p.hip", "qmm_k4_s.hip", "qmm_k2_p.hip", "qmm_k2_s.hip", "qmm_th2.hip", "qmm_th4.hip", "qmm_th8.hip", "qmm_tb8.hip", "qmm_rows_b4.hip", "qmm_rows_b28.hip", "qmm_rows_h4.hip", "qmm_rows_h28.hip", "qmm_gu.hip", "quant.hip", "qtyped.hip", "addnorm.hip", "diag.hip", "moe.hip", "moe_decode.hip", "api.cpp"]
 
@@ -47,6 +50,25 @@ def _compile(src: str) -> str:
     return obj
 
 
+def build_pyops() -> str:
+    """_pyops.so: host C++ against this interpreter's torch, linked to liblisaq.so beside it."""
+    import torch
+
+    base = os.path.dirname(torch.__file__)
+    inc, lib = os.path.join(base, "include"), os.path.join(base, "lib")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1",
+           "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-isystem", inc,
+           "-isystem", os.path.join(inc, "torch", "csrc", "api", "include"),
+           "-I", sysconfig.get_paths()["include"], "-isystem", "/opt/rocm/include", os.path.join(CSRC, "pyops.cpp"),
+           "-o", PYOPS + ".tmp", "-L" + lib, "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip",
+           "-L" + HERE, "-l:liblisaq.so", "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed for pyops.cpp:\n{r.stderr}")
+    os.replace(PYOPS + ".tmp", PYOPS)
+    return PYOPS
+
+
 def build(verbose: bool = False) -> str:
     os.makedirs(OBJ, exist_ok=True)
     with cf.ThreadPoolExecutor(max_workers=min(len(SOURCES), os.cpu_count() or 4)) as ex:
@@ -56,6 +78,7 @@ def build(verbose: bool = False) -> str:
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stderr}")
     os.replace(OUT + ".tmp", OUT)
+    build_pyops()
     if verbose:
         print(f"built {OUT}")
     return OUT

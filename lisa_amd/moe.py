@@ -55,6 +55,9 @@ class SwitchGlu:
 
     def forward(self, x: torch.Tensor, logits: torch.Tensor, top_k: int, return_routing: bool = False):
         """x [..., H] bf16, logits [..., E] f32 -> [..., H] bf16."""
+        if x.dim() == 2 and logits.dim() == 2:
+            return ops.moe_forward(x, logits, self.gate.triple(), self.up.triple(), self.down.triple(), top_k,
+                                   self.group_size, self.bits, return_routing=return_routing)
         lead = x.shape[:-1]
         H = x.shape[-1]
         res = ops.moe_forward(x.reshape(-1, H), logits.reshape(-1, logits.shape[-1]), self.gate.triple(),

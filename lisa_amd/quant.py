@@ -58,11 +58,8 @@ class QuantizedLinear:
         return self.weight.shape[0]
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        """[..., K] -> [..., N] (flattened to 2-D for the matmul, quant.rs:306-321)."""
-        lead = x.shape[:-1]
-        flat = x.reshape(-1, x.shape[-1])
-        y = ops.quantized_matmul(flat, self.weight, self.scales, self.biases, True, self.group_size, self.bits)
-        return y.reshape(*lead, self.dims_out())
+        """[..., K] -> [..., N] (the leading dimensions are rows of one matmul, quant.rs:306-321)."""
+        return ops.quantized_matmul(x, self.weight, self.scales, self.biases, True, self.group_size, self.bits)
 
     __call__ = forward
 

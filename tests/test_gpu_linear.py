@@ -465,3 +465,47 @@ def test_addnorm_folded_kernels_agree(dev, force_path, N, K):
         outs.append([from_dev_bf16(t) for t in (y, sm, nm)])
     for a, c in zip(*outs):
         assert np.array_equal(a, c)
+
+
+@pytest.mark.parametrize("dtype,bits,M", [("bf16", 4, 1), ("bf16", 4, 40), ("bf16", 8, 3), ("f16", 4, 30), ("f32", 2, 2)])
+def test_native_call_path(dev, dtype, bits, M):
+    """quantized_matmul's native call path against the Python path on every form of the arguments that one of them
+    takes: leading dimensions, Parameters, uint32 codes, non-contiguous views, mixed dtypes, a side stream; what
+    the Python path refuses is refused with the same error."""
+    import torch
+
+    from lisa_amd import _lib
+
+    dt = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[dtype]
+    g = torch.Generator(device=dev)
+    g.manual_seed(M + bits)
+    N, K, gs = 264, 1024, 64
+    w = torch.randint(-(2**31), 2**31, (N, K * bits // 32), dtype=torch.int32, device=dev, generator=g)
+    s, b = ((torch.randn(N, K // gs, device=dev, generator=g) * 0.02).to(dt) for _ in range(2))
+    x = torch.randn(M, K, device=dev, generator=g).to(dt)
+    python = lambda *a: (ops._mm_typed(*a, True, gs, bits, torch.promote_types(a[0].dtype, a[2].dtype))
+                         if dtype != "bf16" or bits == 8 or a[0].dtype != a[2].dtype
+                         else ops._mm("lisaq_quantized_matmul", *a, True, gs, bits))
+    native = _lib.native().linear
+    ref = python(x, w, s, b)
+    plain = [(x, w, s, b), (x.view(M, 1, K), w, s, b), (torch.nn.Parameter(x), w, s, b), (x, w.view(torch.uint32), s, b)]
+    for a in plain:
+        y = native(*a, gs, bits, 0)
+        assert y is not None and y.dtype == ref.dtype and tuple(y.shape) == (*a[0].shape[:-1], N) and not y.requires_grad
+        assert torch.equal(y.view(M, N), ref) and torch.equal(ops.quantized_matmul(*a, True, gs, bits).view(M, N), ref)
+    wide = torch.stack([x, x], -1)[..., 0]  # strided
+    other = torch.float32 if dtype != "f32" else torch.float16
+    for a in [(wide, w, s, b), (x, w, s.t().contiguous().t(), b), (x.to(other), w, s, b)]:
+        assert native(*a, gs, bits, 0) is None
+        assert torch.equal(ops.quantized_matmul(*a, True, gs, bits), python(*a))
+    for a in [(x, w, s, None), (x[:, :512], w, s, b), (x, w[:, :8], s, b), (x, w, s[:5], b), (x, w.float(), s, b),
+              (x.cpu(), w, s, b)]:
+        assert native(*a, gs, bits, 0) is None
+        with pytest.raises(ops.LisaqError):
+            ops.quantized_matmul(*a, True, gs, bits)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        y = ops.quantized_matmul(x, w, s, b, True, gs, bits)
+    side.synchronize()
+    assert torch.equal(y, ref)
