@@ -204,7 +204,7 @@ constexpr int kGatherMvRows = 16;
 // knows one (moe_forward: a token picks an expert at most once, so T);
 // otherwise R.  It only sizes the matvec rows and decides if matmul tiles can
 // occur; the tables still follow the actual runs.
-// tall: matmul tiles of kTallBM rows (runs known to average >= 192 rows).
+// tall: matmul tiles of kTallBM rows (runs known to average >= kTallAvg rows).
 // gu: tables for gate|up + SwiGLU (N = I): matvec entries of half a block's
 // rows (the other half of its waves take the up weights), matmul tiles of the
 // gate|up matmul kernel.
@@ -1054,10 +1054,10 @@ struct MoeLayout {
 };
 
 // The down projection of the fused-gate|up prefill takes kTallBM-row matmul
-// tiles when runs average >= 192 rows (as the gate|up matmul does).
+// tiles when runs average >= kTallAvg rows (as the gate|up matmul does).
 static bool moe_down_tall(int64_t T, int64_t H, int64_t I, int E, int k, int gs, int bits) {
   return moe_gu_path(T, H, I, E, k, gs, bits) && tune_int("LISAQ_MOE_DOWN_TALL", 1) != 0 &&
-         T * k >= 192 * (int64_t)E;
+         T * k >= kTallAvg * (int64_t)E;
 }
 
 static MoeLayout moe_layout(int64_t T, int64_t H, int64_t I, int E, int k, int gs, int bits) {

@@ -20,14 +20,17 @@ namespace lisaq {
 constexpr bool kSkip(int mt) { return mt <= 2 || mt == 9; }
 
 
-// Row tile: 288 rows when the average expert run is at least 192 rows (the
-// dequantized weights then serve more rows; measured at E = 128, k = 8,
-// H = 2048, I = 768: T = 4096 313 vs 330 us with 256- against 128-row tiles;
-// 288 rows take a run of 256 + a few rows in one tile instead of a full tile
-// and a short one), else 128 rows (T = 512: 97 vs 131 us, most runs fit one
-// 128-row tile).
+// Row tile: 288 rows when the average expert run is at least kTallAvg rows,
+// else 128 rows.  A K-step of a tile costs about 0.55 us + 6 ns per active row
+// (dequantization, copies and the barrier do not depend on the rows), so one
+// tall tile per run, its empty 32-row blocks skipped, beats a 128-row tile
+// and a second one or a short one as soon as runs pass 128 rows.  Whole block,
+// 128 -> 288 rows (E = 128, k = 8, H = 2048, I = 768): T = 1800 (112 rows a
+// run) 291 -> 303 us, T = 2100 338 -> 316, T = 2500 386 -> 337, T = 3000 442 ->
+// 358; E = 32: T = 500 (125 rows) 120 -> 103; E = 64, H = 1024, I = 512: T =
+// 1500 (187 rows) 130 -> 97.
 int qmm_gu_rows(int64_t R, int E) {
-  return tune_int("LISAQ_GU_ROWS", R >= 192 * (int64_t)E ? kTallBM : 128);
+  return R >= kTallAvg * (int64_t)E ? kTallBM : 128;
 }
 
 template <int MT, int WN = 8, int NB = 3>
@@ -67,7 +70,7 @@ int qmm_gu_launch(hipStream_t stream, const QmmParams& p, int bits, int gs, int 
 }
 
 // Gather launches of 288-row tiles (the MoE prefill's down projection when
-// runs average >= 192 rows) and of 64-row tiles (the short last tile of a
+// runs average >= kTallAvg rows) and of 64-row tiles (the short last tile of a
 // run, skipping the matrix instructions of an empty 32-row block).
 int qmm_gather_launch(hipStream_t stream, const QmmParams& p, int bits, int gs, int grid, int rows) {
   qmm_fn fn = nullptr;

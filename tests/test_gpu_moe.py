@@ -546,3 +546,27 @@ def test_gather_short_last_tiles(dev, oracle, force_path, runs):
     assert np.array_equal(a, a0)
     ref = _gather_ref(oracle, x, W, S, B, ids, ops.qmv_batch_limit(K, N))
     assert_close_bf16(y, ref)
+
+
+@pytest.mark.parametrize("T,bits", [(479, 4), (480, 4), (480, 2), (700, 4)])
+def test_moe_forward_tile_height_rule(dev, T, bits):
+    """Runs averaging just below and from 120 rows on (128- and 288-row tiles; 175 rows: a run's second tile too):
+    moe_forward bitwise equal to the composition over 128-row gather tiles."""
+    import torch
+
+    rng = np.random.default_rng(T + bits)
+    E, k, H, I = 16, 4, 256, 320
+    G, U, D = (_expert_stack(rng, E, n, m, bits) for n, m in ((I, H), (I, H), (H, I)))
+    x = to_dev_bf16(np_x(rng, T, H), dev)
+    lg = to_dev(rng.standard_normal((T, E)).astype(np.float32), dev)
+    lg[:, 0] += 1.5  # one run well past 288 rows
+    dv = [tuple(to_dev_u32(a, dev) if i == 0 else to_dev_bf16(a, dev) for i, a in enumerate(st)) for st in (G, U, D)]
+    out = ops.moe_forward(x, lg, dv[0], dv[1], dv[2], k, 64, bits)
+    ridx, rw = ops.moe_route(lg, k)
+    srt, order, rows, inv, offs = ops.moe_sort(ridx.reshape(-1), E, k)
+    assert offs.diff().min().item() >= ops.qmv_batch_limit(H, I)  # (every run with the matmul arithmetic)
+    xs = ops.gather_rows(x, rows)
+    g, u = (ops.gather_qmm(xs, *dv[i], rhs_indices=srt, bits=bits) for i in (0, 1))
+    d = ops.gather_qmm(ops.swiglu(g, u), *dv[2], rhs_indices=srt, bits=bits)
+    ref = ops.moe_combine(d, rw.reshape(-1), inv, T, k)
+    assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
