@@ -663,8 +663,11 @@ int lisaq_quantized_matmul_serial_rows(void* stream, const void* x, const uint32
   const QmvConfig c = qmv_config(1, N, K, gs, bits);
   // Eight or four rows at a time on one weight stream with the one-row
   // kernels' arithmetic (the persistent and wave-rows kernels give every row
-  // the same bits; eight where eight staged rows of x fit the LDS); the rows
-  // left (at most three) go the pair way below.  Measured (4-bit, cold,
+  // the same bits): five to eight rows in one launch of six or eight where that
+  // many staged rows of x fit the LDS (7 rows as one launch instead of four, a
+  // pair and a single: 9728 x 2560 24.8 -> 21.2 us, 17408 x 5120 49.7 -> 44.8;
+  // 6 rows 19.8 -> 17.3, 39.8 -> 36.1; 5 rows 18.1 -> 17.4, 37.7 -> 37.3), else
+  // fours; the rows left (at most three) go the pair way below.  Measured (4-bit, cold,
   // graph-replayed, these rows vs pairs): 2560 x 9728 4 rows 12.1 vs 17.3 us,
   // 8 rows (two fours) 24.2 vs 34.2; 9728 x 2560 4 rows 13.4 vs 14.7, 8 rows
   // 21.2 vs 29.0; the north-star shape 4 rows 26.8 vs 26.7, 8 rows 51.4 vs
@@ -675,7 +678,7 @@ int lisaq_quantized_matmul_serial_rows(void* stream, const void* x, const uint32
     while (M - r_done >= 4) {
       const int64_t left = M - r_done;
       int64_t mr = 0;
-      if (left >= 8 && qmvs_rows_supported(8, N, K, gs, bits)) mr = 8;
+      if (left >= 5 && qmvs_rows_supported(left, N, K, gs, bits)) mr = left;
       else if (qmvs_rows_supported(4, N, K, gs, bits)) mr = 4;
       if (!mr) break;
       QmvParams p{};

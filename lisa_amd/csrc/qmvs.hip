@@ -304,7 +304,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void qmvs_rows_kernel(QmvParams p)
   constexpr int WPC = CB / 4;
   constexpr int PPW = 16 / BITS;
   constexpr int NP = WPC * PPW;
-  constexpr int MH = (MR == 8 && J >= 3) ? 2 : 4;  // rows of x per step inside a pass
+  constexpr int MH = MR == 6 ? (J >= 3 ? 2 : 3) : (MR == 8 && J >= 3) ? 2 : 4;  // rows of x per step inside a pass
   static_assert(MR % MH == 0, "rows of x in steps of MH");
   typedef uint32_t chunk_t __attribute__((ext_vector_type(WPC)));
 
@@ -618,10 +618,10 @@ int qmvs_launch(hipStream_t stream, const QmvConfig& c, QmvParams p, int bits, i
 
 // ---------------------------------------------------------------------------
 // Verify rows: RW = 2 (the RW x MR chains share the registers with four rows'
-// pairs); MR = 4 for 3-4 rows, 8 for 5-8; x and its sums must fit the LDS
+// pairs); MR = 4 for 3-4 rows, 6 for 5-6, 8 for 7-8; x and its sums must fit the LDS
 // (eight rows at K = 9728 do not: the caller runs two launches of four).
 static constexpr int kRowsRW = 2;
-static int qmvs_rows_mr(int64_t M) { return M <= 4 ? 4 : 8; }
+static int qmvs_rows_mr(int64_t M) { return M <= 4 ? 4 : M <= 6 ? 6 : 8; }
 // the next block's W and scales/biases loaded during this block's arithmetic
 // (two scale/bias buffers per wave) up to three passes (four with four rows
 // of x), eight rows of x from three passes on then held two at a time
@@ -664,8 +664,8 @@ int qmvs_rows_launch(hipStream_t stream, QmvParams p, int bits) {
   if (!qmvs_rows_supported(p.M, p.N, p.K, 64, bits) || p.tiles)
     return set_error(LISAQ_EUNSUPPORTED, "qmvs_rows: M=%d N=%d K=%d bits=%d", p.M, p.N, p.K, bits);
   const int C = p.K / 32, J = (C + 63) / 64, MR = qmvs_rows_mr(p.M);
-  qmvs_fn fn = bits == 4 ? (MR == 4 ? qmvs_rows_pick<4, 4>(J) : qmvs_rows_pick<4, 8>(J))
-                         : (MR == 4 ? qmvs_rows_pick<2, 4>(J) : qmvs_rows_pick<2, 8>(J));
+  qmvs_fn fn = bits == 4 ? (MR == 4 ? qmvs_rows_pick<4, 4>(J) : MR == 6 ? qmvs_rows_pick<4, 6>(J) : qmvs_rows_pick<4, 8>(J))
+                         : (MR == 4 ? qmvs_rows_pick<2, 4>(J) : MR == 6 ? qmvs_rows_pick<2, 6>(J) : qmvs_rows_pick<2, 8>(J));
   if (!fn) return set_error(LISAQ_EUNSUPPORTED, "qmvs_rows: J=%d MR=%d", J, MR);
   p.chunks = C;
   p.G = p.K / 64;

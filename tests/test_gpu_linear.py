@@ -262,6 +262,20 @@ def test_serial_rows_bitwise_equal_to_single_rows(dev, force_path, bits, M):
         force_path("LISAQ_SERIAL_ROWS", None)
 
 
+@pytest.mark.parametrize("M,N,K,bits", [(5, 100, 512, 4), (7, 33, 2560, 4), (6, 2051, 4096, 2), (5, 300, 6400, 4),
+                                        (6, 40, 9728, 4), (7, 40, 9728, 2), (7, 16, 10240, 4)])
+def test_serial_rows_five_to_seven_in_one_launch(dev, M, N, K, bits):
+    """Five to seven verify rows in one launch of six or eight (one to five passes over K, row tails; K = 9728 and
+    10240: six or fours, by what fits the LDS): every row bitwise the one-row call's."""
+    rng = np.random.default_rng(M + N + K)
+    w, s, b = np_linear(rng, N, K, bits, 64)
+    x = np_x(rng, M, K)
+    batched = _run(ops.quantized_matmul_serial_rows, dev, x, w, s, b, 64, bits)
+    for r in range(M):
+        one = _run(ops.quantized_matmul, dev, x[r:r + 1], w, s, b, 64, bits)
+        assert np.array_equal(batched[r:r + 1], one), r
+
+
 def test_repeated_calls_deterministic(dev):
     """Split-K partials are summed in slab order: identical bits every call."""
     rng = np.random.default_rng(5)
