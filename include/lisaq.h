@@ -110,9 +110,8 @@ LISAQ_API int lisaq_quantized_matmul(void* stream, const void* x, const uint32_t
  * the matvec arithmetic (f32, per-group scale*sum(x*q) + bias*sum(x),
  * QM:767-830, 996-1088), larger M the matmul arithmetic (weights rounded to T
  * from an f32 fma, f32 accumulation, QM:585-703, 1208-1326); y rounded to T
- * once.  The matvec: one wave per output row (x staged in LDS for f32 and
- * from four rows on; f16 with 4-bit codes through dot instructions).  The
- * matmul: the bf16 2/4-bit matmul's kernel for bf16 and f16 where K is a
+ * once.  The matvec: x staged in LDS, one to four output rows per wave (x or w
+ * off 16 bytes: one wave per output row).  The matmul: the bf16 2/4-bit matmul's kernel for bf16 and f16 where K is a
  * multiple of 64 and of two groups and the tensors are aligned for it (x and w
  * 16 bytes, the others 4), which splits K in a workspace of
  * lisaq_quantized_matmul_workspace bytes (256-byte aligned; without it the

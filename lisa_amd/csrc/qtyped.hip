@@ -12,12 +12,15 @@
 //    :585-703): every weight dequantized to T, w = T(scale * q + bias) from an
 //    f32 fma, then y = x . w^T with f32 accumulation, rounded to T once.
 //
-// Kernels: one wave per output row for the matvec; for the matmul of the
+// Kernels: for the matvec x in LDS and several output rows per wave (a wave per
+// output row for unaligned x or W); for the matmul of the
 // problems that the bf16 2/4-bit matmul's kernel does not take in their type
 // (f32, rows of an odd number of groups, addresses off its alignment) the
 // matrix cores with bf16/f16 (below), else 64 x 64 register-tiled f32 FMA.
 #include "lisaq_common.h"
 #include "qmv.h"
+#include "qmv_dev.h"
+#include <utility>
 
 namespace lisaq {
 
@@ -102,233 +105,162 @@ __global__ __launch_bounds__(256) void qmv_typed_kernel(const void* x, const uin
   }
 }
 
-// The same matvec with x staged in LDS: up to four rows of x (in T) copied
-// once per workgroup, the workgroup's waves then walk rows of W with a grid
-// stride, each lane loading its chunk's code words at once; the fused
-// multiply-adds are those of the kernel above in the same order (the same
-// bits).  LDS: MB x K values of T.
-template <int DT>
-__device__ __forceinline__ void ld8(const unsigned char* xl, int i, float* v) {  // values i .. i+7 of the LDS row image
-  if constexpr (DT == 1) {
-    const f32x4 a = *reinterpret_cast<const f32x4*>(xl + i * 4), c = *reinterpret_cast<const f32x4*>(xl + i * 4 + 16);
-    v[0] = a[0]; v[1] = a[1]; v[2] = a[2]; v[3] = a[3]; v[4] = c[0]; v[5] = c[1]; v[6] = c[2]; v[7] = c[3];
-  } else {
-    const u32x4 a = *reinterpret_cast<const u32x4*>(xl + i * 2);
+// Matvec with x in LDS and several rows of W per wave: the kernel for x and W
+// 16-byte aligned.  A lane takes pieces lane, lane + 64, ... of a row -- a piece
+// is one load, 16 codes of 8 bits, 32 of 4 or 2 -- of RW rows at a time, the
+// next pieces' loads in flight while these are computed; each value of x read
+// from LDS and each conversion of a code serve RW rows and MR rows of x.  Codes become f32 by
+// v_cvt_f32_ubyte, and per piece (inside one group)
+//   y += scale * sum(x * q) + bias * sum(x),
+// all in f32, sum(x) of a piece once per workgroup.
+// What bounds it: one row of x, the stream of W; from two rows on VALU issue
+// (per code ~(4.9 + 2.5 MR) cycles of a SIMD).  Against the
+// kernels it replaced (x from global memory; one row of W per wave with x in
+// LDS; f16 4-bit dot instructions), us: bf16 8-bit 9728 x 2560 1 row 9.9 -> 6.0
+// (4.4 TB/s), 4 rows 16.8 -> 11.6, 12 rows 43 -> 26; f16 8-bit 17408 x 5120 1 row
+// 22.8 -> 18.1, 12 rows 149 -> 71; f16 4-bit the same shape 1 row 17.3 both, 4
+// rows 42 -> 34; f32 4-bit 2560 x 9728 1 row 11.4 -> 9.4, 4 rows 48 -> 16.5.
+// x in LDS: planes of 16 bytes, plane q of every piece side by side (a wave's
+// reads of a plane are contiguous), then the sums.
+template <int DT, int BITS>
+struct Piece {
+  static constexpr int P = BITS == 8 ? 16 : 32;      // codes
+  static constexpr int WORDS = P * BITS / 32;        // u32 words: 4, 4 or 2
+  static constexpr int V = DT == 1 ? 4 : 8;          // values of x per 16-byte plane
+  static constexpr int PL = P / V;                   // planes
+  static constexpr int SZ = DT == 1 ? 4 : 2;         // bytes of a value
+};
+
+// codes V q .. V q + V - 1 of a piece as f32
+template <int BITS, int V, int q>
+__device__ __forceinline__ void piece_codes(const uint32_t* w, float* o) {
+#pragma unroll
+  for (int j = 0; j < V; ++j) {
+    const int i = V * q + j;  // (compile-time after unrolling)
+    if constexpr (BITS == 8) o[j] = (float)((w[i / 4] >> (8 * (i % 4))) & 0xFFu);
+    else if constexpr (BITS == 4) o[j] = (float)((((w[i / 8] >> (4 * (i & 1))) & 0x0F0F0F0Fu) >> (8 * (i % 8 / 2))) & 0xFFu);
+    else o[j] = (float)((((w[i / 16] >> (2 * (i & 3))) & 0x03030303u) >> (8 * (i % 16 / 4))) & 0xFFu);
+  }
+}
+
+template <typename F, int... Q>
+__device__ __forceinline__ void for_planes(F&& f, std::integer_sequence<int, Q...>) {
+  (f(std::integral_constant<int, Q>{}), ...);
+}
+
+template <int DT, int BITS, int GS, int MR, int RW>
+__global__ __launch_bounds__(256) void qmv_typed_rows_kernel(const void* x, const uint32_t* w, const void* s,
+                                                             const void* b, void* y, int M, int N, int K) {
+  using Pc = Piece<DT, BITS>;
+  typedef uint32_t wv_t __attribute__((ext_vector_type(Pc::WORDS)));
+  extern __shared__ __attribute__((aligned(16))) unsigned char xsm[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int C = K / Pc::P, G = K / GS;
+  const int64_t wstride = K / (32 / BITS);
+  const int m0 = blockIdx.y * MR, mr = M - m0 < MR ? M - m0 : MR;
+  float* const xsum = reinterpret_cast<float*>(xsm + (size_t)MR * K * Pc::SZ);  // [MR][C]
+  for (int m = 0; m < MR; ++m) {  // (rows past M: copies of the last, never stored)
+    const u32x4* src = reinterpret_cast<const u32x4*>(static_cast<const unsigned char*>(x) +
+                                                      (int64_t)(m0 + (m < mr ? m : mr - 1)) * K * Pc::SZ);
+    u32x4* dst = reinterpret_cast<u32x4*>(xsm + (size_t)m * K * Pc::SZ);
+    for (int e = tid; e < C * Pc::PL; e += 256) dst[(e % Pc::PL) * C + e / Pc::PL] = src[e];
+  }
+  __syncthreads();
+  // plane q of piece c of row m as f32
+  auto plane = [&](int m, int q, int c, float* v) {
+    const u32x4 a = reinterpret_cast<const u32x4*>(xsm + (size_t)m * K * Pc::SZ)[q * C + c];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      if constexpr (DT == 0) {
-        v[2 * e] = __uint_as_float(a[e] << 16);
-        v[2 * e + 1] = __uint_as_float(a[e] & 0xffff0000u);
+      const uint32_t u = a[e];
+      if constexpr (DT == 1) {
+        v[e] = __uint_as_float(u);
+      } else if constexpr (DT == 0) {
+        v[2 * e] = __uint_as_float(u << 16);
+        v[2 * e + 1] = __uint_as_float(u & 0xffff0000u);
       } else {
-        v[2 * e] = (float)__builtin_bit_cast(_Float16, (uint16_t)(a[e] & 0xffffu));
-        v[2 * e + 1] = (float)__builtin_bit_cast(_Float16, (uint16_t)(a[e] >> 16));
+        v[2 * e] = (float)__builtin_bit_cast(_Float16, (uint16_t)(u & 0xffffu));
+        v[2 * e + 1] = (float)__builtin_bit_cast(_Float16, (uint16_t)(u >> 16));
       }
     }
-  }
-}
-
-template <int DT, int BITS, int GS>
-__global__ __launch_bounds__(256) void qmv_typed_lds_kernel(const void* x, const uint32_t* w, const void* s,
-                                                            const void* b, void* y, int M, int N, int K, int MB) {
-  constexpr int MBX = 4;     // rows of x per group (at most)
-  constexpr int WPC = BITS;  // u32 words per 32-code chunk
-  constexpr int SZ = DT == 1 ? 4 : 2;
-  extern __shared__ __attribute__((aligned(16))) unsigned char xsm[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int C = K / 32, G = K / GS;
-  const int64_t wstride = K / (32 / BITS);
-  for (int m0 = 0; m0 < M; m0 += MB) {
-    const int mb = M - m0 < MB ? M - m0 : MB;
-    __syncthreads();  // (the previous group's reads are done)
-    {
-      const unsigned char* src = static_cast<const unsigned char*>(x) + (int64_t)m0 * K * SZ;
-      const int nbytes = mb * K * SZ;  // (K * SZ: a multiple of 64)
-      for (int i = tid * 16; i < nbytes; i += 256 * 16)
-        *reinterpret_cast<u32x4*>(xsm + i) = *reinterpret_cast<const u32x4*>(src + i);
+  };
+  for (int i = tid; i < MR * C; i += 256) {
+    float t = 0.f;
+#pragma unroll
+    for (int q = 0; q < Pc::PL; ++q) {
+      float v[Pc::V];
+      plane(i / C, q, i % C, v);
+#pragma unroll
+      for (int e = 0; e < Pc::V; ++e) t += v[e];
     }
-    __syncthreads();
-    for (int n = blockIdx.x * 4 + wave; n < N; n += gridDim.x * 4) {  // (wave-uniform)
-      const uint32_t* wrow = w + (int64_t)n * wstride;
-      float part[MBX];
+    xsum[i] = t;
+  }
+  __syncthreads();
+
+  struct Row {
+    wv_t w[RW];
+    float s[RW], b[RW];
+  };
+  for (int n0 = (blockIdx.x * 4 + wave) * RW; n0 < N; n0 += gridDim.x * 4 * RW) {  // (wave-uniform)
+    auto load = [&](int c, Row& o) {  // piece c (clamped: the last one, never used) of the RW rows
+      const int cc = c < C ? c : C - 1, g = cc * Pc::P / GS;
 #pragma unroll
-      for (int r = 0; r < MBX; ++r) part[r] = 0.f;
-      for (int c = lane; c < C; c += 64) {
-        uint32_t wv[WPC];
-        if constexpr (WPC == 2) {
-          const uint2 v = *reinterpret_cast<const uint2*>(wrow + c * 2);
-          wv[0] = v.x;
-          wv[1] = v.y;
-        } else {
+      for (int r = 0; r < RW; ++r) {
+        const int64_t n = n0 + r < N ? n0 + r : N - 1;
+        o.w[r] = *reinterpret_cast<const wv_t*>(w + n * wstride + cc * Pc::WORDS);
+        o.s[r] = ld<DT>(s, n * G + g);
+        o.b[r] = ld<DT>(b, n * G + g);
+      }
+    };
+    float part[RW][MR] = {};
+    auto piece = [&](int c, const Row& o) {
+      if (c >= C) return;
+      float dot[RW][MR] = {};
+      auto one = [&](auto qi) {
+        constexpr int q = decltype(qi)::value;
+        float xv[MR][Pc::V];
 #pragma unroll
-          for (int i = 0; i < WPC; i += 4) {
-            const u32x4 v = *reinterpret_cast<const u32x4*>(wrow + c * WPC + i);
-            wv[i] = v[0];
-            wv[i + 1] = v[1];
-            wv[i + 2] = v[2];
-            wv[i + 3] = v[3];
-          }
+        for (int m = 0; m < MR; ++m) plane(m, q, c, xv[m]);
+#pragma unroll
+        for (int r = 0; r < RW; ++r) {
+          uint32_t wd[Pc::WORDS];
+#pragma unroll
+          for (int e = 0; e < Pc::WORDS; ++e) wd[e] = o.w[r][e];
+          float cv[Pc::V];
+          piece_codes<BITS, Pc::V, q>(wd, cv);
+#pragma unroll
+          for (int e = 0; e < Pc::V; ++e)
+#pragma unroll
+            for (int m = 0; m < MR; ++m) dot[r][m] = fmaf(xv[m][e], cv[e], dot[r][m]);
         }
-        const int g = c * 32 / GS;
-        const float sc = ld<DT>(s, (int64_t)n * G + g), bi = ld<DT>(b, (int64_t)n * G + g);
+      };
+      for_planes(one, std::make_integer_sequence<int, Pc::PL>{});
 #pragma unroll
-        for (int r = 0; r < MBX; ++r) {
-          if (r >= mb) break;
-          const unsigned char* xr = xsm + (int64_t)r * K * SZ;
-          float dot = 0.f, xs = 0.f;
+      for (int m = 0; m < MR; ++m) {
+        const float xs = xsum[m * C + c];
 #pragma unroll
-          for (int j8 = 0; j8 < 32; j8 += 8) {
-            float xv[8];
-            ld8<DT>(xr, c * 32 + j8, xv);
-#pragma unroll
-            for (int jj = 0; jj < 8; ++jj) {
-              const int j = j8 + jj;
-              const float q = (float)((wv[j / (32 / BITS)] >> (BITS * (j % (32 / BITS)))) & ((1u << BITS) - 1u));
-              dot = fmaf(xv[jj], q, dot);
-              xs += xv[jj];
-            }
-          }
-          part[r] = fmaf(sc, dot, fmaf(bi, xs, part[r]));
-        }
+        for (int r = 0; r < RW; ++r) part[r][m] = fmaf(o.s[r], dot[r][m], fmaf(o.b[r], xs, part[r][m]));
       }
-#pragma unroll
-      for (int r = 0; r < MBX; ++r) {
-        if (r >= mb) break;
-        const float t = wsum64(part[r]);
-        if (lane == 0) st<DT>(y, (int64_t)(m0 + r) * N + n, t);
-      }
+    };
+    Row ra, rb;
+    load(lane, ra);
+    int c = lane;
+    for (int j = 0; j < C; j += 128, c += 128) {  // (uniform)
+      if (j + 64 < C) load(c + 64, rb);
+      piece(c, ra);
+      if (j + 128 < C) load(c + 128, ra);
+      if (j + 64 < C) piece(c + 64, rb);
     }
+    float out = 0.f;
+#pragma unroll
+    for (int r = 0; r < RW; ++r)
+#pragma unroll
+      for (int m = 0; m < MR; ++m) {
+        const float t = qmvdev::wave_sum(part[r][m]);
+        out = lane == r * MR + m ? t : out;
+      }
+    const int r = lane / MR, m = lane % MR;
+    if (lane < RW * MR && n0 + r < N && m < mr) st<DT>(y, (int64_t)(m0 + m) * N + n0 + r, out);
   }
-}
-
-// f16 with 4-bit codes: the matvec on dot instructions.  A code q becomes
-// the f16 128 + q exactly (bits 0x5800 | q << 3), so one word of 8 codes
-// gives the pairs (128 + q_j, 128 + q_{j+4}) with one shift, one mask and one
-// shift-or, and v_dot2_f32_f16 takes each against the pair (x_j, x_{j+4}) of
-// f16 x (products exact in f32, f32 accumulation).  Per 32-code chunk:
-// y += s * (acc - 128 sum(x)) + b * sum(x), sum(x) of the chunk in f32 once
-// per workgroup.  Up to four rows of x staged in LDS as those pairs, with the
-// chunk sums beside; rows of W walked with a grid stride.  The summation
-// order differs from the plain kernel's (within the output tolerance).
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-
-template <int GS>
-__global__ __launch_bounds__(256) void qmv_f16_dot_kernel(const void* x, const uint32_t* w, const void* s,
-                                                          const void* b, void* y, int M, int N, int K, int MB) {
-  constexpr int MBX = 4;
-  extern __shared__ __attribute__((aligned(16))) unsigned char xsm[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int C = K / 32, G = K / GS;
-  const int64_t wstride = K / 8;  // u32 words per row
-  uint32_t* xp = reinterpret_cast<uint32_t*>(xsm);                          // [MB][K / 2] pairs
-  float* xsum = reinterpret_cast<float*>(xsm + (size_t)MB * K * 2);         // [MB][C]
-  for (int m0 = 0; m0 < M; m0 += MB) {
-    const int mb = M - m0 < MB ? M - m0 : MB;
-    __syncthreads();  // (the previous group's reads are done)
-    {
-      // each thread: 8 values of x -> the pairs (x0,x4), (x1,x5), (x2,x6), (x3,x7)
-      const u32x4* src = reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(x) + (int64_t)m0 * K);
-      const int nblk = mb * K / 8;
-      for (int i = tid; i < nblk; i += 256) {
-        const u32x4 v = src[i];
-        u32x4 o;
-        o[0] = __builtin_amdgcn_perm(v[2], v[0], 0x05040100u);
-        o[1] = __builtin_amdgcn_perm(v[2], v[0], 0x07060302u);
-        o[2] = __builtin_amdgcn_perm(v[3], v[1], 0x05040100u);
-        o[3] = __builtin_amdgcn_perm(v[3], v[1], 0x07060302u);
-        reinterpret_cast<u32x4*>(xp)[i] = o;
-      }
-      // chunk sums of x in f32, in index order
-      const uint16_t* xh = static_cast<const uint16_t*>(x) + (int64_t)m0 * K;
-      for (int i = tid; i < mb * C; i += 256) {
-        float t = 0.f;
-        for (int j = 0; j < 32; ++j) t += (float)__builtin_bit_cast(_Float16, xh[(int64_t)i * 32 + j]);
-        xsum[i] = t;
-      }
-    }
-    __syncthreads();
-    for (int n = blockIdx.x * 4 + wave; n < N; n += gridDim.x * 4) {  // (wave-uniform)
-      const uint32_t* wrow = w + (int64_t)n * wstride;
-      float part[MBX];
-#pragma unroll
-      for (int r = 0; r < MBX; ++r) part[r] = 0.f;
-      for (int c = lane; c < C; c += 64) {
-        const u32x4 wv = *reinterpret_cast<const u32x4*>(wrow + c * 4);
-        uint32_t wp[16];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) wp[4 * i + j] = (((wv[i] >> (4 * j)) & 0x000F000Fu) << 3) | 0x58005800u;
-        const int g = c * 32 / GS;
-        const float sc = ld<2>(s, (int64_t)n * G + g), bi = ld<2>(b, (int64_t)n * G + g);
-#pragma unroll
-        for (int r = 0; r < MBX; ++r) {
-          if (r >= mb) break;
-          const u32x4* xr = reinterpret_cast<const u32x4*>(xp + (size_t)r * (K / 2) + c * 16);
-          float acc = 0.f;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const u32x4 xv = xr[i];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              // (the element copied out first: a bit cast of a vector element
-              // in place read the vector's first element for every j)
-              const uint32_t xw = xv[j];
-              acc = __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, xw), __builtin_bit_cast(f16x2, wp[4 * i + j]), acc,
-                                           false);
-            }
-          }
-          const float xs = xsum[r * C + c];
-          part[r] = fmaf(sc, fmaf(-128.0f, xs, acc), fmaf(bi, xs, part[r]));
-        }
-      }
-#pragma unroll
-      for (int r = 0; r < MBX; ++r) {
-        if (r >= mb) break;
-        const float t = wsum64(part[r]);
-        if (lane == 0) st<2>(y, (int64_t)(m0 + r) * N + n, t);
-      }
-    }
-  }
-}
-
-// f16 with 4-bit codes at one row of x: the same dot-instruction arithmetic
-// with a wave per output row on a grid of all rows (like the kernel reading
-// x from global memory above): each lane reads its chunk's 32 values of x
-// (cached), pairs them, and takes sum(x) of the chunk with dots against (1, 1).
-template <int GS>
-__global__ __launch_bounds__(256) void qmv_f16_dot1_kernel(const void* x, const uint32_t* w, const void* s,
-                                                           const void* b, void* y, int M, int N, int K) {
-  const int lane = threadIdx.x & 63;
-  const int n = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (n >= N) return;
-  const int C = K / 32, G = K / GS;
-  const uint32_t* wrow = w + (int64_t)n * (K / 8);
-  const u32x4* xq = static_cast<const u32x4*>(x);
-  float part = 0.f;
-  for (int c = lane; c < C; c += 64) {
-    const u32x4 wv = *reinterpret_cast<const u32x4*>(wrow + c * 4);
-    const int g = c * 32 / GS;
-    const float sc = ld<2>(s, (int64_t)n * G + g), bi = ld<2>(b, (int64_t)n * G + g);
-    float acc = 0.f, xs = 0.f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const u32x4 v = xq[c * 4 + i];  // values 32 c + 8 i .. + 7
-      uint32_t pr[4];
-      pr[0] = __builtin_amdgcn_perm(v[2], v[0], 0x05040100u);  // (x0, x4)
-      pr[1] = __builtin_amdgcn_perm(v[2], v[0], 0x07060302u);  // (x1, x5)
-      pr[2] = __builtin_amdgcn_perm(v[3], v[1], 0x05040100u);  // (x2, x6)
-      pr[3] = __builtin_amdgcn_perm(v[3], v[1], 0x07060302u);  // (x3, x7)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const uint32_t wp = (((wv[i] >> (4 * j)) & 0x000F000Fu) << 3) | 0x58005800u;
-        acc = __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, pr[j]), __builtin_bit_cast(f16x2, wp), acc, false);
-        xs = __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, pr[j]), __builtin_bit_cast(f16x2, 0x3C003C00u), xs, false);
-      }
-    }
-    part = fmaf(sc, fmaf(-128.0f, xs, acc), fmaf(bi, xs, part));
-  }
-  const float t = wsum64(part);
-  if (lane == 0) st<2>(y, n, t);
 }
 
 // Matmul: 64 x 64 output tile per workgroup, K in steps of 32 through LDS (x
@@ -524,29 +456,43 @@ __global__ __launch_bounds__(256) void qmm_typed_mfma_kernel(const void* x, cons
 
 typedef void (*typed_fn)(const void*, const uint32_t*, const void*, const void*, void*, int, int, int);
 
-typedef void (*typed_mv_fn)(const void*, const uint32_t*, const void*, const void*, void*, int, int, int, int);
+struct TypedRows {
+  typed_fn fn;
+  int rw;  // rows of W per wave
+};
 
-template <int DT, int BITS>
-typed_mv_fn pick_mv_lds_gs(int gs) {
-  if (gs == 32) return qmv_typed_lds_kernel<DT, BITS, 32>;
-  if (gs == 64) return qmv_typed_lds_kernel<DT, BITS, 64>;
-  if (gs == 128) return qmv_typed_lds_kernel<DT, BITS, 128>;
-  return nullptr;
+template <int DT, int BITS, int GS>
+TypedRows pick_rows_mr(int MR, int RW) {
+  if (MR == 1 && RW == 1) return {qmv_typed_rows_kernel<DT, BITS, GS, 1, 1>, 1};
+  if (MR == 1 && RW == 2) return {qmv_typed_rows_kernel<DT, BITS, GS, 1, 2>, 2};
+  if (MR == 1 && RW == 4) return {qmv_typed_rows_kernel<DT, BITS, GS, 1, 4>, 4};
+  if (MR == 2 && RW == 2) return {qmv_typed_rows_kernel<DT, BITS, GS, 2, 2>, 2};
+  if (MR == 2 && RW == 4) return {qmv_typed_rows_kernel<DT, BITS, GS, 2, 4>, 4};
+  if (MR == 4 && RW == 2) return {qmv_typed_rows_kernel<DT, BITS, GS, 4, 2>, 2};
+  if (MR == 4 && RW == 4) return {qmv_typed_rows_kernel<DT, BITS, GS, 4, 4>, 4};
+  return {nullptr, 0};
 }
 
 template <int DT>
-typed_mv_fn pick_mv_lds_bits(int bits, int gs) {
-  if (bits == 2) return pick_mv_lds_gs<DT, 2>(gs);
-  if (bits == 4) return pick_mv_lds_gs<DT, 4>(gs);
-  if (bits == 8) return pick_mv_lds_gs<DT, 8>(gs);
-  return nullptr;
+TypedRows pick_rows_dt(int bits, int gs, int MR, int RW) {
+  auto by_gs = [&](auto bt) -> TypedRows {
+    constexpr int B = decltype(bt)::value;
+    if (gs == 32) return pick_rows_mr<DT, B, 32>(MR, RW);
+    if (gs == 64) return pick_rows_mr<DT, B, 64>(MR, RW);
+    if (gs == 128) return pick_rows_mr<DT, B, 128>(MR, RW);
+    return {nullptr, 0};
+  };
+  if (bits == 2) return by_gs(std::integral_constant<int, 2>{});
+  if (bits == 4) return by_gs(std::integral_constant<int, 4>{});
+  if (bits == 8) return by_gs(std::integral_constant<int, 8>{});
+  return {nullptr, 0};
 }
 
-typed_mv_fn pick_mv_lds(int dtype, int bits, int gs) {
-  if (dtype == LISAQ_DTYPE_BF16) return pick_mv_lds_bits<0>(bits, gs);
-  if (dtype == LISAQ_DTYPE_F32) return pick_mv_lds_bits<1>(bits, gs);
-  if (dtype == LISAQ_DTYPE_F16) return pick_mv_lds_bits<2>(bits, gs);
-  return nullptr;
+TypedRows pick_rows(int dtype, int bits, int gs, int MR, int RW) {
+  if (dtype == LISAQ_DTYPE_BF16 && bits == 8) return pick_rows_dt<0>(bits, gs, MR, RW);
+  if (dtype == LISAQ_DTYPE_F32) return pick_rows_dt<1>(bits, gs, MR, RW);
+  if (dtype == LISAQ_DTYPE_F16) return pick_rows_dt<2>(bits, gs, MR, RW);
+  return {nullptr, 0};
 }
 
 template <int DT, int BITS, int TB>
@@ -610,56 +556,33 @@ int launch_typed_mm(hipStream_t st, bool matvec, const void* x, const uint32_t* 
   // grid.y carries the 64-row tiles of M (at most 65535 of them)
   if (!matvec && (M + 63) / 64 > 65535)
     return set_error(LISAQ_EINVAL_SHAPE, "quantized_matmul_typed: M=%lld exceeds %d rows", (long long)M, 65535 * 64);
-  // f16 x with 4-bit codes at one row: the one-row dot kernel (x, W 16-byte aligned)
-  if (matvec && dtype == LISAQ_DTYPE_F16 && bits == 4 && M == 1 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
-      reinterpret_cast<uintptr_t>(w) % 16 == 0 && tune_int("LISAQ_TYPED_F16_DOT1", 1) != 0) {
-    typed_fn f1 = gs == 32 ? qmv_f16_dot1_kernel<32> : gs == 64 ? qmv_f16_dot1_kernel<64>
-                : gs == 128 ? qmv_f16_dot1_kernel<128> : nullptr;
-    if (f1) {
-      hipLaunchKernelGGL(f1, dim3((unsigned)((N + 3) / 4)), dim3(256), 0, st, x, w, s, b, y, (int)M, (int)N, (int)K);
-      return check_launch("quantized_matmul_typed");
-    }
-  }
-  // f16 x with 4-bit codes, two rows of x or more: the dot-instruction matvec
-  // (x, W 16-byte aligned).  Measured (17408 x 5120, graph-replayed; kernel
-  // reading x from global memory -> this one): M=2 33.8 -> 29.0 us, M=4
-  // 56.2 -> 44.7; one row stays on the global-x kernel (22.4 vs 23.4 here,
-  // 7.8 vs 6.8 at 2560 x 9728): its 4352 small workgroups hide the latency
-  // of each row's loads, which this kernel's rows walked in turn do not
-  if (matvec && dtype == LISAQ_DTYPE_F16 && bits == 4 && M >= 2 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
-      reinterpret_cast<uintptr_t>(w) % 16 == 0 && tune_int("LISAQ_TYPED_F16_DOT", 1) != 0) {
-    const int64_t per_row = K * 2 + (K / 32) * 4;  // pairs + chunk sums
-    const int64_t mbd = (160 * 1024) / per_row;
-    typed_mv_fn fd = gs == 32 ? qmv_f16_dot_kernel<32> : gs == 64 ? qmv_f16_dot_kernel<64>
-                   : gs == 128 ? qmv_f16_dot_kernel<128> : nullptr;
-    if (fd && mbd >= 1) {
-      const int MB = (int)(mbd < 4 ? mbd : 4) < M ? (int)(mbd < 4 ? mbd : 4) : (int)M;
-      const int lds = (int)(MB * per_row);
-      if (int rc = allow_dyn_lds((const void*)fd, lds, "quantized_matmul_typed")) return rc;
-      const int64_t rows4 = (N + 3) / 4;
-      const unsigned grid = (unsigned)(rows4 < 2048 ? rows4 : 2048);
-      hipLaunchKernelGGL(fd, dim3(grid), dim3(256), lds, st, x, w, s, b, y, (int)M, (int)N, (int)K, MB);
-      return check_launch("quantized_matmul_typed");
-    }
-  }
-  // matvec with x staged in LDS (rows of x per group as the LDS allows, at
-  // most four; x 16-byte aligned): for f32, and for 16-bit x from four rows
-  // on.  Measured (gs 64, graph-replayed; global-x kernel -> this one):
-  // 17408 x 5120 4-bit f32 M=1 51.8 -> 27.5 us, M=4 161.9 -> 96.0, f16 M=4
-  // 62.2 -> 52.2 but f16 M=1 19.7 -> 24.8 (one row: the global-x kernel's
-  // 4352 small workgroups hide the x reads better than 1024 staging ones)
-  const int xsz = dtype == LISAQ_DTYPE_F32 ? 4 : 2;
-  const int64_t mbl = (160 * 1024) / (K * xsz);
-  if (matvec && mbl >= 1 && (dtype == LISAQ_DTYPE_F32 || M >= 4) && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
-      reinterpret_cast<uintptr_t>(w) % 16 == 0 && tune_int("LISAQ_TYPED_MV_LDS", 1) != 0) {
-    typed_mv_fn fl = pick_mv_lds(dtype, bits, gs);
-    if (fl) {
-      const int MB = (int)(mbl < 4 ? mbl : 4) < M ? (int)(mbl < 4 ? mbl : 4) : (int)M;
-      const int lds = (int)(MB * K * xsz);
-      if (int rc = allow_dyn_lds((const void*)fl, lds, "quantized_matmul_typed")) return rc;
-      const int64_t rows4 = (N + 3) / 4;
-      const unsigned grid = (unsigned)(rows4 < 1024 ? rows4 : 1024);
-      hipLaunchKernelGGL(fl, dim3(grid), dim3(256), lds, st, x, w, s, b, y, (int)M, (int)N, (int)K, MB);
+  // Matvec, x and W 16-byte aligned and a row of x fits the LDS: the rows
+  // kernel.  Rows of x per workgroup (MR): four save re-reading a large W where
+  // they take at most 48 KB of LDS (f16 8-bit 17408 x 5120 4 rows 30.5 us, two
+  // at a time 37.2; 12 rows 71 / 90), two otherwise (bf16 8-bit 9728 x 2560 4 rows
+  // 11.6 us, 15.3 four at a time; 12 rows 26 / 31), one where two pass that
+  // (bf16 8-bit 5120 x 17408 4 rows 42 us, 62 / 48 at four / two).  Rows of W per
+  // wave (RW): one row of x two, one below 4096 rows (f32 1000 x 8192 RW 2 6.0 us,
+  // RW 4 7.6); else four, two where that leaves a compute unit without a workgroup.
+  const int P = bits == 8 ? 16 : 32;
+  const int64_t per_row = K * (dtype == LISAQ_DTYPE_F32 ? 4 : 2) + K / P * 4;
+  if (matvec && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0 &&
+      per_row <= 160 * 1024) {
+    const int64_t room = 48 * 1024;
+    const int MR = M >= 3 && N * K * bits / 8 >= ((int64_t)32 << 20) && 4 * per_row <= room ? 4
+                   : M >= 2 && 2 * per_row <= room                                          ? 2
+                                                                                            : 1;
+    const int64_t groups = (M + MR - 1) / MR;
+    const int RW = M == 1 ? (N >= 4096 ? 2 : 1) : (N + 15) / 16 * groups >= 256 ? 4 : 2;
+    const TypedRows k = pick_rows(dtype, bits, gs, MR, MR == 1 && M > 1 ? 4 : RW);
+    if (k.fn) {
+      const int lds = (int)(MR * per_row);
+      if (int rc = allow_dyn_lds((const void*)k.fn, lds, "quantized_matmul_typed")) return rc;
+      // as many workgroups as the chip holds (each stages x once), at most 8 per compute unit
+      const int64_t blocks = (N + 4 * k.rw - 1) / (4 * k.rw), per_cu = (160 * 1024) / lds < 8 ? (160 * 1024) / lds : 8;
+      const int64_t cap = 256 * per_cu;
+      hipLaunchKernelGGL(k.fn, dim3((unsigned)(blocks < cap ? blocks : cap), (unsigned)groups), dim3(256), lds, st, x,
+                         w, s, b, y, (int)M, (int)N, (int)K);
       return check_launch("quantized_matmul_typed");
     }
   }

@@ -179,3 +179,32 @@ def test_few_rows_matmul(dev, oracle, dtype, bits, M, N, K, gs):
     ref = xf.astype(np.float64) @ wd.astype(np.float64).T
     _close(got.float().cpu().numpy(), ref, dtype, f"{dtype} bits={bits} {M}x{N}x{K}")
     assert torch.equal(got, run())
+
+
+@pytest.mark.parametrize("dtype,bits", [("bf16", 8), ("f16", 2), ("f16", 4), ("f16", 8), ("f32", 2), ("f32", 4), ("f32", 8)])
+@pytest.mark.parametrize("M,N,K,gs", [
+    (1, 3, 32, 32),         # one piece (two of 8 bits), fewer rows than a wave takes
+    (1, 4097, 2080, 32),    # two rows of W per wave, a tail row, 65 pieces of 32 (one past a wave's pass)
+    (2, 70, 4224, 128),     # two rows of x, few workgroups
+    (3, 4100, 2560, 64),    # a group of two and one, four rows of W per wave
+    (5, 17408, 2560, 64),   # (8 bits: groups of four rows of x, one in the second)
+    (7, 500, 17408, 64),    # long rows: one row of x per workgroup
+    (12, 1001, 1024, 64),   # the most rows here, N odd
+])
+def test_typed_matvec_rows(dev, oracle, dtype, bits, M, N, K, gs):
+    """The matvec with x in LDS at the edges of its pieces, row groups and rows per wave, against the oracle; the
+    same rows from an x that is not 16-byte aligned (a wave per output row) within the output's rounding of them."""
+    import torch
+
+    rng = np.random.default_rng(M * 31 + N + K + bits)
+    w, s, b = np_linear(rng, N, K, bits, gs, s_std=0.02 if bits < 8 else 0.002)
+    sf = oracle._round_to(bf16_bits_to_f32(s), dtype)
+    bf = oracle._round_to(bf16_bits_to_f32(b), dtype)
+    xf = oracle._round_to(rng.standard_normal((M, K)).astype(np.float32), dtype)
+    assert M < ops.qmv_batch_limit(K, N)
+    x, wd, sd, bd = _tensor(xf, dtype, dev), to_dev_u32(w, dev), _tensor(sf, dtype, dev), _tensor(bf, dtype, dev)
+    ref = oracle.qmv_typed(xf, w, sf, bf, gs, bits)
+    _close(ops.quantized_matmul(x, wd, sd, bd, True, gs, bits).float().cpu().numpy(), ref, dtype, "rows kernel")
+    off = torch.empty(M * K + 1, dtype=x.dtype, device=dev)[1:].view(M, K)
+    off.copy_(x)
+    _close(ops.quantized_matmul(off, wd, sd, bd, True, gs, bits).float().cpu().numpy(), ref, dtype, "unaligned x")
