@@ -601,7 +601,6 @@ __global__ __launch_bounds__(64 * WN * WM) void qmm_kernel(QmmParams p) {
     const int xs1 = xs == NB - 1 ? 0 : xs + 1;    // (k+1) % NB
     const unsigned char* xb = smem + xs * L::X;
     const unsigned char* xb1 = smem + xs1 * L::X;
-    float s24[NT], b32[NT];  // scale * 2^24 and bias of the W being dequantized
     uint32_t lo[NT][G::WPL], hi[NT][G::WPL], c4[NT][G::WPL][4];  // split codes of the words being dequantized
     // scale/bias block sb + 1 is copied during global step sb * SBK - 1, at
     // the earliest one step after the prologue's reads (a first step at
@@ -674,11 +673,7 @@ __global__ __launch_bounds__(64 * WN * WM) void qmm_kernel(QmmParams p) {
         if constexpr (d * SLOTS / NPIECE == sl) {
           constexpr int dnt = d / (G::WPL * PPW), dw = d / PPW % G::WPL, dp = d % PPW;
           const uint32_t wv = word(wn, dnt, dw);
-          if constexpr (d % (G::WPL * PPW) == 0) {
-            s24[dnt] = sf(wn, dnt) * 16777216.0f;
-            b32[dnt] = bf(wn, dnt);
-          }
-          const float s_ = s24[dnt], b_ = b32[dnt];
+          const float s_ = sf(wn, dnt) * 16777216.0f, b_ = bf(wn, dnt);
           if constexpr (BITS == 8) {
             bnxt[dnt][dw * 2 + dp] = opaque(deq_pair<CT>(pair_code8<dp>(wv), s_, b_));
           } else if constexpr (BITS == 4) {
