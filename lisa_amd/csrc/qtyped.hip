@@ -456,6 +456,111 @@ __global__ __launch_bounds__(256) void qmm_typed_mfma_kernel(const void* x, cons
 
 typedef void (*typed_fn)(const void*, const uint32_t*, const void*, const void*, void*, int, int, int);
 
+// f32 matmul on the matrix cores: the same contract (weights are the f32
+// fma(scale, q, bias), f32 accumulation) with v_mfma_f32_32x32x2_f32, each of
+// four waves a 32 x 32 tile of f32 products.  Two forms:
+//  * KS = false: a 64 x 64 tile, the waves its quarters, K in steps of 32;
+//  * KS = true (fewer such tiles than compute units): a 32 x 32
+//    tile, K in steps of 128 of which each wave takes 32, the four sums added
+//    through LDS in wave order.
+// Bounded by the matrix cores (157 TFLOP/s; a step is sixteen of their 64-cycle
+// instructions per wave, its loads for the next step in flight).  The 64 x 64
+// FMA tiles it replaced left most of the chip idle at small sizes and read
+// every operand from LDS per product: 4-bit 64 x 4096 x 4096 458 -> 40 us, 256 x
+// 4096 x 4096 561 -> 100 (86 TFLOP/s).
+// LDS rows padded by 16 bytes: the 32 rows of a read fall on distinct banks.
+template <int BITS, int GS, bool KS>
+__global__ __launch_bounds__(256) void qmm_f32_mfma_kernel(const void* xv, const uint32_t* w, const void* sv,
+                                                           const void* bv, void* yv, int M, int N, int K) {
+  constexpr int T = KS ? 32 : 64, BK = KS ? 128 : 32, RS = BK + 4;  // tile, K step, LDS row in floats
+  constexpr int TPR = 256 / T, VPT = BK / TPR;                     // staging threads per row, values per thread
+  const float* const x = static_cast<const float*>(xv);
+  const float* const s = static_cast<const float*>(sv);
+  const float* const b = static_cast<const float*>(bv);
+  float* const y = static_cast<float*>(yv);
+  __shared__ __attribute__((aligned(16))) float xa[2][T * RS], wb[2][T * RS];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = lane >> 5, col = lane & 31;
+  const int m0 = blockIdx.y * T, n0 = blockIdx.x * T;
+  const int wm = KS ? 0 : (wave >> 1) * 32, wn = KS ? 0 : (wave & 1) * 32, wk = KS ? wave * 32 : 0;
+  const int G = K / GS;
+  const int sr = tid / TPR, sc = (tid % TPR) * VPT;  // staging role: row, first value of the step
+  const float* const xrow = x + (int64_t)(m0 + sr < M ? m0 + sr : M - 1) * K;  // (rows past the matrices: never stored)
+  const int nr = n0 + sr < N ? n0 + sr : N - 1;
+  const uint32_t* const wrow = w + (int64_t)nr * (K / (32 / BITS));
+  constexpr int NW = VPT * BITS >= 32 ? VPT * BITS / 32 : 1;  // code words of a thread's values
+  f32x4 xr[VPT / 4];
+  uint32_t cw[NW];
+  float scale, bias;
+  auto fetch = [&](int k0) {
+    const int k = k0 + sc;
+    const bool in = k < K;  // (K is a multiple of 32, VPT of a thread lie inside or outside)
+    const int kk = in ? k : 0;
+#pragma unroll
+    for (int i = 0; i < VPT / 4; ++i) {
+      xr[i] = *reinterpret_cast<const f32x4*>(xrow + kk + 4 * i);
+      if (!in) xr[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int i = 0; i < NW; ++i) cw[i] = wrow[kk * BITS / 32 + i];
+    if constexpr (VPT * BITS < 32) cw[0] >>= BITS * (kk % (32 / BITS));
+    scale = in ? s[(int64_t)nr * G + kk / GS] : 0.f;
+    bias = in ? b[(int64_t)nr * G + kk / GS] : 0.f;
+  };
+  auto stage = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < VPT / 4; ++i) {
+      *reinterpret_cast<f32x4*>(&xa[buf][sr * RS + sc + 4 * i]) = xr[i];
+      f32x4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int j = 4 * i + e;
+        v[e] = fmaf(scale, (float)((cw[j * BITS / 32] >> (BITS * (j % (32 / BITS)))) & ((1u << BITS) - 1u)), bias);
+      }
+      *reinterpret_cast<f32x4*>(&wb[buf][sr * RS + sc + 4 * i]) = v;
+    }
+  };
+  f32x16 acc = {};
+  fetch(0);
+  stage(0);
+  __syncthreads();
+  for (int k0 = 0, buf = 0; k0 < K; k0 += BK, buf ^= 1) {
+    const bool more = k0 + BK < K;
+    if (more) fetch(k0 + BK);
+    // half-wave h takes the values 16 h .. 16 h + 15 of the wave's 32
+    const float* const ar = &xa[buf][(wm + col) * RS + wk + 16 * half];
+    const float* const br = &wb[buf][(wn + col) * RS + wk + 16 * half];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const f32x4 a = *reinterpret_cast<const f32x4*>(ar + 4 * i), c = *reinterpret_cast<const f32x4*>(br + 4 * i);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], c[e], acc, 0, 0, 0);
+    }
+    if (more) stage(buf ^ 1);  // (buffer buf ^ 1 was last read before the previous barrier)
+    __syncthreads();
+  }
+  // the accumulator: column col, rows 8 (i / 4) + 4 half + i % 4
+  if constexpr (KS) {
+    float* const ex = xa[0];  // [4 waves][1024]
+    static_assert(2 * T * RS >= 4 * 1024, "sums fit");
+#pragma unroll
+    for (int i = 0; i < 16; ++i) ex[wave * 1024 + i * 64 + lane] = acc[i];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int i = wave * 4 + j, e = i * 64 + lane;
+      const float t = ((ex[e] + ex[1024 + e]) + ex[2048 + e]) + ex[3072 + e];
+      const int m = m0 + 8 * (i / 4) + 4 * half + i % 4, n = n0 + col;
+      if (m < M && n < N) y[(int64_t)m * N + n] = t;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int m = m0 + wm + 8 * (i / 4) + 4 * half + i % 4, n = n0 + wn + col;
+      if (m < M && n < N) y[(int64_t)m * N + n] = acc[i];
+    }
+  }
+}
+
 struct TypedRows {
   typed_fn fn;
   int rw;  // rows of W per wave
@@ -486,6 +591,21 @@ TypedRows pick_rows_dt(int bits, int gs, int MR, int RW) {
   if (bits == 4) return by_gs(std::integral_constant<int, 4>{});
   if (bits == 8) return by_gs(std::integral_constant<int, 8>{});
   return {nullptr, 0};
+}
+
+template <bool KS>
+typed_fn pick_f32(int bits, int gs) {
+  auto by_gs = [&](auto bt) -> typed_fn {
+    constexpr int B = decltype(bt)::value;
+    if (gs == 32) return qmm_f32_mfma_kernel<B, 32, KS>;
+    if (gs == 64) return qmm_f32_mfma_kernel<B, 64, KS>;
+    if (gs == 128) return qmm_f32_mfma_kernel<B, 128, KS>;
+    return nullptr;
+  };
+  if (bits == 2) return by_gs(std::integral_constant<int, 2>{});
+  if (bits == 4) return by_gs(std::integral_constant<int, 4>{});
+  if (bits == 8) return by_gs(std::integral_constant<int, 8>{});
+  return nullptr;
 }
 
 TypedRows pick_rows(int dtype, int bits, int gs, int MR, int RW) {
@@ -551,6 +671,16 @@ int launch_typed_mm(hipStream_t st, bool matvec, const void* x, const uint32_t* 
     if (dtype == LISAQ_DTYPE_BF16) fn = wide ? pick_mfma<0, 2>(bits, gs) : pick_mfma<0, 1>(bits, gs);
     else fn = wide ? pick_mfma<2, 2>(bits, gs) : pick_mfma<2, 1>(bits, gs);
     if (wide) tile = 128;
+  }
+  // f32: the matrix-core matmul (x 16-byte aligned), in 64 x 64 tiles where
+  // those make a workgroup per compute unit, else 32 x 32 with K over the waves
+  // (4-bit, 64- / 32-row tiles: 64 x 4096 x 4096, 64 tiles, 99.8 / 39.8 us; 16 x
+  // 9728 x 2560, 152 tiles, 63 / 41; 256 x 4096 x 4096, 256 tiles, 100 / 126; 40 x
+  // 17408 x 2560, 272 tiles, 106 / 99; 900 x 2048 x 2048, 480 tiles, 87 / 125)
+  if (!matvec && fn && dtype == LISAQ_DTYPE_F32 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && (M + 31) / 32 <= 65535) {
+    const bool ks = ((M + 63) / 64) * ((N + 63) / 64) < 256;
+    fn = ks ? pick_f32<true>(bits, gs) : pick_f32<false>(bits, gs);
+    tile = ks ? 32 : 64;
   }
   if (!fn) return set_error(LISAQ_EUNSUPPORTED, "quantized_matmul_typed: dtype=%d bits=%d gs=%d", dtype, bits, gs);
   // grid.y carries the 64-row tiles of M (at most 65535 of them)

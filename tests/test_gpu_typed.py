@@ -208,3 +208,30 @@ def test_typed_matvec_rows(dev, oracle, dtype, bits, M, N, K, gs):
     off = torch.empty(M * K + 1, dtype=x.dtype, device=dev)[1:].view(M, K)
     off.copy_(x)
     _close(ops.quantized_matmul(off, wd, sd, bd, True, gs, bits).float().cpu().numpy(), ref, dtype, "unaligned x")
+
+
+@pytest.mark.parametrize("bits", [2, 4, 8])
+@pytest.mark.parametrize("M,N,K,gs", [
+    (33, 5, 32, 32),         # one K-step, a quarter of a 128-value step; fewer columns than a tile
+    (70, 100, 416, 32),      # 32 x 32 tiles, row and column tails, K ends inside a step
+    (25, 2100, 3072, 128),   # the fewest rows
+    (1500, 1470, 320, 64),   # 64 x 64 tiles (24 x 23), row and column tails
+])
+def test_f32_matmul_matrix_cores(dev, oracle, bits, M, N, K, gs):
+    """The f32 matmul on the matrix cores: relative error of the whole result against float64 at most that of f32
+    sums of K products (K 2^-24 bounds every order; the square root is typical)."""
+    import torch
+
+    rng = np.random.default_rng(M + N + K + bits)
+    w, s, b = np_linear(rng, N, K, bits, gs, s_std=0.02 if bits < 8 else 0.002)
+    sf, bf = bf16_bits_to_f32(s), bf16_bits_to_f32(b)
+    xf = rng.standard_normal((M, K)).astype(np.float32)
+    assert M >= ops.qmv_batch_limit(K, N)
+    y = ops.quantized_matmul(_tensor(xf, "f32", dev), to_dev_u32(w, dev), _tensor(sf, "f32", dev),
+                             _tensor(bf, "f32", dev), True, gs, bits).cpu().numpy()
+    q = np.stack([(w >> np.uint32(bits * j)) & np.uint32(2**bits - 1) for j in range(32 // bits)], -1).reshape(N, K)
+    wd = np.repeat(sf, gs, 1).astype(np.float64) * q + np.repeat(bf, gs, 1)
+    ref = xf.astype(np.float64) @ wd.T
+    bound = 2.0**-24 * (K * np.abs(xf).astype(np.float64) @ np.abs(wd).T / np.sqrt(K) + np.abs(ref))
+    assert (np.abs(y - ref) <= 4 * bound).all()
+    assert np.linalg.norm(y - ref) <= 1e-6 * np.linalg.norm(ref) * max(1.0, np.sqrt(K / 1024))
