@@ -115,67 +115,74 @@ __global__ __launch_bounds__(256) void quant_kernel(const T* __restrict__ w, uin
   }
 }
 
-// The same rule with 8 consecutive values per thread: GS / 8 neighbouring lanes
-// own a group, so a wave reads 1 KB (bf16) of consecutive values per load and
-// stores consecutive code words, and the group's range is two DPP reductions
-// (minimum and maximum are exact in any order).  One thread per group reads 2
-// bytes at a stride of a whole group: every load touched 64 cache lines, and
-// 9728 x 2560 bf16 -> 4 bits took 950 us for 64 MB (then dequantize: 916 us
-// for both calls; 35 us with this kernel, the same bits).
+// The same rule with 16 consecutive values per thread: GS / 16 neighbouring lanes
+// own a group, so a wave reads 2 KB (bf16) of consecutive values and stores
+// consecutive code words, and the group's range is two DPP reductions (minimum
+// and maximum are exact in any order).  One thread per group reads 2 bytes at
+// a stride of a whole group: every load touched 64 cache lines, and 9728 x 2560
+// bf16 -> 4 bits took 950 us for 64 MB; here 17 us (3.7 TB/s).
 //
-// Codes: round(fl((v - bias) / scale)), halves away from zero.  The IEEE
-// division is ~10 operations per value and decides only quotients next to a
-// half: u = (v - bias) * fl(1 / scale) is within 2^-22 |u| of the quotient, so
-// where u (in [-1/2, 300)) is further than 1e-4 from a half, both round to
-// the same integer.  A wave with any other value (ties, NaN, infinities, a scale
-// whose reciprocal could be denormal) divides.
+// Codes: roundf(d), d = fl(a / s) with a = fl(v - bias) and, signs taken out, s > 0:
+// without the IEEE division (~10 operations per value, and bf16 values meet
+// halves often).  k = floor(a * fl(1 / s)) is the integer below d or, within the
+// product's error of an integer, its neighbour; either way roundf(d) is k + 1 if
+// d >= h and k if not, h = k + 1/2.  d >= h exactly where a / s >= h - g / 2, g the
+// gap below h in f32 (the midpoint rounds to h, whose mantissa is even), i.e.
+// (a - h s) + (g / 2) s >= 0.  Near a half a - h s is a multiple of ulp(s) / 2
+// below 2^10 of them (h < 2^9 is a multiple of 1/2), so its fma is exact, and the
+// second fma's rounding keeps the sum's sign.  A NaN stays one up to the minimum,
+// which gives the largest code as roundf's path does.  Infinities and scales far
+// from 1 divide.
 template <int CTRL>
 __device__ __forceinline__ float dpp_f32(float v) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
 }
 
+constexpr int kQuantVals = 16;
+
 template <typename T, int BITS, int GS>
-__global__ __launch_bounds__(256) void quant8_kernel(const T* __restrict__ w, uint32_t* __restrict__ wq,
-                                                     T* __restrict__ scales, T* __restrict__ biases,
-                                                     int64_t nchunks) {
-  constexpr int L = GS / 8;  // lanes per group: 4, 8 or 16 of a 16-lane DPP row
+__global__ __launch_bounds__(256) void quant16_kernel(const T* __restrict__ w, uint32_t* __restrict__ wq,
+                                                      T* __restrict__ scales, T* __restrict__ biases,
+                                                      int64_t nchunks) {
+  constexpr int V = kQuantVals, L = GS / V;  // values per thread; lanes per group: 2, 4 or 8 of a 16-lane DPP row
   const int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   // (a group's chunks are all inside or all outside the matrix)
   if (c >= nchunks) return;
-  float v[8];
+  float v[V];
   if constexpr (sizeof(T) == 2) {
-    const u32x4 a = *reinterpret_cast<const u32x4*>(w + c * 8);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      v[2 * j] = bf2f_lo(a[j]);
-      v[2 * j + 1] = bf2f_hi(a[j]);
+    for (int i = 0; i < V / 8; ++i) {
+      const u32x4 a = *reinterpret_cast<const u32x4*>(w + c * V + 8 * i);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        v[8 * i + 2 * j] = bf2f_lo(a[j]);
+        v[8 * i + 2 * j + 1] = bf2f_hi(a[j]);
+      }
     }
   } else {
-    const f32x4 a0 = *reinterpret_cast<const f32x4*>(w + c * 8), a1 = *reinterpret_cast<const f32x4*>(w + c * 8 + 4);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      v[j] = a0[j];
-      v[4 + j] = a1[j];
+    for (int i = 0; i < V / 4; ++i) {
+      const f32x4 a = *reinterpret_cast<const f32x4*>(w + c * V + 4 * i);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[4 * i + j] = a[j];
     }
   }
   constexpr float maxq = (float)((1u << BITS) - 1u);
   float w_min = 3.40282347e38f, w_max = 0.0f;
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
+  for (int j = 0; j < V; ++j) {
     w_min = fminf(w_min, v[j]);
     w_max = fmaxf(w_max, v[j]);
   }
   w_min = fminf(w_min, dpp_f32<0xB1>(w_min));  // lane ^ 1
   w_max = fmaxf(w_max, dpp_f32<0xB1>(w_max));
-  w_min = fminf(w_min, dpp_f32<0x4E>(w_min));  // lane ^ 2
-  w_max = fmaxf(w_max, dpp_f32<0x4E>(w_max));
+  if constexpr (L >= 4) {
+    w_min = fminf(w_min, dpp_f32<0x4E>(w_min));  // lane ^ 2
+    w_max = fmaxf(w_max, dpp_f32<0x4E>(w_max));
+  }
   if constexpr (L >= 8) {
     w_min = fminf(w_min, dpp_f32<0x141>(w_min));  // mirrored half rows: the other four of eight
     w_max = fmaxf(w_max, dpp_f32<0x141>(w_max));
-  }
-  if constexpr (L >= 16) {
-    w_min = fminf(w_min, dpp_f32<0x140>(w_min));  // mirrored rows: the other eight
-    w_max = fmaxf(w_max, dpp_f32<0x140>(w_max));
   }
   float scale = fmaxf(__fdiv_rn(w_max - w_min, maxq), 1e-7f);
   const bool side = fabsf(w_min) > fabsf(w_max);
@@ -185,40 +192,50 @@ __global__ __launch_bounds__(256) void quant8_kernel(const T* __restrict__ w, ui
   const bool at_zero = q0 == 0.0f;
   if (!at_zero) scale = __fdiv_rn(edge, q0);
   const float bias = at_zero ? 0.0f : edge;
-  const float r = __fdiv_rn(1.0f, scale);
-  float a[8], q[8];
-  bool sure = fabsf(scale) < 1e30f && fabsf(scale) > 1e-30f;
+  const float sa = fabsf(scale), sg = scale < 0.0f ? -1.0f : 1.0f;
+  const float r = __fdiv_rn(1.0f, sa), sb = -bias * sg, g2 = sa * 5.9604645e-8f;  // (2^-24 s)
+  const bool sure = sa < 1e30f && sa > 1e-30f && fabsf(w_min) < 1e30f && w_max < 1e30f;
+  float q[V];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    a[j] = __fsub_rn(v[j], bias);
-    const float u = __fmul_rn(a[j], r);
-    const float fl = floorf(u), f = u - fl;
-    sure = sure && fabsf(f - 0.5f) > 1e-4f && u < 300.0f && u > -0.5f;
-    q[j] = fminf(f > 0.5f ? fl + 1.0f : fl, maxq);
+  for (int j = 0; j < V; ++j) {
+    const float a = fmaf(v[j], sg, sb);
+    const float h = floorf(a * r) + 0.5f;
+    // 2^p with p the exponent of the value below |h|: g / 2 = 2^p 2^-24
+    const float e2p = __uint_as_float((__float_as_uint(h) - 1u) & 0x7F800000u);
+    const float e = fmaf(e2p, g2, fmaf(-h, sa, a));
+    q[j] = fminf(h + __builtin_copysignf(0.5f, e), maxq);
   }
-  if (!__all(sure)) {
+  constexpr int NW = V * BITS / 32, CPH = 16 / BITS;  // words; codes per half word
+  uint32_t o[NW];
+  if (__all(sure)) {
+    // half words as sums of powers (exact in f32), one conversion each
 #pragma unroll
-    for (int j = 0; j < 8; ++j) q[j] = fminf(roundf(__fdiv_rn(a[j], scale)), maxq);
-  }
-  uint32_t code[8];
+    for (int i = 0; i < NW; ++i) {
+      uint32_t hw[2];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) code[j] = (uint32_t)(int32_t)q[j] & ((1u << BITS) - 1u);
-  if constexpr (BITS == 4) {
-    uint32_t o = 0;
+      for (int h = 0; h < 2; ++h) {
+        const float* qq = q + (2 * i + h) * CPH;
+        float t = qq[CPH - 1];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) o |= code[j] << (4 * j);
-    wq[c] = o;
-  } else if constexpr (BITS == 8) {
-    u32x2 o = {0u, 0u};
-#pragma unroll
-    for (int j = 0; j < 8; ++j) o[j / 4] |= code[j] << (8 * (j % 4));
-    *reinterpret_cast<u32x2*>(wq + c * 2) = o;
+        for (int e = CPH - 2; e >= 0; --e) t = fmaf(t, (float)(1u << BITS), qq[e]);
+        hw[h] = (uint32_t)t;
+      }
+      o[i] = hw[0] | (hw[1] << 16);
+    }
   } else {
-    uint32_t o = 0;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) o |= code[j] << (2 * j);
-    reinterpret_cast<uint16_t*>(wq)[c] = (uint16_t)o;
+    for (int i = 0; i < NW; ++i) {
+      o[i] = 0;
+#pragma unroll
+      for (int e = 0; e < 2 * CPH; ++e) {
+        const float qf = fminf(roundf(__fdiv_rn(__fsub_rn(v[2 * CPH * i + e], bias), scale)), maxq);
+        o[i] |= ((uint32_t)(int32_t)qf & ((1u << BITS) - 1u)) << (e * BITS);
+      }
+    }
   }
+  if constexpr (NW == 4) *reinterpret_cast<u32x4*>(wq + c * 4) = u32x4{o[0], o[1], o[2], o[3]};
+  else if constexpr (NW == 2) *reinterpret_cast<u32x2*>(wq + c * 2) = u32x2{o[0], o[1]};
+  else wq[c] = o[0];
   if (c % L == 0) {
     store_from_f32(scales, c / L, scale);
     store_from_f32(biases, c / L, bias);
@@ -226,11 +243,11 @@ __global__ __launch_bounds__(256) void quant8_kernel(const T* __restrict__ w, ui
 }
 
 template <typename T, int BITS>
-static void launch_quant8(hipStream_t st, const T* w, uint32_t* wq, T* s, T* b, int64_t nchunks, int gs) {
+static void launch_quant16(hipStream_t st, const T* w, uint32_t* wq, T* s, T* b, int64_t nchunks, int gs) {
   const dim3 grid((unsigned)((nchunks + 255) / 256));
-  if (gs == 32) hipLaunchKernelGGL((quant8_kernel<T, BITS, 32>), grid, dim3(256), 0, st, w, wq, s, b, nchunks);
-  else if (gs == 64) hipLaunchKernelGGL((quant8_kernel<T, BITS, 64>), grid, dim3(256), 0, st, w, wq, s, b, nchunks);
-  else hipLaunchKernelGGL((quant8_kernel<T, BITS, 128>), grid, dim3(256), 0, st, w, wq, s, b, nchunks);
+  if (gs == 32) hipLaunchKernelGGL((quant16_kernel<T, BITS, 32>), grid, dim3(256), 0, st, w, wq, s, b, nchunks);
+  else if (gs == 64) hipLaunchKernelGGL((quant16_kernel<T, BITS, 64>), grid, dim3(256), 0, st, w, wq, s, b, nchunks);
+  else hipLaunchKernelGGL((quant16_kernel<T, BITS, 128>), grid, dim3(256), 0, st, w, wq, s, b, nchunks);
 }
 
 template <typename T>
@@ -238,14 +255,14 @@ static int launch_quantize_t(hipStream_t st, const T* w, uint32_t* wq, T* s, T* 
                              int bits) {
   const int64_t ngroups = rows * (K / gs);
   if (ngroups == 0) return LISAQ_OK;
-  // eight values per thread where the group sizes and alignments of the packed
+  // sixteen values per thread where the group sizes and alignments of the packed
   // format's layers allow its loads and stores; anything else a thread per group
-  const bool al = (uintptr_t)w % 16 == 0 && (uintptr_t)wq % 8 == 0;
-  if (al && (gs == 32 || gs == 64 || gs == 128) && ngroups * gs / 8 <= (int64_t)1 << 38) {
-    const int64_t nchunks = ngroups * gs / 8;
-    if (bits == 4) launch_quant8<T, 4>(st, w, wq, s, b, nchunks, gs);
-    else if (bits == 2) launch_quant8<T, 2>(st, w, wq, s, b, nchunks, gs);
-    else launch_quant8<T, 8>(st, w, wq, s, b, nchunks, gs);
+  const bool al = (uintptr_t)w % 16 == 0 && (uintptr_t)wq % 16 == 0;
+  if (al && (gs == 32 || gs == 64 || gs == 128) && ngroups * gs / kQuantVals <= (int64_t)1 << 38) {
+    const int64_t nchunks = ngroups * gs / kQuantVals;
+    if (bits == 4) launch_quant16<T, 4>(st, w, wq, s, b, nchunks, gs);
+    else if (bits == 2) launch_quant16<T, 2>(st, w, wq, s, b, nchunks, gs);
+    else launch_quant16<T, 8>(st, w, wq, s, b, nchunks, gs);
     return check_launch("quantize");
   }
   hipLaunchKernelGGL(quant_kernel<T>, dim3((unsigned)((ngroups + 255) / 256)), dim3(256), 0, st, w, wq, s, b, ngroups,
