@@ -622,9 +622,9 @@ int lisaq_quantized_matmul_typed(void* stream, const void* x, const uint32_t* w,
   const bool matvec = M < lisaq_qmv_batch_limit(K, N);
   // f16 and 8-bit matmuls on the bf16 matmul's kernel (measured, f16 4-bit
   // 1000 x 5120 x 5120: 217 us on qmm_typed_mfma_kernel, 69 us here).  Its
-  // scale/bias copies are 16 bytes of a row at dword granularity, so rows of
-  // an even number of groups from a dword on; other rows and addresses, and
-  // sizes past its 32-bit offsets, stay on the kernels of qtyped.hip.
+  // scale/bias copies are 16 bytes of a row from a dword on: other addresses,
+  // sizes past its 32-bit offsets and rows of an odd number of groups (which the
+  // kernel takes, not measured here) stay on the kernels of qtyped.hip.
   if (!matvec && dtype != LISAQ_DTYPE_F32 && K % 64 == 0 && K / gs % 2 == 0 && aligned(x, 16) && aligned(w, 16) &&
       aligned(s, 4) && aligned(b, 4) && aligned(y, 4) && M * K < ((int64_t)1 << 31) &&
       N * K * bits / 8 < ((int64_t)1 << 32)) {

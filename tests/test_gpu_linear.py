@@ -523,3 +523,40 @@ def test_native_call_path(dev, dtype, bits, M):
         y = ops.quantized_matmul(x, w, s, b, True, gs, bits)
     side.synchronize()
     assert torch.equal(y, ref)
+
+
+@pytest.mark.parametrize("bits", [4, 2])
+@pytest.mark.parametrize("M,N,K,gs", [
+    (40, 1, 64, 64),         # one group in all
+    (40, 264, 64, 64),       # one group a row
+    (20, 264, 320, 64),      # five groups a row: one scale/bias block
+    (100, 77, 384, 128),     # three groups of 128
+    (300, 260, 960, 64),     # fifteen: the last block holds seven
+    (33, 300, 576, 64),      # nine: the last block holds one
+    (100, 513, 2880, 64),    # 45 groups, split over K
+    (300, 100, 1152, 128),   # nine groups of 128
+    (700, 516, 320, 64),     # several row tiles
+    (4352, 4352, 1088, 64),  # 17 groups, 17 x 17 tiles: 256-row tiles, the last round split over K
+])
+def test_matmul_odd_group_counts(dev, oracle, M, N, K, gs, bits):
+    """Rows of an odd number of groups: the scales of the matrix's last row end off a dword, and its last group counts
+    like any other -- every column against the oracle's arithmetic in float64, with and without a workspace."""
+    import torch
+
+    from lisa_amd import _lib
+
+    rng = np.random.default_rng(M + N + K + bits)
+    w, s, b = np_linear(rng, N, K, bits, gs, s_std=0.02 if bits == 4 else 0.05, s_floor=0.01)
+    x = np_x(rng, M, K)
+    xd, wd, sd, bd = to_dev_bf16(x, dev), to_dev_u32(w, dev), to_dev_bf16(s, dev), to_dev_bf16(b, dev)
+    cols = np.unique(np.r_[np.arange(min(N, 40)), np.arange(max(N - 40, 0), N), rng.integers(0, N, 40)])
+    ref = oracle.qmm_typed(bf16_bits_to_f32(x), w[cols], bf16_bits_to_f32(s)[cols], bf16_bits_to_f32(b)[cols], gs,
+                           bits, "bf16").astype(np.float32)
+    got = from_dev_bf16(ops.qmm(xd, wd, sd, bd, gs, bits))
+    assert_close_bf16(got[:, cols], ref, what=f"qmm M={M} N={N} K={K} bits={bits} gs={gs}")
+    y = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
+    _lib.call("lisaq_qmm", torch.cuda.current_stream().cuda_stream, xd.data_ptr(), wd.data_ptr(), sd.data_ptr(),
+              bd.data_ptr(), y.data_ptr(), M, N, K, gs, bits, None, 0)
+    assert_close_bf16(from_dev_bf16(y)[:, cols], ref, what=f"unsplit M={M} N={N} K={K} bits={bits} gs={gs}")
+    if M >= ops.qmv_batch_limit(K, N):
+        assert np.array_equal(from_dev_bf16(ops.quantized_matmul(xd, wd, sd, bd, True, gs, bits)), got)

@@ -570,3 +570,35 @@ def test_moe_forward_tile_height_rule(dev, T, bits):
     d = ops.gather_qmm(ops.swiglu(g, u), *dv[2], rhs_indices=srt, bits=bits)
     ref = ops.moe_combine(d, rw.reshape(-1), inv, T, k)
     assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
+
+
+@pytest.mark.parametrize("runs,N,K,gs,bits", [((300, 65, 33, 129, 1, 513, 70), 200, 320, 64, 4),
+                                              ((300, 65, 33, 129, 1, 513, 70), 200, 320, 64, 2),
+                                              ((200, 300, 40, 257), 264, 576, 64, 4),
+                                              ((128, 64, 90), 96, 384, 128, 4)])
+def test_gather_odd_group_counts(dev, oracle, runs, N, K, gs, bits):
+    """Expert stacks whose rows have an odd number of groups: every expert's last column (whose last scale ends off a
+    dword) through the tall, 128-row and short tiles of gather_qmm and gather_qmm_swiglu, against the oracle."""
+    rng = np.random.default_rng(sum(runs) + K + bits)
+    E = len(runs)
+    stk = lambda: tuple(a.reshape(E, N, -1) for a in np_linear(rng, E * N, K, bits, gs, s_floor=0.01))
+    W, U = stk(), stk()
+    ids = np.repeat(np.arange(E, dtype=np.int32), runs)
+    R, T = ids.size, 500
+    xt = np_x(rng, T, K)
+    rows = rng.integers(0, T, R).astype(np.int32)
+    x = xt[rows]
+    dw, du = (tuple(to_dev_u32(a, dev) if i == 0 else to_dev_bf16(a, dev) for i, a in enumerate(st)) for st in (W, U))
+    sid = to_dev(ids, dev)
+    y = from_dev_bf16(ops.gather_qmm(to_dev_bf16(x, dev), *dw, rhs_indices=sid, group_size=gs, bits=bits))
+    act = from_dev_bf16(ops.gather_qmm_swiglu(to_dev_bf16(xt, dev), to_dev(rows, dev), dw, du, sid, gs, bits))
+    lim, a = ops.qmv_batch_limit(K, N), 0
+    for e, n in enumerate(runs):
+        b = a + n
+        g = oracle.qmm(x[a:b], W[0][e], W[1][e], W[2][e], gs, bits)
+        ref = g if n >= lim else oracle.qmv(x[a:b], W[0][e], W[1][e], W[2][e], gs, bits)
+        assert_close_bf16(y[a:b], ref, what=f"gather_qmm expert {e} ({n} rows)")
+        u = oracle.f32_to_bf16(oracle.qmm(x[a:b], U[0][e], U[1][e], U[2][e], gs, bits))
+        ref = bf16_bits_to_f32(oracle.swiglu(oracle.f32_to_bf16(g), u))
+        assert_close_bf16(act[a:b], ref, rtol=2e-2, what=f"gather_qmm_swiglu expert {e} ({n} rows)")
+        a = b
