@@ -18,9 +18,8 @@
 //    with the group's scale/bias, v_cvt_pk_bf16_f32.
 //  * The next K-step's x tile and W words are fetched while the current one
 //    runs on the matrix cores.
-// Compute types: bf16 and f16 (CT), 2-, 4- and 8-bit codes.  f16 weights are one
-// v_fma_mixlo/mixhi_f16 per code after the unpack, bf16 ones an fma and half
-// a pack: f16 4-bit 1000 x 5120 x 5120 takes 69 us (758 TFLOP/s; on the
+// Compute types: bf16 and f16 (CT), 2-, 4- and 8-bit codes.  A weight is an
+// fma and half a packed conversion (Ct::pk) after the unpack: f16 4-bit 1000 x 5120 x 5120 takes 69 us (758 TFLOP/s; on the
 // separate 64 x 64 typed tiles 217 us), bf16 8-bit 73 us.
 #pragma once
 #include "lisaq_common.h"
@@ -68,12 +67,14 @@ template <>
 struct Ct<kCtF16> {
   static __device__ __forceinline__ float f(uint16_t h) { return (float)__builtin_bit_cast(_Float16, h); }
   static __device__ __forceinline__ uint32_t pk(float a, float b) {
-    // (the instruction named: from the conversions the compiler forms
-    // v_fma_mixlo/mixhi_f16 with the fma before them, 7.5 cycles of a SIMD
-    // each against 4.2 for v_fma_mix_f32 and for this)
-    uint32_t v;
-    asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(v) : "v"(a), "v"(b));
-    return v;
+    // (both values opaque: the compiler otherwise joins each conversion with the
+    // fma before it to v_fma_mixlo/mixhi_f16, 7.5 cycles of a SIMD each against
+    // 4.2 for v_fma_mix_f32 and for the v_cvt_pk_f16_f32 formed here.  The
+    // conversion itself is not inline asm: the compiler must see the write to
+    // keep two wait states before a matrix instruction that reads it.)
+    asm("" : "+v"(a), "+v"(b));
+    f16x2_t v = {(_Float16)a, (_Float16)b};
+    return __builtin_bit_cast(uint32_t, v);
   }
   static __device__ __forceinline__ uint16_t one(float v) { return __builtin_bit_cast(uint16_t, (_Float16)v); }
   static __device__ __forceinline__ f32x16 mfma(u32x4 a, u32x4 b, f32x16 c) {
@@ -86,7 +87,6 @@ struct Ct<kCtF16> {
 // codes as f16 denormals (value q * 2^-24): with s24 = s * 2^24 (exact),
 // v_fma_mix_f32 forms s24 * (q * 2^-24) + b, whose product equals s * q
 // exactly, so each result is fmaf(s, q, b) bit for bit (|s| < 2^104).
-// (f16 weights: the fma and its rounding are one v_fma_mixlo/mixhi_f16 each.)
 template <int CT = kCtBf16>
 __device__ __forceinline__ uint32_t deq_pair(uint32_t pair, float s24, float b) {
   const f16x2_t hv = __builtin_bit_cast(f16x2_t, pair);
