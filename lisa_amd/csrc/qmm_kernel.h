@@ -464,24 +464,27 @@ __global__ __launch_bounds__(64 * WN * WM) void qmm_kernel(QmmParams p) {
   };
   // An odd number of groups puts every other row off a dword, and the last
   // group of the matrix's last row into a dword that straddles the array's
-  // end, which the descriptor's range check returns as zero.  So the last block of
-  // such rows is copied two bytes early: its groups (at most seven) then lie two
-  // bytes further on in the block, and every dword of a row's groups ends
-  // with the row.  All rows alike, so it costs scalar instructions only (2048
-  // rows of 17408 x 5120 317.1 -> 317.6 us, 203 rows of 5120 x 17408 56.7 -> 56.4).
-  // A single block (fewer than eight groups) has nothing before its first row:
-  // its last group is stored on its own below.
-  const int sb_odd = GS > 32 && (p.G & 1) && p.G > 8 ? p.G >> 3 : -1;
-  // scale/bias block sb (groups 8 sb .. 8 sb + 7 of every row; past a row's
-  // end: the next row's groups or zeros, never used) into block buffer sb % 2
-  auto issue_sb = [&](int sb) {
+  // end, which the descriptor's range check returns as zero.  So such rows are
+  // cut into blocks from their end: block 0 starts `pad` groups before the row
+  // and every dword of a row's blocks ends with the row.  Steps count from
+  // kbs where scales and biases are meant, and the loop does the same work either
+  // way (a two-byte shift of the last block alone cost it three scalar
+  // instructions a step, 500 x 5120 x 5120 42.1 -> 42.5 us).  Nothing before row 0
+  // is read: the first rows' block 0 is put together in the prologue.
+  const int pad = GS > 32 && (p.G & 1) ? 8 - (p.G & 7) : 0;
+  const int kbs = kb + pad * (GS / BK);
+  // scale/bias block sb (groups 8 sb - pad .. 8 sb - pad + 7 of every row; past
+  // its ends: other rows' groups or zeros, never used) into block buffer sb % 2
+  auto issue_sb = [&](int sb, auto zero) {  // (zero: sb may be 0)
+    const bool b0 = decltype(zero)::value && sb == 0;
     unsigned char* st = smem + L::SB0 + (sb & 1) * L::SBB;
 #pragma unroll
     for (int q = 0; q < SBI; ++q) {
       const int idx = wave + NWV * q;  // 0 .. 2*SI-1: s row blocks, then b row blocks
       const bool is_b = idx >= SI;
       const int blk = is_b ? idx - SI : idx;
-      buf_lds16(rsb[q], sbrow[q] * 2u, (uint32_t)(sb * 16 - (sb == sb_odd ? 2 : 0)),
+      const uint32_t row = b0 && sbrow[q] >= (uint32_t)pad ? sbrow[q] - (uint32_t)pad : sbrow[q];
+      buf_lds16(rsb[q], row * 2u, b0 ? 0u : (uint32_t)(sb * 8 - pad) * 2u,
                 st + (is_b ? L::SBA : 0) + blk * 64 * 16);
     }
   };
@@ -499,9 +502,8 @@ __global__ __launch_bounds__(64 * WN * WM) void qmm_kernel(QmmParams p) {
     const int e = kl & 1;  // step within the pair
     // the lane's group (gs 32: the step's two groups, one per half-wave) and
     // its block buffer
-    const int g = (kb + kl) * BK / GS + (GS == 32 ? h : 0);
-    const int early = GS > 32 && (g >> 3) == sb_odd ? 2 : 0;
-    const unsigned char* sbb = smem + L::SB0 + ((g >> 3) & 1) * L::SBB + (g & 7) * 2 + early;
+    const int g = (kbs + kl) * BK / GS + (GS == 32 ? h : 0);
+    const unsigned char* sbb = smem + L::SB0 + ((g >> 3) & 1) * L::SBB + (g & 7) * 2;
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
       const int r = (wn * NT + nt) * 32 + col;
@@ -559,12 +561,12 @@ __global__ __launch_bounds__(64 * WN * WM) void qmm_kernel(QmmParams p) {
   };
   uint32_t bA[NT][16], bB[NT][16];  // B operands of the current / next step
   // scale/bias blocks: the first two in the prologue; block sb + 1 during
-  // step sb * SBK - 1 (global steps), after the last read of block sb - 1
+  // step sb * SBK - 1 (steps from kbs), after the last read of block sb - 1
   // (step sb * SBK - 3) and landed before the first read of block sb + 1
   // (step (sb + 1) * SBK - 2); none past the last step's block
-  const int sb_last = (kb + nk - 1) / SBK;
-  issue_sb(kb / SBK);
-  if (kb / SBK + 1 <= sb_last) issue_sb(kb / SBK + 1);
+  const int sb_last = (kbs + nk - 1) / SBK;
+  issue_sb(kbs / SBK, std::true_type{});
+  if (kbs / SBK + 1 <= sb_last) issue_sb(kbs / SBK + 1, std::false_type{});
   issue_x(kc(0), 0, 0, XI);
   issue_wpair(0, 0);
   issue_wpair(1, 1);
@@ -572,9 +574,10 @@ __global__ __launch_bounds__(64 * WN * WM) void qmm_kernel(QmmParams p) {
   // x(0), W pairs 0 and 1 landed (this wave's part; x(1) may be in flight)
   if (xshort) wait_vm<(VM_X > 1 ? VM_X - 1 : 0)>();
   else wait_vm<VM_X>();
-  // fewer than eight groups, an odd number of them: the lanes that copied the
-  // matrix's last row store its last group (the copy has landed)
-  if (GS > 32 && (p.G & 1) && p.G < 8) {
+  // an odd number of groups: the lanes whose row starts fewer than `pad` groups
+  // into the array (and was copied from its start) put block 0's groups in
+  // their places (the copy has landed)
+  if (pad > 0 && kbs / SBK == 0) {
 #pragma unroll
     for (int q = 0; q < SBI; ++q) {
       const int idx = wave + NWV * q;
@@ -582,9 +585,9 @@ __global__ __launch_bounds__(64 * WN * WM) void qmm_kernel(QmmParams p) {
       const int blk = is_b ? idx - SI : idx;
       const bool up = GU && blk >= SI / 2;
       const uint16_t* base = is_b ? (up ? bi2 : bi) : (up ? sc2 : sc);
-      unsigned char* st = smem + L::SB0 + (is_b ? L::SBA : 0) + (blk * 64 + lane) * 16;
-      if (sbrow[q] == (uint32_t)(p.N - 1) * (uint32_t)p.G)
-        *reinterpret_cast<uint16_t*>(st + (p.G - 1) * 2) = base[(int64_t)p.N * p.G - 1];
+      uint16_t* st = reinterpret_cast<uint16_t*>(smem + L::SB0 + (is_b ? L::SBA : 0) + (blk * 64 + lane) * 16);
+      if (sbrow[q] < (uint32_t)pad)
+        for (int g = 0; g < 8 - pad; ++g) st[pad + g] = base[sbrow[q] + g];
     }
     wait_lgkm0();
   }
@@ -633,7 +636,7 @@ __global__ __launch_bounds__(64 * WN * WM) void qmm_kernel(QmmParams p) {
     // scale/bias block sb + 1 is copied during global step sb * SBK - 1, at
     // the earliest one step after the prologue's reads (a first step at
     // sb * SBK - 1 defers it to the next)
-    const int kq = (kt == 1 && (kb + 1) % SBK == 0) ? kb + 1 : kb + kt + 1;
+    const int kq = (kt == 1 && (kbs + 1) % SBK == 0) ? kbs + 1 : kbs + kt + 1;
     const int sb_next = kq / SBK + 1;
     const bool sb_now = kt >= 1 && kq % SBK == 0 && sb_next <= sb_last;
     static_for<SLOTS>([&](auto SI) {
@@ -682,7 +685,7 @@ __global__ __launch_bounds__(64 * WN * WM) void qmm_kernel(QmmParams p) {
       // scale/bias block (every SBK steps), then copies: copy q at slot
       // q * (3 NMF) / NCOPY
       if constexpr (sl == 0) {
-        if (sb_now) issue_sb(sb_next);
+        if (sb_now) issue_sb(sb_next, std::false_type{});
       }
       static_for<NCOPY>([&](auto QI) {
         constexpr int q = decltype(QI)::value;
