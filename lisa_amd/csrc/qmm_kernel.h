@@ -98,10 +98,25 @@ __device__ __forceinline__ uint32_t pair_bytes(uint32_t lo, uint32_t hi) {
   return __builtin_amdgcn_perm(hi, lo, (0x0Cu << 24) | ((4u + I) << 16) | (0x0Cu << 8) | (uint32_t)I);
 }
 
-// Codes 2 I and 2 I + 1 of a word of 8-bit codes, each into one half.
-template <int I>
-__device__ __forceinline__ uint32_t pair_code8(uint32_t w) {
-  return __builtin_amdgcn_perm(0u, w, (0x0Cu << 24) | ((2u * I + 1u) << 16) | (0x0Cu << 8) | (2u * I));
+// Scale operand of the pairs: s * 2^24 (deq_pair).  8-bit codes of bf16 matmuls
+// take s itself: every bf16 scale counts there, and s * 2^24 overflows from |s|
+// = 2^104 on.
+template <int BITS, int CT>
+__device__ __forceinline__ float deq_scale(float s) {
+  return BITS == 8 && CT == kCtBf16 ? s : s * 16777216.0f;
+}
+// Two weights from codes 2 I and 2 I + 1 of a word of 8-bit codes (s: deq_scale).
+// bf16: byte conversions and plain fmas, five operations against four (1000 x
+// 5120 x 5120 64.8 -> 66.2 us, 24 rows of 17408 x 5120 27.2 -> 27.8, 25 of 9728 x 2560
+// 12.8 -> 13.0; choosing by a wave-uniform branch in the few-rows matmul took the
+// same time).  f16 this way: 1000 x 5120 x 5120 68.0 -> 70.1 us.
+template <int I, int CT>
+__device__ __forceinline__ uint32_t deq_pair8(uint32_t w, float s, float b) {
+  if constexpr (CT == kCtBf16)
+    return Ct<CT>::pk(fmaf(s, (float)((w >> (16 * I)) & 0xFFu), b), fmaf(s, (float)((w >> (16 * I + 8)) & 0xFFu), b));
+  else
+    return deq_pair<CT>(__builtin_amdgcn_perm(0u, w, (0x0Cu << 24) | ((2u * I + 1u) << 16) | (0x0Cu << 8) | (2u * I)),
+                        s, b);
 }
 
 template <typename F, int... I>
@@ -115,16 +130,17 @@ __device__ __forceinline__ void static_for(F&& f) {
 }
 
 // All codes of a word as pairs of weights in natural K order (16 / words-per-32-codes of them).
+// (s: deq_scale of the group's scale)
 template <int BITS, int CT>
-__device__ __forceinline__ void deq_word(uint32_t wv, float s24, float b, uint32_t* o) {
+__device__ __forceinline__ void deq_word(uint32_t wv, float s, float b, uint32_t* o) {
   if constexpr (BITS == 8) {
-    o[0] = deq_pair<CT>(pair_code8<0>(wv), s24, b);
-    o[1] = deq_pair<CT>(pair_code8<1>(wv), s24, b);
+    o[0] = deq_pair8<0, CT>(wv, s, b);
+    o[1] = deq_pair8<1, CT>(wv, s, b);
   } else if constexpr (BITS == 4) {
     const uint32_t lo = opaque(wv & 0x0F0F0F0Fu), hi = opaque((wv >> 4) & 0x0F0F0F0Fu);
     static_for<4>([&](auto PI) {
       constexpr int d = decltype(PI)::value;
-      o[d] = deq_pair<CT>(pair_bytes<d>(lo, hi), s24, b);
+      o[d] = deq_pair<CT>(pair_bytes<d>(lo, hi), s, b);
     });
   } else {
     uint32_t c[4];
@@ -132,7 +148,7 @@ __device__ __forceinline__ void deq_word(uint32_t wv, float s24, float b, uint32
     for (int q = 0; q < 4; ++q) c[q] = opaque((wv >> (2 * q)) & 0x03030303u);
     static_for<8>([&](auto PI) {
       constexpr int d = decltype(PI)::value, m = d / 2, e = (d % 2) * 2;
-      o[d] = deq_pair<CT>(pair_bytes<m>(c[e], c[e + 1]), s24, b);
+      o[d] = deq_pair<CT>(pair_bytes<m>(c[e], c[e + 1]), s, b);
     });
   }
 }
@@ -527,10 +543,10 @@ __global__ __launch_bounds__(64 * WN * WM) void qmm_kernel(QmmParams p) {
   auto dequant_all = [&](const WLane& r, uint32_t (*bop)[16]) {
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
-      const float s24 = sf(r, nt) * 16777216.0f, b_ = bf(r, nt);
+      const float s_ = deq_scale<BITS, CT>(sf(r, nt)), b_ = bf(r, nt);
       static_for<G::WPL>([&](auto WI_) {
         constexpr int jw = decltype(WI_)::value;
-        deq_word<BITS, CT>(word(r, nt, jw), s24, b_, &bop[nt][jw * (16 / G::WPL)]);
+        deq_word<BITS, CT>(word(r, nt, jw), s_, b_, &bop[nt][jw * (16 / G::WPL)]);
       });
     }
   };
@@ -704,9 +720,9 @@ __global__ __launch_bounds__(64 * WN * WM) void qmm_kernel(QmmParams p) {
         if constexpr (d * SLOTS / NPIECE == sl) {
           constexpr int dnt = d / (G::WPL * PPW), dw = d / PPW % G::WPL, dp = d % PPW;
           const uint32_t wv = word(wn, dnt, dw);
-          const float s_ = sf(wn, dnt) * 16777216.0f, b_ = bf(wn, dnt);
+          const float s_ = deq_scale<BITS, CT>(sf(wn, dnt)), b_ = bf(wn, dnt);
           if constexpr (BITS == 8) {
-            bnxt[dnt][dw * 2 + dp] = opaque(deq_pair<CT>(pair_code8<dp>(wv), s_, b_));
+            bnxt[dnt][dw * 2 + dp] = opaque(deq_pair8<dp, CT>(wv, s_, b_));
           } else if constexpr (BITS == 4) {
             if constexpr (dp == 0) {
               lo[dnt][dw] = opaque(wv & 0x0F0F0F0Fu);

@@ -188,11 +188,11 @@ __global__ __launch_bounds__(1024) void qmm_rows_kernel(QmmParams p) {
         for (int mt = 0; mt < MT; ++mt)
           av[j][mt] = *reinterpret_cast<const u32x4*>(xs + x_lds_off(mt * 32 + col, 4 * h + j));
       __builtin_amdgcn_sched_barrier(0);
-      const float s24 = C::f(sv) * 16777216.0f, bs = C::f(bv);
+      const float s_ = deq_scale<BITS, CT>(C::f(sv)), bs = C::f(bv);
       uint32_t bop[16];
       static_for<WPL>([&](auto JI) {
         constexpr int j = decltype(JI)::value;
-        deq_word<BITS, CT>(wv[j], s24, bs, &bop[j * (16 / WPL)]);
+        deq_word<BITS, CT>(wv[j], s_, bs, &bop[j * (16 / WPL)]);
       });
 #pragma unroll
       for (int j = 0; j < 4; ++j)

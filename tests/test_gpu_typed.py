@@ -235,3 +235,27 @@ def test_f32_matmul_matrix_cores(dev, oracle, bits, M, N, K, gs):
     bound = 2.0**-24 * (K * np.abs(xf).astype(np.float64) @ np.abs(wd).T / np.sqrt(K) + np.abs(ref))
     assert (np.abs(y - ref) <= 4 * bound).all()
     assert np.linalg.norm(y - ref) <= 1e-6 * np.linalg.norm(ref) * max(1.0, np.sqrt(K / 1024))
+
+
+@pytest.mark.parametrize("M,N,K,gs", [(25, 264, 2176, 64), (40, 100, 384, 64), (150, 300, 256, 128), (700, 264, 512, 32)])
+def test_bf16_8bit_matmul_scale_range(dev, oracle, M, N, K, gs):
+    """bf16 scales over their whole range (2^104 and more among them) with 8-bit codes: every weight is
+    bf16(fma(scale, q, bias)), finite wherever that is, for code 0 too."""
+    import torch
+
+    rng = np.random.default_rng(M + N + K)
+    w, s, b = np_linear(rng, N, K, 8, gs, s_std=0.002)
+    w[:, ::3] &= np.uint32(0xFFFF00FF)  # zeros among the codes
+    sf, bf = bf16_bits_to_f32(s).copy(), bf16_bits_to_f32(b)
+    sf[3], sf[N // 2], sf[N - 1] = 2.0**104, -(2.0**108), 1.5 * 2.0**106
+    sf[5], bf = 2.0**-120, bf.copy()
+    xf = oracle._round_to(rng.standard_normal((M, K)).astype(np.float32), "bf16")
+    assert M >= ops.qmv_batch_limit(K, N)
+    y = ops.quantized_matmul(_tensor(xf, "bf16", dev), to_dev_u32(w, dev), _tensor(sf, "bf16", dev),
+                             _tensor(bf, "bf16", dev), True, gs, 8).float().cpu().numpy().astype(np.float64)
+    ref = oracle.qmm_typed(xf, w, sf, bf, gs, 8, "bf16")
+    # one rounding to bf16 (2^-9 relative) and f32 sums of K products (K 2^-24 of the sum of magnitudes)
+    q = oracle.unpack(w, K, 8).astype(np.float64)
+    wt = np.abs(np.repeat(sf.astype(np.float64), gs, 1) * q + np.repeat(bf.astype(np.float64), gs, 1))
+    bound = 2.0**-8 * np.abs(ref) + K * 2.0**-24 * (np.abs(xf).astype(np.float64) @ wt.T)
+    assert np.isfinite(y).all() and (np.abs(y - ref) <= bound).all()
