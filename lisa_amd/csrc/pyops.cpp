@@ -11,7 +11,10 @@
 // the way -- or where the C ABI reports an error; ops.py then takes its own
 // path, which converts, raises the op's errors, or hands the mode what it
 // expects.  Nothing is kept between calls.  Split-K partials come from torch's
-// allocator, in the order of the caller's stream.
+// allocator and go back when the call returns, in the order of the caller's
+// stream.  A captured call's replays write them again, and only a capture that
+// torch began keeps freed memory to itself: under any capture they share the
+// output's storage and live as long as it does.
 #include <Python.h>
 #include <ATen/TensorSubclassLikeUtils.h>
 #include <ATen/core/TensorBase.h>
@@ -81,9 +84,30 @@ Tensor output(const Tensor& x, int64_t N) {
   return at::empty(sizes, x.options());
 }
 
-Tensor scratch(const Tensor& x, size_t bytes) {
-  return at::empty({(int64_t)bytes}, x.options().dtype(at::kByte));
-}
+// The output [..., N] of x and `bytes` of scratch for the call's launches
+struct Outputs {
+  Tensor y, ws;
+  void* wp = nullptr;
+  Outputs(const Tensor& x, int64_t N, size_t bytes, void* stream) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (bytes && hipStreamIsCapturing(static_cast<hipStream_t>(stream), &st) == hipSuccess &&
+        st != hipStreamCaptureStatusNone) {
+      c10::SmallVector<int64_t, 5> sizes(x.sizes().begin(), x.sizes().end());
+      sizes.back() = N;
+      const int64_t ybytes = (x.numel() / x.size(-1) * N * (int64_t)x.element_size() + 255) / 256 * 256;
+      ws = at::empty({ybytes + (int64_t)bytes}, x.options().dtype(at::kByte));
+      wp = static_cast<char*>(ws.data_ptr()) + ybytes;
+      y = at::empty({0}, x.options());
+      y.set_(ws.storage(), 0, sizes);
+      return;
+    }
+    if (bytes) {
+      ws = at::empty({(int64_t)bytes}, x.options().dtype(at::kByte));
+      wp = ws.data_ptr();
+    }
+    y = output(x, N);
+  }
+};
 
 #define LISAQ_NONE_UNLESS(cond) \
   if (!(cond)) Py_RETURN_NONE
@@ -109,11 +133,10 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   size_t bytes = 0;
   if (!typed || (code != LISAQ_DTYPE_F32 && M >= lisaq_qmv_batch_limit(K, N)))
     bytes = lisaq_quantized_matmul_workspace(M, N, K, (int)gs, (int)bits);
-  Tensor ws;
-  if (bytes) ws = scratch(*x, bytes);
-  void* const wp = bytes ? ws.data_ptr() : nullptr;
-  Tensor y = output(*x, N);
   void* const st = stream_of(*x);
+  Outputs o(*x, N, bytes, st);
+  Tensor& y = o.y;
+  void* const wp = o.wp;
   int rc;
   if (typed)
     rc = lisaq_quantized_matmul_typed(st, x->data_ptr(), q.codes_ptr(), q.s->data_ptr(), q.b->data_ptr(),
@@ -143,13 +166,12 @@ PyObject* addnorm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int64_t M = x->size(0), K = x->size(1), N = q.w->size(0);
   LISAQ_NONE_UNLESS(M > 0 && K > 0 && N > 0 && nw->numel() == K && q.shape(N, K, gs, bits));
   const size_t bytes = lisaq_quantized_matmul_workspace(M, N, K, (int)gs, (int)bits);
-  Tensor ws;
-  if (bytes) ws = scratch(*x, bytes);
-  Tensor y = output(*x, N), sum = output(*x, K), normed = output(*x, K);
-  const int rc = lisaq_qmv_addnorm(stream_of(*x), x->data_ptr(), r->data_ptr(), nw->data_ptr(), q.codes_ptr(),
+  void* const st = stream_of(*x);
+  Outputs o(*x, N, bytes, st);
+  Tensor &y = o.y, sum = output(*x, K), normed = output(*x, K);
+  const int rc = lisaq_qmv_addnorm(st, x->data_ptr(), r->data_ptr(), nw->data_ptr(), q.codes_ptr(),
                                    q.s->data_ptr(), q.b->data_ptr(), sum.data_ptr(), normed.data_ptr(), y.data_ptr(),
-                                   M, N, K, (float)PyFloat_AS_DOUBLE(a[6]), (int)gs, (int)bits,
-                                   bytes ? ws.data_ptr() : nullptr, bytes);
+                                   M, N, K, (float)PyFloat_AS_DOUBLE(a[6]), (int)gs, (int)bits, o.wp, bytes);
   LISAQ_NONE_UNLESS(rc == LISAQ_OK);
   PyObject* out = PyTuple_New(3);
   if (!out) return nullptr;

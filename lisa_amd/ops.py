@@ -164,13 +164,22 @@ def _mm_typed(x, w, scales, biases, transpose, group_size, bits, dt):
              f"quantized_matmul: w {tuple(w.shape)} does not match K={K}, bits={bits}")
     _require(scales.shape == (N, K // group_size) and biases.shape == scales.shape, _lib.EINVAL_SHAPE,
              f"quantized_matmul: scales/biases {tuple(scales.shape)} != ({N}, {K // group_size})")
-    y = torch.empty(*x.shape[:-1], N, dtype=dt, device=x.device)
     # split-K partials of the 16-bit matmuls: from torch's allocator, in the
     # order of the caller's stream (calls on several streams share nothing)
     nbytes = 0
     if dt != torch.float32 and M >= qmv_batch_limit(K, N):
         nbytes = _lib.load().lisaq_quantized_matmul_workspace(M, N, K, group_size, bits)
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device) if nbytes else None
+    with torch.cuda.device(x.device):
+        capturing = nbytes > 0 and torch.cuda.is_current_stream_capturing()
+    if capturing:
+        # (replays write the partials again: they live as long as the output, in its storage)
+        ybytes = -(-M * N * dt.itemsize // 256) * 256
+        buf = torch.empty(ybytes + nbytes, dtype=torch.uint8, device=x.device)
+        ws = buf[ybytes:]
+        y = torch.empty(0, dtype=dt, device=x.device).set_(buf.untyped_storage(), 0, (*x.shape[:-1], N))
+    else:
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device) if nbytes else None
+        y = torch.empty(*x.shape[:-1], N, dtype=dt, device=x.device)
     _lib.call("lisaq_quantized_matmul_typed", _stream(x), x.data_ptr(), w.data_ptr(), scales.data_ptr(),
               biases.data_ptr(), y.data_ptr(), M, N, K, 1, group_size, bits, _DTYPE_CODE[dt], _ptr(ws), nbytes)
     return y

@@ -560,3 +560,51 @@ def test_matmul_odd_group_counts(dev, oracle, M, N, K, gs, bits):
     assert_close_bf16(from_dev_bf16(y)[:, cols], ref, what=f"unsplit M={M} N={N} K={K} bits={bits} gs={gs}")
     if M >= ops.qmv_batch_limit(K, N):
         assert np.array_equal(from_dev_bf16(ops.quantized_matmul(xd, wd, sd, bd, True, gs, bits)), got)
+
+
+@pytest.mark.parametrize("dtype,bits,strided", [("bf16", 4, False), ("f16", 4, False), ("bf16", 8, True)])
+def test_scratch_of_a_capture_begun_outside_torch(dev, dtype, bits, strided):
+    """A stream capture that torch did not begin has no memory pool of its own: the split-K scratch of a captured call
+    stays allocated as long as its output, and replays leave other tensors alone.  (strided: the Python call path)"""
+    import ctypes
+
+    import torch
+
+    path = next(l.split()[-1] for l in open("/proc/self/maps") if "libamdhip64" in l)
+    hip = ctypes.CDLL(path)
+    M, N, K, gs = 30, 1024, 5120, 64
+    dt = torch.float16 if dtype == "f16" else torch.bfloat16
+    g = torch.Generator(device=dev)
+    g.manual_seed(bits)
+    w = torch.randint(-(2**31), 2**31, (N, K * bits // 32), dtype=torch.int32, device=dev, generator=g)
+    s, b = ((torch.randn(N, K // gs, device=dev, generator=g) * 0.01).to(dt) for _ in range(2))
+    x = torch.randn(M, K, device=dev, generator=g).to(dt)
+    arg = torch.stack([x, x], -1)[..., 0] if strided else x
+    from lisa_amd import _lib
+    need = _lib.load().lisaq_quantized_matmul_workspace(M, N, K, gs, bits)
+    assert need > M * N * 4 and M >= ops.qmv_batch_limit(K, N)
+    ref = ops.quantized_matmul(x, w, s, b, True, gs, bits)
+    st = torch.cuda.Stream()
+    st.wait_stream(torch.cuda.current_stream())
+    graph, exe = ctypes.c_void_p(), ctypes.c_void_p()
+    with torch.cuda.stream(st):
+        for _ in range(2):
+            ops.quantized_matmul(arg, w, s, b, True, gs, bits)
+        torch.cuda.synchronize()
+        held = torch.cuda.memory_allocated(dev)
+        assert hip.hipStreamBeginCapture(ctypes.c_void_p(st.cuda_stream), 1) == 0
+        y = ops.quantized_matmul(arg, w, s, b, True, gs, bits)
+        assert hip.hipStreamEndCapture(ctypes.c_void_p(st.cuda_stream), ctypes.byref(graph)) == 0
+        assert torch.cuda.memory_allocated(dev) - held >= M * N * 2 + need
+        assert y.is_contiguous() and y.storage_offset() == 0 and tuple(y.shape) == (M, N)
+        others = [torch.full((need,), 7, dtype=torch.uint8, device=dev) for _ in range(4)]
+    assert hip.hipGraphInstantiate(ctypes.byref(exe), graph, None, None, 0) == 0
+    for _ in range(3):
+        y.zero_()
+        torch.cuda.synchronize()
+        assert hip.hipGraphLaunch(exe, ctypes.c_void_p(st.cuda_stream)) == 0
+        torch.cuda.synchronize()
+        assert torch.equal(y, ref)
+        assert all(bool((o == 7).all()) for o in others)
+        assert torch.equal(ops.quantized_matmul(x, w, s, b, True, gs, bits), ref)
+    assert hip.hipGraphExecDestroy(exe) == 0 and hip.hipGraphDestroy(graph) == 0
