@@ -14,7 +14,9 @@
 // allocator and go back when the call returns, in the order of the caller's
 // stream.  A captured call's replays write them again, and only a capture that
 // torch began keeps freed memory to itself: under any capture they share the
-// output's storage and live as long as it does.
+// output's storage and live as long as it does.  The GIL is released over
+// allocation and launch, as a ctypes call does: either can wait for the driver
+// or for room in a full queue.
 #include <Python.h>
 #include <ATen/TensorSubclassLikeUtils.h>
 #include <ATen/core/TensorBase.h>
@@ -24,6 +26,8 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+
+#include <mutex>
 
 #include "../../include/lisaq.h"
 
@@ -109,6 +113,16 @@ struct Outputs {
   }
 };
 
+// The arguments' tensors stay alive without the GIL: the caller's frame holds them.
+class NoGil {
+  PyThreadState* const state_ = PyEval_SaveThread();
+
+ public:
+  NoGil() = default;
+  NoGil(const NoGil&) = delete;
+  ~NoGil() { PyEval_RestoreThread(state_); }
+};
+
 #define LISAQ_NONE_UNLESS(cond) \
   if (!(cond)) Py_RETURN_NONE
 
@@ -130,23 +144,26 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int64_t M = x->numel() / K;
   const bool typed = code != LISAQ_DTYPE_BF16 || bits == 8;
   LISAQ_NONE_UNLESS(!(typed && serial));
-  size_t bytes = 0;
-  if (!typed || (code != LISAQ_DTYPE_F32 && M >= lisaq_qmv_batch_limit(K, N)))
-    bytes = lisaq_quantized_matmul_workspace(M, N, K, (int)gs, (int)bits);
-  void* const st = stream_of(*x);
-  Outputs o(*x, N, bytes, st);
-  Tensor& y = o.y;
-  void* const wp = o.wp;
+  Tensor y;
   int rc;
-  if (typed)
-    rc = lisaq_quantized_matmul_typed(st, x->data_ptr(), q.codes_ptr(), q.s->data_ptr(), q.b->data_ptr(),
-                                      y.data_ptr(), M, N, K, 1, (int)gs, (int)bits, code, wp, bytes);
-  else if (serial)
-    rc = lisaq_quantized_matmul_serial_rows(st, x->data_ptr(), q.codes_ptr(), q.s->data_ptr(), q.b->data_ptr(),
-                                            y.data_ptr(), M, N, K, 1, (int)gs, (int)bits, wp, bytes);
-  else
-    rc = lisaq_quantized_matmul(st, x->data_ptr(), q.codes_ptr(), q.s->data_ptr(), q.b->data_ptr(), y.data_ptr(), M,
-                                N, K, 1, (int)gs, (int)bits, wp, bytes);
+  {
+    NoGil nogil;
+    size_t bytes = 0;
+    if (!typed || (code != LISAQ_DTYPE_F32 && M >= lisaq_qmv_batch_limit(K, N)))
+      bytes = lisaq_quantized_matmul_workspace(M, N, K, (int)gs, (int)bits);
+    void* const st = stream_of(*x);
+    Outputs o(*x, N, bytes, st);
+    if (typed)
+      rc = lisaq_quantized_matmul_typed(st, x->data_ptr(), q.codes_ptr(), q.s->data_ptr(), q.b->data_ptr(),
+                                        o.y.data_ptr(), M, N, K, 1, (int)gs, (int)bits, code, o.wp, bytes);
+    else if (serial)
+      rc = lisaq_quantized_matmul_serial_rows(st, x->data_ptr(), q.codes_ptr(), q.s->data_ptr(), q.b->data_ptr(),
+                                              o.y.data_ptr(), M, N, K, 1, (int)gs, (int)bits, o.wp, bytes);
+    else
+      rc = lisaq_quantized_matmul(st, x->data_ptr(), q.codes_ptr(), q.s->data_ptr(), q.b->data_ptr(), o.y.data_ptr(),
+                                  M, N, K, 1, (int)gs, (int)bits, o.wp, bytes);
+    y = std::move(o.y);
+  }
   LISAQ_NONE_UNLESS(rc == LISAQ_OK);
   return THPVariable_Wrap(std::move(y));
   END_HANDLE_TH_ERRORS
@@ -165,13 +182,20 @@ PyObject* addnorm(PyObject*, PyObject* const* a, Py_ssize_t n) {
                     q.read(a + 3, 2, at::kBFloat16, x->device()) && !modes_active());
   const int64_t M = x->size(0), K = x->size(1), N = q.w->size(0);
   LISAQ_NONE_UNLESS(M > 0 && K > 0 && N > 0 && nw->numel() == K && q.shape(N, K, gs, bits));
-  const size_t bytes = lisaq_quantized_matmul_workspace(M, N, K, (int)gs, (int)bits);
-  void* const st = stream_of(*x);
-  Outputs o(*x, N, bytes, st);
-  Tensor &y = o.y, sum = output(*x, K), normed = output(*x, K);
-  const int rc = lisaq_qmv_addnorm(st, x->data_ptr(), r->data_ptr(), nw->data_ptr(), q.codes_ptr(),
-                                   q.s->data_ptr(), q.b->data_ptr(), sum.data_ptr(), normed.data_ptr(), y.data_ptr(),
-                                   M, N, K, (float)PyFloat_AS_DOUBLE(a[6]), (int)gs, (int)bits, o.wp, bytes);
+  Tensor y, sum, normed;
+  int rc;
+  {
+    NoGil nogil;
+    const size_t bytes = lisaq_quantized_matmul_workspace(M, N, K, (int)gs, (int)bits);
+    void* const st = stream_of(*x);
+    Outputs o(*x, N, bytes, st);
+    sum = output(*x, K);
+    normed = output(*x, K);
+    rc = lisaq_qmv_addnorm(st, x->data_ptr(), r->data_ptr(), nw->data_ptr(), q.codes_ptr(), q.s->data_ptr(),
+                           q.b->data_ptr(), sum.data_ptr(), normed.data_ptr(), o.y.data_ptr(), M, N, K,
+                           (float)PyFloat_AS_DOUBLE(a[6]), (int)gs, (int)bits, o.wp, bytes);
+    y = std::move(o.y);
+  }
   LISAQ_NONE_UNLESS(rc == LISAQ_OK);
   PyObject* out = PyTuple_New(3);
   if (!out) return nullptr;
@@ -189,8 +213,14 @@ PyObject* swiglu(PyObject*, PyObject* const* a, Py_ssize_t n) {
   LISAQ_NONE_UNLESS(n == 2 && plain(a[0], &g) && plain(a[1], &u) && g->sizes() == u->sizes() &&
                     g->scalar_type() == at::kBFloat16 && u->scalar_type() == at::kBFloat16 &&
                     g->device() == u->device() && g->numel() > 0 && !modes_active());
-  Tensor act = at::empty(g->sizes(), g->options());
-  LISAQ_NONE_UNLESS(lisaq_swiglu(stream_of(*g), g->data_ptr(), u->data_ptr(), act.data_ptr(), g->numel()) == LISAQ_OK);
+  Tensor act;
+  int rc;
+  {
+    NoGil nogil;
+    act = at::empty(g->sizes(), g->options());
+    rc = lisaq_swiglu(stream_of(*g), g->data_ptr(), u->data_ptr(), act.data_ptr(), g->numel());
+  }
+  LISAQ_NONE_UNLESS(rc == LISAQ_OK);
   return THPVariable_Wrap(std::move(act));
   END_HANDLE_TH_ERRORS
 }
@@ -214,12 +244,20 @@ PyObject* moe(PyObject*, PyObject* const* a, Py_ssize_t n) {
                     u.w->size(0) == E && d.w->size(0) == E && H % gs == 0 && I % gs == 0 && g.shape(I, H, gs, bits) &&
                     u.shape(I, H, gs, bits) && d.shape(H, I, gs, bits));
   LISAQ_NONE_UNLESS((size_t)ws->numel() >= lisaq_moe_workspace(T, H, I, (int)E, (int)k, (int)gs, (int)bits));
-  Tensor out = at::empty(x->sizes(), x->options());
-  const int rc = lisaq_moe_forward(
-      stream_of(*x), x->data_ptr(), static_cast<const float*>(lg->data_ptr()), g.codes_ptr(), g.s->data_ptr(),
-      g.b->data_ptr(), u.codes_ptr(), u.s->data_ptr(), u.b->data_ptr(), d.codes_ptr(), d.s->data_ptr(),
-      d.b->data_ptr(), out.data_ptr(), T, H, I, (int)E, (int)k, (int)gs, (int)bits, nullptr, nullptr, ws->data_ptr(),
-      (size_t)ws->numel());
+  Tensor out;
+  int rc;
+  {
+    NoGil nogil;
+    out = at::empty(x->sizes(), x->options());
+    // the launches of one call stay together on a stream: the next call's use the same workspace
+    static std::mutex mu;
+    std::lock_guard<std::mutex> lock(mu);
+    rc = lisaq_moe_forward(
+        stream_of(*x), x->data_ptr(), static_cast<const float*>(lg->data_ptr()), g.codes_ptr(), g.s->data_ptr(),
+        g.b->data_ptr(), u.codes_ptr(), u.s->data_ptr(), u.b->data_ptr(), d.codes_ptr(), d.s->data_ptr(),
+        d.b->data_ptr(), out.data_ptr(), T, H, I, (int)E, (int)k, (int)gs, (int)bits, nullptr, nullptr, ws->data_ptr(),
+        (size_t)ws->numel());
+  }
   LISAQ_NONE_UNLESS(rc == LISAQ_OK);
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
@@ -238,9 +276,15 @@ PyObject* dequantize(PyObject*, PyObject* const* a, Py_ssize_t n) {
   LISAQ_NONE_UNLESS(K % gs == 0 && s->numel() == rows * (K / gs) && b->numel() == s->numel());
   c10::SmallVector<int64_t, 5> sizes(w->sizes().begin(), w->sizes().end());
   sizes.back() = K;
-  Tensor out = at::empty(sizes, s->options());
-  LISAQ_NONE_UNLESS(lisaq_dequantize(stream_of(*w), static_cast<const uint32_t*>(w->data_ptr()), s->data_ptr(),
-                                     b->data_ptr(), out.data_ptr(), rows, K, (int)gs, (int)bits) == LISAQ_OK);
+  Tensor out;
+  int rc;
+  {
+    NoGil nogil;
+    out = at::empty(sizes, s->options());
+    rc = lisaq_dequantize(stream_of(*w), static_cast<const uint32_t*>(w->data_ptr()), s->data_ptr(), b->data_ptr(),
+                          out.data_ptr(), rows, K, (int)gs, (int)bits);
+  }
+  LISAQ_NONE_UNLESS(rc == LISAQ_OK);
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
 }
@@ -256,13 +300,19 @@ PyObject* quantize(PyObject*, PyObject* const* a, Py_ssize_t n) {
   LISAQ_NONE_UNLESS(K % gs == 0 && gs % (32 / bits) == 0);
   c10::SmallVector<int64_t, 5> sizes(w->sizes().begin(), w->sizes().end());
   sizes.back() = K * bits / 32;
-  Tensor wq = at::empty(sizes, w->options().dtype(at::kInt));
-  sizes.back() = K / gs;
-  Tensor s = at::empty(sizes, w->options()), b = at::empty(sizes, w->options());
-  LISAQ_NONE_UNLESS(lisaq_quantize(stream_of(*w), w->data_ptr(),
-                                   w->scalar_type() == at::kFloat ? LISAQ_DTYPE_F32 : LISAQ_DTYPE_BF16,
-                                   static_cast<uint32_t*>(wq.data_ptr()), s.data_ptr(), b.data_ptr(), rows, K,
-                                   (int)gs, (int)bits) == LISAQ_OK);
+  Tensor wq, s, b;
+  int rc;
+  {
+    NoGil nogil;
+    wq = at::empty(sizes, w->options().dtype(at::kInt));
+    sizes.back() = K / gs;
+    s = at::empty(sizes, w->options());
+    b = at::empty(sizes, w->options());
+    rc = lisaq_quantize(stream_of(*w), w->data_ptr(),
+                        w->scalar_type() == at::kFloat ? LISAQ_DTYPE_F32 : LISAQ_DTYPE_BF16,
+                        static_cast<uint32_t*>(wq.data_ptr()), s.data_ptr(), b.data_ptr(), rows, K, (int)gs, (int)bits);
+  }
+  LISAQ_NONE_UNLESS(rc == LISAQ_OK);
   PyObject* out = PyTuple_New(3);
   if (!out) return nullptr;
   PyTuple_SET_ITEM(out, 0, THPVariable_Wrap(std::move(wq)));

@@ -608,3 +608,47 @@ def test_scratch_of_a_capture_begun_outside_torch(dev, dtype, bits, strided):
         assert all(bool((o == 7).all()) for o in others)
         assert torch.equal(ops.quantized_matmul(x, w, s, b, True, gs, bits), ref)
     assert hip.hipGraphExecDestroy(exe) == 0 and hip.hipGraphDestroy(graph) == 0
+
+
+def test_native_calls_leave_other_threads_running(dev):
+    """A call that waits for room in a full queue does not stop the process's other Python threads."""
+    import threading
+    import time
+
+    import torch
+
+    g, u = (torch.randn(8, 64, device=dev).to(torch.bfloat16) for _ in range(2))
+    ref = ops.swiglu(g, u)
+    cycles, busy = 100_000, 0.0
+    while busy < 0.7:  # (a spin of about a second, whatever its clock)
+        cycles = int(cycles * (min(10.0, 0.9 / busy) if busy > 1e-4 else 10.0))
+        torch.cuda.synchronize()
+        t0 = time.perf_counter()
+        torch.cuda._sleep(cycles)
+        torch.cuda.synchronize()
+        busy = time.perf_counter() - t0
+    gap, stop = [0.0], threading.Event()
+
+    def watch():
+        last = time.perf_counter()
+        while not stop.is_set():
+            time.sleep(0.0005)
+            now = time.perf_counter()
+            gap[0], last = max(gap[0], now - last), now
+
+    th = threading.Thread(target=watch)
+    th.start()
+    done = torch.cuda.Event()
+    torch.cuda._sleep(cycles)
+    done.record()
+    slowest, calls, t0 = 0.0, 0, time.perf_counter()
+    while not done.query() and time.perf_counter() - t0 < 5 * busy:
+        t = time.perf_counter()
+        y = ops.swiglu(g, u)
+        slowest, calls = max(slowest, time.perf_counter() - t), calls + 1
+    stop.set()
+    th.join()
+    torch.cuda.synchronize()
+    print(f"busy {busy:.2f} s, {calls} calls, slowest {slowest:.3f} s, longest gap of the other thread {gap[0]:.3f} s")
+    assert torch.equal(y, ref)
+    assert gap[0] < 0.25 * busy
