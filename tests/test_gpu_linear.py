@@ -325,7 +325,7 @@ def test_quantize_bit_exact_f32(dev, oracle, bits):
 @pytest.mark.parametrize("bits", [2, 4, 8])
 def test_quantize_edges_bit_exact(dev, oracle, dtype, bits, gs):
     """Groups that decide a code on a half step, constant, tiny (the scale's floor), huge and one-sided groups, over
-    a count of 8-value chunks that ends inside a workgroup: codes, scales and biases equal the oracle's.  The same
+    a count of 16-value chunks that ends inside a workgroup: codes, scales and biases equal the oracle's.  The same
     values with NaN and infinities among them, from an address that the wide loads cannot take, equal the aligned
     call's bits."""
     import torch
@@ -652,3 +652,94 @@ def test_native_calls_leave_other_threads_running(dev):
     print(f"busy {busy:.2f} s, {calls} calls, slowest {slowest:.3f} s, longest gap of the other thread {gap[0]:.3f} s")
     assert torch.equal(y, ref)
     assert gap[0] < 0.25 * busy
+
+
+def _native_ops(dev):
+    """name -> (native call, Python op, arguments, positions of the tensors among them)"""
+    import torch
+
+    from lisa_amd import _lib
+
+    n = _lib.native()
+    g = torch.Generator(device=dev)
+    g.manual_seed(7)
+    E, k, H, I, gs, bits = 8, 2, 256, 128, 64, 4
+
+    def packed(*lead, K):
+        w = torch.randint(-(2**31), 2**31, (*lead, K * bits // 32), dtype=torch.int32, device=dev, generator=g)
+        s, b = ((torch.randn(*lead, K // gs, device=dev, generator=g) * 0.02).to(torch.bfloat16) for _ in range(2))
+        return w, s, b
+
+    bf = lambda *sh: torch.randn(*sh, device=dev, generator=g).to(torch.bfloat16)
+    x, q = bf(3, H), packed(40, K=H)
+    gate, up, down = packed(E, I, K=H), packed(E, I, K=H), packed(E, H, K=I)
+    xt, lg = bf(5, H), torch.randn(5, E, device=dev, generator=g)
+    ops.moe_forward(xt, lg, gate, up, down, k, gs, bits)  # (makes the workspace)
+    ws = ops.workspace(dev, 0, "moe_forward")
+    moe = lambda *a: ops.moe_forward(a[0], a[1], a[2:5], a[5:8], a[8:11], *a[11:14])
+    return {
+        "linear": (n.linear, lambda *a: ops.quantized_matmul(*a[:4], True, *a[4:6]), (x, *q, gs, bits, 0), range(4)),
+        "addnorm": (n.addnorm, ops.qmv_addnorm, (bf(1, 4608), bf(1, 4608), bf(4608), *packed(40, K=4608), 1e-6, gs, bits),
+                    range(6)),
+        "swiglu": (n.swiglu, ops.swiglu, (bf(3, 40), bf(3, 40)), range(2)),
+        "dequantize": (n.dequantize, ops.dequantize, (*q, gs, bits), range(3)),
+        "quantize": (n.quantize, ops.quantize, (bf(6, H), gs, bits), range(1)),
+        "moe": (n.moe, moe, (xt, lg, *gate, *up, *down, k, gs, bits, ws), range(11)),
+    }
+
+
+_NATIVE = ["linear", "addnorm", "swiglu", "dequantize", "quantize", "moe"]
+
+
+def _same(a, b):
+    import torch
+
+    a, b = (t if isinstance(t, tuple) else (t,) for t in (a, b))
+    return len(a) == len(b) and all(p.dtype == q.dtype and p.shape == q.shape and
+                                    torch.equal(p.contiguous().view(torch.uint8), q.contiguous().view(torch.uint8))
+                                    for p, q in zip(a, b))
+
+
+@pytest.mark.parametrize("name", _NATIVE)
+def test_native_call_accepts_and_declines(dev, name):
+    """Each native call gives what its op's Python path gives (forced by a strided view of one argument at a time), and
+    declines views, other dtypes, host tensors, missing arguments, tensor subclasses, vmap, dispatch and function
+    modes, leaving those to the Python path."""
+    import torch
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    native, op, args, tensors = _native_ops(dev)[name]
+    ref = native(*args)
+    assert ref is not None and _same(ref, op(*args))
+    put = lambda i, t: (*args[:i], t, *args[i + 1:])
+
+    class Sub(torch.Tensor):
+        pass
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, a=(), kw=None):
+            return func(*a, **(kw or {}))
+
+    class Function(TorchFunctionMode):
+        def __torch_function__(self, func, types, a=(), kw=None):
+            return func(*a, **(kw or {}))
+
+    for i in tensors:
+        t = args[i]
+        strided = torch.stack([t, t], -1)[..., 0]
+        assert native(*put(i, torch.nn.Parameter(t, requires_grad=False))) is not None
+        if t.dim() > 1 or t.numel() > 1:
+            assert not strided.is_contiguous() and native(*put(i, strided)) is None
+            assert _same(ref, op(*put(i, strided)))
+        for other in (None, t.cpu(), t.double(), t.as_subclass(Sub), t.to_sparse() if t.dim() == 2 else None):
+            assert native(*put(i, other)) is None
+        seen = []
+        torch.func.vmap(lambda v: (seen.append(native(*put(i, v))), v)[1])(torch.stack([t, t]))
+        assert seen == [None]
+    assert native(*args[:-1]) is None and native(*args, 0) is None
+    for mode in (Dispatch(), Function()):
+        with mode:
+            declined = native(*args)
+        assert declined is None
+    assert _same(ref, native(*args))

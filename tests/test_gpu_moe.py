@@ -548,14 +548,16 @@ def test_gather_short_last_tiles(dev, oracle, force_path, runs):
     assert_close_bf16(y, ref)
 
 
-@pytest.mark.parametrize("T,bits", [(479, 4), (480, 4), (480, 2), (700, 4)])
-def test_moe_forward_tile_height_rule(dev, T, bits):
-    """Runs averaging just below and from 120 rows on (128- and 288-row tiles; 175 rows: a run's second tile too):
-    moe_forward bitwise equal to the composition over 128-row gather tiles."""
+@pytest.mark.parametrize("T,bits,I", [(479, 4, 320), (480, 4, 320), (480, 2, 320), (700, 4, 320), (479, 4, 384),
+                                      (480, 4, 384), (480, 2, 384), (700, 4, 384)])
+def test_moe_forward_tile_height_rule(dev, oracle, T, bits, I):
+    """Runs averaging just below and from 120 rows on (128- and 288-row tiles; 175 rows: a run's second tile too), an
+    odd and an even number of groups in the down projection: moe_forward bitwise equal to the composition over
+    128-row gather tiles, whose gate, up and down of the longest and the shortest run agree with the oracle."""
     import torch
 
     rng = np.random.default_rng(T + bits)
-    E, k, H, I = 16, 4, 256, 320
+    E, k, H = 16, 4, 256
     G, U, D = (_expert_stack(rng, E, n, m, bits) for n, m in ((I, H), (I, H), (H, I)))
     x = to_dev_bf16(np_x(rng, T, H), dev)
     lg = to_dev(rng.standard_normal((T, E)).astype(np.float32), dev)
@@ -567,9 +569,16 @@ def test_moe_forward_tile_height_rule(dev, T, bits):
     assert offs.diff().min().item() >= ops.qmv_batch_limit(H, I)  # (every run with the matmul arithmetic)
     xs = ops.gather_rows(x, rows)
     g, u = (ops.gather_qmm(xs, *dv[i], rhs_indices=srt, bits=bits) for i in (0, 1))
-    d = ops.gather_qmm(ops.swiglu(g, u), *dv[2], rhs_indices=srt, bits=bits)
+    act = ops.swiglu(g, u)
+    d = ops.gather_qmm(act, *dv[2], rhs_indices=srt, bits=bits)
     ref = ops.moe_combine(d, rw.reshape(-1), inv, T, k)
     assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
+    o, xh, ah = offs.cpu().numpy(), from_dev_bf16(xs), from_dev_bf16(act)
+    for e in (int(np.diff(o).argmax()), int(np.diff(o).argmin())):
+        r = slice(o[e], o[e + 1])
+        for got, src, st, what in ((g, xh, G, "gate"), (u, xh, U, "up"), (d, ah, D, "down")):
+            assert_close_bf16(from_dev_bf16(got)[r], oracle.qmm(src[r], st[0][e], st[1][e], st[2][e], 64, bits),
+                              what=f"{what} of expert {e}")
 
 
 @pytest.mark.parametrize("runs,N,K,gs,bits", [((300, 65, 33, 129, 1, 513, 70), 200, 320, 64, 4),

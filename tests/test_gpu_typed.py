@@ -99,14 +99,15 @@ def test_quantized_matmul_typed_long_k(dev, oracle, dtype, M):
     torch.cuda.synchronize()
 
 
+@pytest.mark.parametrize("K", [256, 320])
 @pytest.mark.parametrize("dtype,bits", [("f16", 4), ("bf16", 8), ("f16", 2)])
-def test_quantized_matmul_typed_wide_tiles(dev, oracle, dtype, bits):
-    """M, N ragged and large enough for the matrix-core matmul's 128 x 128 tiles (at least 512 of
-    them: 16 x 33 here), against the oracle's matmul semantics."""
+def test_quantized_matmul_typed_wide_tiles(dev, oracle, dtype, bits, K):
+    """M, N ragged and large: rows of an odd number of groups (K = 320) take the matrix-core tiles of 128 x 128 (at
+    least 512 of them: 16 x 33 here), the others the bf16 matmul's kernel; against the oracle's matmul semantics."""
     import torch
 
     rng = np.random.default_rng(2000 + bits)
-    M, N, K, gs = 2000, 4200, 256, 64
+    M, N, gs = 2000, 4200, 64
     w, s, b = np_linear(rng, N, K, bits, gs, s_std=0.02 if bits < 8 else 0.002)
     sf = oracle._round_to(bf16_bits_to_f32(s), dtype)
     bf = oracle._round_to(bf16_bits_to_f32(b), dtype)
@@ -124,7 +125,9 @@ def test_quantized_matmul_typed_wide_tiles(dev, oracle, dtype, bits):
     (33, 777, 64, 32),       # one K-step, odd N (single stores)
     (130, 300, 1024, 128),   # two row tiles, N a multiple of 4 only; split over K
     (257, 1000, 4608, 64),   # rows past 256, split over K
+    (70, 777, 64, 32),       # one K-step past the few-rows kernel's 64 rows
     (700, 4100, 512, 64),    # several column tiles, the last partial
+    (700, 12288, 128, 64),   # 4 x 48 tiles of 192 rows
     (1300, 12288, 1152, 64), # more than one round of tiles: 256-row tiles with the last round split (2 and 4 bits)
 ])
 def test_typed_matmul_matrix_core_tiles(dev, oracle, dtype, bits, M, N, K, gs):
@@ -159,6 +162,9 @@ def test_typed_matmul_matrix_core_tiles(dev, oracle, dtype, bits, M, N, K, gs):
     (40, 5120, 2560, 128),   # 20 scale groups of 128 a row
     (13, 4100, 5120, 64),    # the fewest rows, several column tiles
     (17, 33000, 512, 64),    # more column tiles than half the compute units: no split
+    (13, 4100, 5120, 32),    # at most 32 rows, groups of 32: every chunk starts a scale block, K parts
+    (25, 100, 2176, 32),     # the same with a chunk that ends partway
+    (32, 300, 2304, 128),    # at most 32 rows, groups of 128 (18 a row)
 ])
 def test_few_rows_matmul(dev, oracle, dtype, bits, M, N, K, gs):
     """The matmul of at most 64 rows at the edges of its chunks, column groups, scale blocks and K parts, against
@@ -259,3 +265,29 @@ def test_bf16_8bit_matmul_scale_range(dev, oracle, M, N, K, gs):
     wt = np.abs(np.repeat(sf.astype(np.float64), gs, 1) * q + np.repeat(bf.astype(np.float64), gs, 1))
     bound = 2.0**-8 * np.abs(ref) + K * 2.0**-24 * (np.abs(xf).astype(np.float64) @ wt.T)
     assert np.isfinite(y).all() and (np.abs(y - ref) <= bound).all()
+
+
+@pytest.mark.parametrize("dtype,bits", [("f32", 2), ("f32", 4), ("f32", 8), ("f16", 2), ("f16", 4), ("f16", 8), ("bf16", 8)])
+@pytest.mark.parametrize("M,N,K,gs", [(40, 70, 96, 32), (130, 200, 384, 64), (65, 1, 128, 128)])
+def test_typed_matmul_unaligned_x(dev, oracle, dtype, bits, M, N, K, gs):
+    """The typed matmul with x off 16 bytes (64 x 64 FMA tiles; row, column and K tails), and with the other tensors
+    off the alignment of the faster kernels, against the oracle."""
+    import torch
+
+    rng = np.random.default_rng(M + N + K + bits)
+    w, s, b = np_linear(rng, N, K, bits, gs, s_std=0.02 if bits < 8 else 0.002)
+    sf = oracle._round_to(bf16_bits_to_f32(s), dtype)
+    bf = oracle._round_to(bf16_bits_to_f32(b), dtype)
+    xf = oracle._round_to(rng.standard_normal((M, K)).astype(np.float32), dtype)
+    assert M >= ops.qmv_batch_limit(K, N)
+    ref = oracle.qmm_typed(xf, w, sf, bf, gs, bits, dtype)
+
+    def off(t):  # the same values one element past a 16-byte boundary
+        o = torch.empty(t.numel() + 1, dtype=t.dtype, device=dev)[1:].view(t.shape)
+        return o.copy_(t)
+
+    x, wd, sd, bd = _tensor(xf, dtype, dev), to_dev_u32(w, dev), _tensor(sf, dtype, dev), _tensor(bf, dtype, dev)
+    run = lambda *a: ops.quantized_matmul(*a, True, gs, bits).float().cpu().numpy()
+    _close(run(off(x), wd, sd, bd), ref, dtype, "unaligned x")
+    _close(run(x, off(wd), sd, bd), ref, dtype, "unaligned w")
+    _close(run(x, wd, off(sd), off(bd)), ref, dtype, "unaligned scales")
