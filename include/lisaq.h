@@ -95,8 +95,8 @@ LISAQ_API int lisaq_set_path_override(const char* name, int value);
  * (NULL/0 when that is 0).  The matvec paths use none; the matmul path uses
  * it for f32 split-K partials when its output grid is too small to fill the
  * GPU (e.g. N = 5120 at M = 128) and runs unsplit, slower, when the
- * workspace is missing or smaller.  Calls that share a workspace must be
- * ordered on one stream. */
+ * workspace is missing or smaller.  The matmul path takes scales below 2^104
+ * in magnitude.  Calls that share a workspace must be ordered on one stream. */
 LISAQ_API int lisaq_quantized_matmul(void* stream, const void* x, const uint32_t* w, const void* scales,
                            const void* biases, void* y, int64_t M, int64_t N, int64_t K,
                            int transpose, int group_size, int bits, void* workspace,
@@ -111,12 +111,13 @@ LISAQ_API int lisaq_quantized_matmul(void* stream, const void* x, const uint32_t
  * QM:767-830, 996-1088), larger M the matmul arithmetic (weights rounded to T
  * from an f32 fma, f32 accumulation, QM:585-703, 1208-1326); y rounded to T
  * once.  The matvec: x staged in LDS, one to four output rows per wave (x or w
- * off 16 bytes: one wave per output row).  The matmul: the bf16 2/4-bit matmul's kernel for bf16 and f16 where K is a
- * multiple of 64 and of two groups and the tensors are aligned for it (x and w
- * 16 bytes, the others 4), which splits K in a workspace of
- * lisaq_quantized_matmul_workspace bytes (256-byte aligned; without it the
- * call runs unsplit); else matrix-core tiles of 64 x 64 or 128 x 128 (x
- * 16-byte aligned) and, for f32, 64 x 64 f32-FMA tiles, without a workspace. */
+ * off 16 bytes: one wave per output row).  The matmul: the bf16 2/4-bit
+ * matmul's kernel for bf16 and f16 where K is a multiple of 64 and of two
+ * groups and the tensors are aligned for it (x and w 16 bytes, the others 4),
+ * which splits K in a workspace of lisaq_quantized_matmul_workspace bytes
+ * (256-byte aligned; without it the call runs unsplit).  Else, without a
+ * workspace: matrix-core tiles of 64 x 64 or 128 x 128, for f32 of 64 x 64 or
+ * 32 x 32, and 64 x 64 f32-FMA tiles for an x off 16 bytes. */
 LISAQ_API int lisaq_quantized_matmul_typed(void* stream, const void* x, const uint32_t* w, const void* scales,
                                            const void* biases, void* y, int64_t M, int64_t N, int64_t K,
                                            int transpose, int group_size, int bits, int dtype, void* workspace,

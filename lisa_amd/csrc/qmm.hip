@@ -1,6 +1,7 @@
 // Prefill matmul (qmm): host side -- tile configuration, kernel choice and
 // launch, and the reduction of split-K partials.  The kernel (its design and
-// arithmetic contract) is in qmm_kernel.h; qmm_k{4,2}_{p,s}.hip instantiate it.
+// arithmetic contract) is in qmm_kernel.h, its form for at most 64 rows in
+// qmm_rows.h; qmm_k{4,2}_{p,s}.hip, qmm_t*.hip and qmm_rows_*.hip instantiate them.
 #include "qmm_rows.h"
 #include <cstdlib>
 

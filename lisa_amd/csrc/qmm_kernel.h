@@ -8,19 +8,18 @@
 // accumulator (steel BlockMMA, gemm.metal:905-919), one bf16 rounding.
 //
 // MI355X design:
-//  * Workgroup = 4 waves side by side along N.  The x tile (BM rows x 64 K)
-//    is staged through LDS (double-buffered) and shared by the 4 waves; each
-//    wave streams and dequantizes only its own W rows, straight from global
-//    memory into the bf16 B operands of v_mfma_f32_32x32x16_bf16 (no LDS round
-//    trip for W, no duplicated dequant work).
-//  * Per lane and K-step of 64: one 16-byte load of packed codes (4-bit), 8
-//    codes per u32 split with one mask into bytes, v_cvt_f32_ubyte*, one FMA
-//    with the group's scale/bias, v_cvt_pk_bf16_f32.
-//  * The next K-step's x tile and W words are fetched while the current one
-//    runs on the matrix cores.
-// Compute types: bf16 and f16 (CT), 2-, 4- and 8-bit codes.  A weight is an
-// fma and half a packed conversion (Ct::pk) after the unpack: f16 4-bit 1000 x 5120 x 5120 takes 69 us (758 TFLOP/s; on the
-// separate 64 x 64 typed tiles 217 us), bf16 8-bit 73 us.
+//  * Workgroup = 8 waves side by side along N.  The x tile (BM rows x 64 K, a
+//    ring of three) and the packed W of a pair of K-steps (two buffers) reach
+//    LDS by direct copies; the waves share x, and each dequantizes only its own
+//    W rows into the B operands of v_mfma_f32_32x32x16 (no duplicated dequant
+//    work).
+//  * Per lane and K-step of 64: one 16-byte LDS read of packed codes (4-bit), 8
+//    codes per u32 split with one mask into bytes, v_perm to pairs, one FMA per
+//    code with the group's scale/bias, half a packed conversion (Ct::pk).
+//  * The next K-steps' x tile and W words are copied, and the next step's W
+//    dequantized, while the current one runs on the matrix cores.
+// Compute types: bf16 and f16 (CT), 2-, 4- and 8-bit codes: f16 4-bit 1000 x
+// 5120 x 5120 68 us (770 TFLOP/s; on 64 x 64 typed tiles 217 us), bf16 8-bit 66.
 #pragma once
 #include "lisaq_common.h"
 #include "qmm.h"
@@ -171,11 +170,6 @@ constexpr int XG = 1024;  // bytes per 8-row group
 
 __device__ __forceinline__ int x_swz(int row) { return (row & 7) ^ ((row >> 3) & 1); }
 __device__ __forceinline__ int x_lds_off(int row, int chunk) { return row * 128 + ((chunk ^ x_swz(row)) << 4); }
-// Packed W tile (4-bit: 32 bytes = two 16-byte halves per row and K-step):
-// the halves of a row swap when bit 2 ^ bit 3 of the row is set, so the
-// B-operand reads (lanes on 32 consecutive rows, one half) are conflict-free
-// in the same sense.
-__device__ __forceinline__ int w_swz(int row) { return ((row >> 2) ^ (row >> 3)) & 1; }
 // The W tile holds two K-steps per row (4-bit: 64 bytes = four 16-byte
 // chunks, logical chunk = 2 * step + half): physical chunk = logical ^
 // w_swz2(row), which puts any 8 consecutive rows' reads of one logical chunk
@@ -189,16 +183,10 @@ __device__ __forceinline__ int w_chunk_swz(int row) {
   return BITS == 8 ? x_swz(row) : BITS == 4 ? w_swz2(row) : 0;
 }
 
-// 16 / 4 / 2 bytes per lane from global memory straight into LDS (lane l
-// writes lds + size*l; lds must be wave-uniform).
+// 16 bytes per lane from global memory straight into LDS (lane l writes lds +
+// 16 l; lds must be wave-uniform).
 __device__ __forceinline__ void load_lds16(const void* g, void* lds) {
   __builtin_amdgcn_global_load_lds(g, (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
-}
-__device__ __forceinline__ void load_lds4(const void* g, void* lds) {
-  __builtin_amdgcn_global_load_lds(g, (__attribute__((address_space(3))) void*)lds, 4, 0, 0);
-}
-__device__ __forceinline__ void load_lds2(const void* g, void* lds) {
-  __builtin_amdgcn_global_load_lds(g, (__attribute__((address_space(3))) void*)lds, 2, 0, 0);
 }
 
 // The same through a buffer descriptor: byte address = base + voffset +
@@ -211,10 +199,6 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t lds_rsrc(const void* p, uint32
 }
 __device__ __forceinline__ void buf_lds16(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, void* lds) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, voff,
-                                           __builtin_amdgcn_readfirstlane(soff), 0, 0);
-}
-__device__ __forceinline__ void buf_lds4(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, void* lds) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 4, voff,
                                            __builtin_amdgcn_readfirstlane(soff), 0, 0);
 }
 
@@ -242,9 +226,9 @@ __device__ __forceinline__ void block_sync() {
 
 // NB: depth of the x ring (x of step k + NB - 1 in flight while step k runs).
 // W: two buffers of two K-steps each (the pair after next in flight).
-template <int BITS, int GS, int MT, int NT, int WN, int NB = 3, int WM = 1>
+template <int BITS, int GS, int MT, int NT, int WN, int NB = 3>
 struct QmmLds {
-  static constexpr int BM = 32 * MT * WM, BN = WN * 32 * NT;
+  static constexpr int BM = 32 * MT, BN = WN * 32 * NT;
   static constexpr int RB = 32 / (32 / BITS) * 8;  // bytes of one W row per K-step (64 codes): 32 or 16
   static constexpr int X = BM / 8 * XG;            // x tile
   static constexpr int W = BN * RB;                // packed W of one K-step
@@ -274,26 +258,22 @@ struct QmmLds {
 //
 // SKIP (tile-table launches; implied by GU): 32-row blocks past the tile's rows
 // skip their matrix instructions.
-//
-// WM: waves along M (WN x WM waves, each MT x 32 rows by NT x 32 columns).
 template <int BITS, int GS, int MT, int NT, int WN, bool SPLIT, bool GU = false, int NB = 3, bool SKIP = GU,
-          int WM = 1, int CT = kCtBf16>
-__global__ __launch_bounds__(64 * WN * WM) void qmm_kernel(QmmParams p) {
+          int CT = kCtBf16>
+__global__ __launch_bounds__(64 * WN) void qmm_kernel(QmmParams p) {
   using G = MGeo<BITS>;
   using C = Ct<CT>;
-  using L = QmmLds<BITS, GS, MT, NT, WN, NB, WM>;
+  using L = QmmLds<BITS, GS, MT, NT, WN, NB>;
   static_assert(!GU || CT == kCtBf16, "SwiGLU epilogue: bf16 only");
-  static_assert(WM == 1 || (!GU && !SKIP), "waves along M: plain tiles only");
   static_assert(NB == 3, "ring depth");
   constexpr int BM = L::BM;
   constexpr int BN = L::BN;
-  constexpr int NWV = WN * WM;  // waves per workgroup
+  constexpr int NWV = WN;  // waves per workgroup
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform
-  const int wn = WM == 1 ? wave : wave % WN;               // column group
-  const int wrow = WM == 1 ? 0 : (wave / WN) * MT * 32;  // first tile row of the wave's row group
+  const int wn = wave;  // column group
   const int col = lane & 31;
   const int h = lane >> 5;
 
@@ -614,7 +594,7 @@ __global__ __launch_bounds__(64 * WN * WM) void qmm_kernel(QmmParams p) {
     dequant_all(w0, bA);
   }
   auto read_a1 = [&](const unsigned char* xb, int j, int mt) -> u32x4 {
-    return *reinterpret_cast<const u32x4*>(xb + x_lds_off(wrow + mt * 32 + col, 4 * h + j));
+    return *reinterpret_cast<const u32x4*>(xb + x_lds_off(mt * 32 + col, 4 * h + j));
   };
   u32x4 a0[MT], a1[MT];
   WLane wA, wB;  // W of the step after the current one (alternating)
@@ -821,7 +801,7 @@ __global__ __launch_bounds__(64 * WN * WM) void qmm_kernel(QmmParams p) {
   auto store = [&](auto put4, auto put1) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
-      const int m = m0 + wrow + mt * 32 + col;
+      const int m = m0 + mt * 32 + col;
       if (m >= M) continue;
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt)
@@ -839,56 +819,54 @@ __global__ __launch_bounds__(64 * WN * WM) void qmm_kernel(QmmParams p) {
         }
     }
   };
-  if constexpr (WM == 1) {
-    if (whole && (!p.tiles || MT >= 8) && (p.N & 7) == 0) {
-      // (plain launches and 256/288-row gather tiles, which runs mostly fill --
-      // a run's short last tile goes to the 64-row kernel: MoE T = 4096
-      // 500 -> 478 us; a 128-row gather tile is often a few rows, which the
-      // direct stores below serve for less)
-      // whole tile through LDS, RB rows at a time ([RB][BN + 8] bf16, 16 bytes
-      // of padding per row), then 16-byte stores along the output rows (a
-      // row of the tile is BN * 2 contiguous bytes of y), after every copy into
-      // the ring has landed (the copies past the last step re-read it) and
-      // every wave is past its last ring read.
-      constexpr int XSn = BN + 8;
-      constexpr int RB = BM * XSn * 2 <= L::TOTAL ? BM : (BM % 128 == 0 && 128 * XSn * 2 <= L::TOTAL) ? 128 : 96;
-      constexpr int NPASS = BM / RB, MTP = RB / 32;
-      static_assert(RB * XSn * 2 <= L::TOTAL && BM % RB == 0, "output tile exchange fits the ring");
-      constexpr int CH = BN / 8, PASSES = RB * CH / (64 * NWV);
-      static_assert(RB * CH % (64 * NWV) == 0, "output passes");
-      wait_vm<0>();
-      uint16_t* ex = reinterpret_cast<uint16_t*>(smem);
-      static_for<NPASS>([&](auto PI) {
-        constexpr int hp = decltype(PI)::value;
-        wait_lgkm0();
-        block_sync();
-        if (hp * RB < M - m0) {
+  if (whole && (!p.tiles || MT >= 8) && (p.N & 7) == 0) {
+    // (plain launches and 256/288-row gather tiles, which runs mostly fill --
+    // a run's short last tile goes to the 64-row kernel: MoE T = 4096
+    // 500 -> 478 us; a 128-row gather tile is often a few rows, which the
+    // direct stores below serve for less)
+    // whole tile through LDS, RB rows at a time ([RB][BN + 8] bf16, 16 bytes
+    // of padding per row), then 16-byte stores along the output rows (a
+    // row of the tile is BN * 2 contiguous bytes of y), after every copy into
+    // the ring has landed (the copies past the last step re-read it) and
+    // every wave is past its last ring read.
+    constexpr int XSn = BN + 8;
+    constexpr int RB = BM * XSn * 2 <= L::TOTAL ? BM : (BM % 128 == 0 && 128 * XSn * 2 <= L::TOTAL) ? 128 : 96;
+    constexpr int NPASS = BM / RB, MTP = RB / 32;
+    static_assert(RB * XSn * 2 <= L::TOTAL && BM % RB == 0, "output tile exchange fits the ring");
+    constexpr int CH = BN / 8, PASSES = RB * CH / (64 * NWV);
+    static_assert(RB * CH % (64 * NWV) == 0, "output passes");
+    wait_vm<0>();
+    uint16_t* ex = reinterpret_cast<uint16_t*>(smem);
+    static_for<NPASS>([&](auto PI) {
+      constexpr int hp = decltype(PI)::value;
+      wait_lgkm0();
+      block_sync();
+      if (hp * RB < M - m0) {
 #pragma unroll
-          for (int mt = hp * MTP; mt < (hp + 1) * MTP; ++mt)
+        for (int mt = hp * MTP; mt < (hp + 1) * MTP; ++mt)
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
+          for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-              for (int g = 0; g < 4; ++g) {
-                const f32x16& a = acc[mt][nt];
-                const int c = (wn * NT + nt) * 32 + 8 * g + 4 * h;
-                *reinterpret_cast<u32x2*>(ex + ((mt - hp * MTP) * 32 + col) * XSn + c) =
-                    u32x2{C::pk(a[4 * g], a[4 * g + 1]), C::pk(a[4 * g + 2], a[4 * g + 3])};
-              }
-        }
-        wait_lgkm0();
-        block_sync();
+            for (int g = 0; g < 4; ++g) {
+              const f32x16& a = acc[mt][nt];
+              const int c = (wn * NT + nt) * 32 + 8 * g + 4 * h;
+              *reinterpret_cast<u32x2*>(ex + ((mt - hp * MTP) * 32 + col) * XSn + c) =
+                  u32x2{C::pk(a[4 * g], a[4 * g + 1]), C::pk(a[4 * g + 2], a[4 * g + 3])};
+            }
+      }
+      wait_lgkm0();
+      block_sync();
 #pragma unroll
-        for (int ps = 0; ps < PASSES; ++ps) {
-          const int c = ps * 64 * NWV + (int)threadIdx.x;
-          const int r = c / CH, cc = (c % CH) * 8;
-          const int m = m0 + hp * RB + r;
-          if (m >= M || nt0 + cc >= p.N) continue;
-          *reinterpret_cast<u32x4*>(y + (int64_t)m * p.N + nt0 + cc) =
-              *reinterpret_cast<const u32x4*>(ex + r * XSn + cc);
-        }
-      });
-      return;
-    }
+      for (int ps = 0; ps < PASSES; ++ps) {
+        const int c = ps * 64 * NWV + (int)threadIdx.x;
+        const int r = c / CH, cc = (c % CH) * 8;
+        const int m = m0 + hp * RB + r;
+        if (m >= M || nt0 + cc >= p.N) continue;
+        *reinterpret_cast<u32x4*>(y + (int64_t)m * p.N + nt0 + cc) =
+            *reinterpret_cast<const u32x4*>(ex + r * XSn + cc);
+      }
+    });
+    return;
   }
   if (whole) {
     store([&](int m, int n, float v0, float v1, float v2, float v3) {
@@ -927,9 +905,9 @@ qmm_fn qmm_get_impl(int gs, int MT, int* lds) {
   auto one = [&](auto mt) -> qmm_fn {
     constexpr int M_ = decltype(mt)::value;
     *lds = QmmLds<BITS, 64, M_, 1, 8>::TOTAL;  // (group-size independent)
-    if (gs == 32) return qmm_kernel<BITS, 32, M_, 1, 8, SPLIT, false, 3, false, 1, CT>;
-    if (gs == 64) return qmm_kernel<BITS, 64, M_, 1, 8, SPLIT, false, 3, false, 1, CT>;
-    if (gs == 128) return qmm_kernel<BITS, 128, M_, 1, 8, SPLIT, false, 3, false, 1, CT>;
+    if (gs == 32) return qmm_kernel<BITS, 32, M_, 1, 8, SPLIT, false, 3, false, CT>;
+    if (gs == 64) return qmm_kernel<BITS, 64, M_, 1, 8, SPLIT, false, 3, false, CT>;
+    if (gs == 128) return qmm_kernel<BITS, 128, M_, 1, 8, SPLIT, false, 3, false, CT>;
     return nullptr;
   };
   // split launches exist in two layouts only: per-part partials [S][M][N]

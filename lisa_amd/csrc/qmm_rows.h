@@ -15,9 +15,9 @@
 // qmm_kernel.h -> here: 4-bit 17408 x 5120 24 rows 31.2 -> 22.7 us, 64 rows 36.1
 // -> 30.1; 5120 x 17408 16 rows 31.8 -> 21.8; 2560 x 9728 32 rows 17.6 -> 14.6;
 // 8-bit 9728 x 2560 24 rows 14.5 -> 12.0.  Left: ~6 us of launch, first copies
-// and sums, 4 us of the reduction launch, and the dequantization (11 us of VALU
+// and sums, 4 us of the reduction launch, and the dequantization (7 us of VALU
 // cycles at 17408 x 5120 on the 204 of 256 units that three parts of 68 tiles
-// use; 8-bit codes take the same time, 3.9 TB/s).  Eight waves with the next
+// use).  Eight waves with the next
 // chunk's LDS reads issued a chunk ahead: the same times.
 //
 // Workgroup: 256 columns by all 32 * MT rows of one K part.  Wave w takes the

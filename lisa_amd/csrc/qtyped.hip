@@ -13,10 +13,10 @@
 //    f32 fma, then y = x . w^T with f32 accumulation, rounded to T once.
 //
 // Kernels: for the matvec x in LDS and several output rows per wave (a wave per
-// output row for unaligned x or W); for the matmul of the
-// problems that the bf16 2/4-bit matmul's kernel does not take in their type
-// (f32, rows of an odd number of groups, addresses off its alignment) the
-// matrix cores with bf16/f16 (below), else 64 x 64 register-tiled f32 FMA.
+// output row for unaligned x or W).  For the matmul, of the problems that the
+// bf16 2/4-bit matmul's kernel does not take in their type (f32, rows of an odd
+// number of groups, addresses off its alignment): the matrix cores in bf16, f16
+// or f32, and 64 x 64 register-tiled f32 FMA for an x off 16 bytes.
 #include "lisaq_common.h"
 #include "qmv.h"
 #include "qmv_dev.h"
@@ -587,8 +587,10 @@ TypedRows pick_rows_dt(int bits, int gs, int MR, int RW) {
     if (gs == 128) return pick_rows_mr<DT, B, 128>(MR, RW);
     return {nullptr, 0};
   };
-  if (bits == 2) return by_gs(std::integral_constant<int, 2>{});
-  if (bits == 4) return by_gs(std::integral_constant<int, 4>{});
+  if constexpr (DT != LISAQ_DTYPE_BF16) {  // (bf16 with 2 and 4 bits: qmv*.hip, qmm*.h)
+    if (bits == 2) return by_gs(std::integral_constant<int, 2>{});
+    if (bits == 4) return by_gs(std::integral_constant<int, 4>{});
+  }
   if (bits == 8) return by_gs(std::integral_constant<int, 8>{});
   return {nullptr, 0};
 }
@@ -609,7 +611,7 @@ typed_fn pick_f32(int bits, int gs) {
 }
 
 TypedRows pick_rows(int dtype, int bits, int gs, int MR, int RW) {
-  if (dtype == LISAQ_DTYPE_BF16 && bits == 8) return pick_rows_dt<0>(bits, gs, MR, RW);
+  if (dtype == LISAQ_DTYPE_BF16) return pick_rows_dt<0>(bits, gs, MR, RW);
   if (dtype == LISAQ_DTYPE_F32) return pick_rows_dt<1>(bits, gs, MR, RW);
   if (dtype == LISAQ_DTYPE_F16) return pick_rows_dt<2>(bits, gs, MR, RW);
   return {nullptr, 0};
@@ -625,8 +627,10 @@ typed_fn pick_mfma_gs(int gs) {
 
 template <int DT, int TB>
 typed_fn pick_mfma(int bits, int gs) {
-  if (bits == 2) return pick_mfma_gs<DT, 2, TB>(gs);
-  if (bits == 4) return pick_mfma_gs<DT, 4, TB>(gs);
+  if constexpr (DT != LISAQ_DTYPE_BF16) {
+    if (bits == 2) return pick_mfma_gs<DT, 2, TB>(gs);
+    if (bits == 4) return pick_mfma_gs<DT, 4, TB>(gs);
+  }
   if (bits == 8) return pick_mfma_gs<DT, 8, TB>(gs);
   return nullptr;
 }
@@ -641,8 +645,10 @@ typed_fn pick_gs(int gs) {
 
 template <bool MV, int DT>
 typed_fn pick_bits(int bits, int gs) {
-  if (bits == 2) return pick_gs<MV, DT, 2>(gs);
-  if (bits == 4) return pick_gs<MV, DT, 4>(gs);
+  if constexpr (DT != LISAQ_DTYPE_BF16) {
+    if (bits == 2) return pick_gs<MV, DT, 2>(gs);
+    if (bits == 4) return pick_gs<MV, DT, 4>(gs);
+  }
   if (bits == 8) return pick_gs<MV, DT, 8>(gs);
   return nullptr;
 }
@@ -693,7 +699,8 @@ int launch_typed_mm(hipStream_t st, bool matvec, const void* x, const uint32_t* 
   // 11.6 us, 15.3 four at a time; 12 rows 26 / 31), one where two pass that
   // (bf16 8-bit 5120 x 17408 4 rows 42 us, 62 / 48 at four / two).  Rows of W per
   // wave (RW): one row of x two, one below 4096 rows (f32 1000 x 8192 RW 2 6.0 us,
-  // RW 4 7.6); else four, two where that leaves a compute unit without a workgroup.
+  // RW 4 7.6); several rows of x one at a time four; else four, two where that
+  // leaves a compute unit without a workgroup.
   const int P = bits == 8 ? 16 : 32;
   const int64_t per_row = K * (dtype == LISAQ_DTYPE_F32 ? 4 : 2) + K / P * 4;
   if (matvec && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0 &&
