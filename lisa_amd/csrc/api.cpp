@@ -594,6 +594,21 @@ int lisaq_quantized_matmul(void* stream, const void* x, const uint32_t* w, const
   return run_qmm((hipStream_t)stream, x, w, s, b, y, M, N, K, gs, bits, ws, ws_bytes);
 }
 
+// Small 16-bit typed matmuls that the 64 x 64 tiles of qtyped.hip do faster than
+// the bf16 matmul's kernel: a tile is one pass over K without a ring to fill or
+// partials to sum, so its time is ~1.5 us + 13.7 ns per value of K, for up to one
+// tile per compute unit and so on by rounds.  Measured (tiles here / there, us): f16
+// 4-bit 64 x 1024 x 128 3.9 / 5.9, 512 x 4096 x 256 (512 tiles) 7.0 / 7.8, 256 x
+// 16384 x 256 (1024 tiles) 10.7 / 9.5; bf16 8-bit 130 x 300 x 512 8.5 / 11.4, 1024 x
+// 1024 x 1024 14.6 / 17.6, 512 x 4096 x 1024 18.2 / 20.4; at 32 rows and fewer the
+// few-rows kernel is level from K = 384 on, at 64 from 768.
+static bool typed_tiles_faster(int64_t M, int64_t N, int64_t K) {
+  const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64);
+  if (M <= 64 && K > (M <= 32 ? 256 : 512)) return false;
+  if (K > 768) return K <= 1024 && M >= 128 && M <= 1024 && tiles >= 48 && tiles <= 512;
+  return K * tiles <= 768 * 256;
+}
+
 int lisaq_quantized_matmul_typed(void* stream, const void* x, const uint32_t* w, const void* s, const void* b,
                                  void* y, int64_t M, int64_t N, int64_t K, int transpose, int gs, int bits, int dtype,
                                  void* ws, size_t ws_bytes) {
@@ -625,7 +640,7 @@ int lisaq_quantized_matmul_typed(void* stream, const void* x, const uint32_t* w,
   // scale/bias copies are 16 bytes of a row from a dword on: other addresses,
   // sizes past its 32-bit offsets and rows of an odd number of groups (which the
   // kernel takes, not measured here) stay on the kernels of qtyped.hip.
-  if (!matvec && dtype != LISAQ_DTYPE_F32 && K % 64 == 0 && K / gs % 2 == 0 && aligned(x, 16) && aligned(w, 16) &&
+  if (!matvec && dtype != LISAQ_DTYPE_F32 && !typed_tiles_faster(M, N, K) && K % 64 == 0 && K / gs % 2 == 0 && aligned(x, 16) && aligned(w, 16) &&
       aligned(s, 4) && aligned(b, 4) && aligned(y, 4) && M * K < ((int64_t)1 << 31) &&
       N * K * bits / 8 < ((int64_t)1 << 32)) {
     const bool room = ws != nullptr && aligned(ws, 256);
@@ -666,8 +681,9 @@ int lisaq_quantized_matmul_serial_rows(void* stream, const void* x, const uint32
   // the same bits): five to eight rows in one launch of six or eight where that
   // many staged rows of x fit the LDS (7 rows as one launch instead of four, a
   // pair and a single: 9728 x 2560 24.8 -> 21.2 us, 17408 x 5120 49.7 -> 44.8;
-  // 6 rows 19.8 -> 17.3, 39.8 -> 36.1; 5 rows 18.1 -> 17.4, 37.7 -> 37.3), else
-  // fours; the rows left (at most three) go the pair way below.  Measured (4-bit, cold,
+  // 6 rows 19.8 -> 17.3, 39.8 -> 36.1; 5 rows 18.1 -> 17.4, 37.7 -> 37.3; not 5
+  // 2-bit rows from three passes over K on: 17408 x 5120 35.5 -> 37.4, nor 7 rows
+  // from four passes on: 5120 x 6400 32.3 -> 33.3), else fours; the rows left (at most three) go the pair way below.  Measured (4-bit, cold,
   // graph-replayed, these rows vs pairs): 2560 x 9728 4 rows 12.1 vs 17.3 us,
   // 8 rows (two fours) 24.2 vs 34.2; 9728 x 2560 4 rows 13.4 vs 14.7, 8 rows
   // 21.2 vs 29.0; the north-star shape 4 rows 26.8 vs 26.7, 8 rows 51.4 vs
@@ -678,7 +694,8 @@ int lisaq_quantized_matmul_serial_rows(void* stream, const void* x, const uint32
     while (M - r_done >= 4) {
       const int64_t left = M - r_done;
       int64_t mr = 0;
-      if (left >= 5 && qmvs_rows_supported(left, N, K, gs, bits)) mr = left;
+      const bool slower = (left == 5 && bits == 2 && K > 4096) || (left == 7 && K > 6144);
+      if (left >= 5 && !slower && qmvs_rows_supported(left, N, K, gs, bits)) mr = left;
       else if (qmvs_rows_supported(4, N, K, gs, bits)) mr = 4;
       if (!mr) break;
       QmvParams p{};

@@ -96,8 +96,10 @@ QmmConfig qmm_config(int64_t M, int64_t N, int64_t K, int gs, int bits, bool all
   // 35.9 and 42.6 us at 17408 x 5120, those 38.0 and 40.6.  Its scale blocks
   // start on a dword, so rows of an even number of groups; 2 bits in groups of
   // 32 from 33 rows on need more LDS than there is.
-  if (rows_ok && split_forced == 0 && M <= tune_int("LISAQ_QMM_ROWS", 64) && K / gs % 2 == 0 && N * (K / gs) >= 8 &&
-      !(bits == 2 && gs == 32 && M > 32)) {
+  // From 33 rows on K has to be longer than 256: 64 x 8192 x 256 takes 7.2 us on
+  // 128-row tiles, 7.7 there (33 rows 7.2 both).
+  if (rows_ok && split_forced == 0 && M <= tune_int("LISAQ_QMM_ROWS", 64) && (M <= 32 || nk > 4) &&
+      K / gs % 2 == 0 && N * (K / gs) >= 8 && !(bits == 2 && gs == 32 && M > 32)) {
     c.rows = true;
     c.MT = M <= 32 ? 1 : 2;
     c.NT = 1;
@@ -111,7 +113,10 @@ QmmConfig qmm_config(int64_t M, int64_t N, int64_t K, int gs, int bits, bool all
     if (allow_split && c.grid <= 128) {
       int S = 256 / c.grid;
       if (S > 16) S = 16;
-      if (S > nc / 2) S = nc / 2 > 0 ? nc / 2 : 1;
+      // (four chunks of 128 codes stay whole: two parts of two cost more in
+      // their sums, 64 rows of 16384 x 512)
+      if (S > nc / 2) S = nc / 2;
+      if (nc * ks <= 8) S = 1;
       const int per = (nc + S - 1) / S;
       c.S = (nc + per - 1) / per;  // every part non-empty
     }

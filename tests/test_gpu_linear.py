@@ -743,3 +743,16 @@ def test_native_call_accepts_and_declines(dev, name):
             declined = native(*args)
         assert declined is None
     assert _same(ref, native(*args))
+
+
+@pytest.mark.parametrize("bits", [4, 2])
+@pytest.mark.parametrize("M,N,K,gs", [(20, 8, 64, 32), (13, 40, 192, 32), (32, 300, 128, 64), (1, 77, 256, 128),
+                                      (32, 515, 256, 32), (33, 300, 256, 64), (64, 100, 128, 64), (64, 260, 320, 32)])
+def test_few_rows_short_rows(dev, oracle, M, N, K, gs, bits):
+    """The matmul of few rows forced on rows of one chunk and less, and past 32 rows on both sides of the K from which
+    it is chosen."""
+    rng = np.random.default_rng(M + N + K + bits)
+    w, s, b = np_linear(rng, N, K, bits, gs, s_std=0.02 if bits == 4 else 0.05)
+    x = np_x(rng, M, K)
+    got = _run(ops.qmm, dev, x, w, s, b, gs, bits)
+    assert_close_bf16(got, oracle.qmm(x, w, s, b, gs, bits), what=f"M={M} N={N} K={K} bits={bits} gs={gs}")

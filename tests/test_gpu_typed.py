@@ -125,7 +125,7 @@ def test_quantized_matmul_typed_wide_tiles(dev, oracle, dtype, bits, K):
     (33, 777, 64, 32),       # one K-step, odd N (single stores)
     (130, 300, 1024, 128),   # two row tiles, N a multiple of 4 only; split over K
     (257, 1000, 4608, 64),   # rows past 256, split over K
-    (70, 777, 64, 32),       # one K-step past the few-rows kernel's 64 rows
+    (2100, 8200, 64, 32),    # one K-step, too many tiles for the 64 x 64 ones
     (700, 4100, 512, 64),    # several column tiles, the last partial
     (700, 12288, 128, 64),   # 4 x 48 tiles of 192 rows
     (1300, 12288, 1152, 64), # more than one round of tiles: 256-row tiles with the last round split (2 and 4 bits)
@@ -165,6 +165,11 @@ def test_typed_matmul_matrix_core_tiles(dev, oracle, dtype, bits, M, N, K, gs):
     (13, 4100, 5120, 32),    # at most 32 rows, groups of 32: every chunk starts a scale block, K parts
     (25, 100, 2176, 32),     # the same with a chunk that ends partway
     (32, 300, 2304, 128),    # at most 32 rows, groups of 128 (18 a row)
+    (33, 8, 640, 64),        # past 32 rows: five chunks, a part of a column group
+    (64, 40, 704, 32),       # a chunk that ends partway (eleven K-steps), 22 groups a row
+    (40, 300, 512, 64),      # the last K on 64 x 64 tiles (typed)
+    (130, 4100, 768, 64),    # (past 64 rows) 195 tiles of 64 x 64 at their last K but one
+    (128, 3072, 1024, 128),  # 96 of them at their last K
 ])
 def test_few_rows_matmul(dev, oracle, dtype, bits, M, N, K, gs):
     """The matmul of at most 64 rows at the edges of its chunks, column groups, scale blocks and K parts, against
@@ -243,7 +248,7 @@ def test_f32_matmul_matrix_cores(dev, oracle, bits, M, N, K, gs):
     assert np.linalg.norm(y - ref) <= 1e-6 * np.linalg.norm(ref) * max(1.0, np.sqrt(K / 1024))
 
 
-@pytest.mark.parametrize("M,N,K,gs", [(25, 264, 2176, 64), (40, 100, 384, 64), (150, 300, 256, 128), (700, 264, 512, 32)])
+@pytest.mark.parametrize("M,N,K,gs", [(25, 264, 2176, 64), (40, 100, 640, 64), (150, 300, 1280, 128), (700, 264, 1280, 32)])
 def test_bf16_8bit_matmul_scale_range(dev, oracle, M, N, K, gs):
     """bf16 scales over their whole range (2^104 and more among them) with 8-bit codes: every weight is
     bf16(fma(scale, q, bias)), finite wherever that is, for code 0 too."""
