@@ -107,19 +107,20 @@ __global__ __launch_bounds__(256) void qmv_typed_kernel(const void* x, const uin
 
 // Matvec with x in LDS and several rows of W per wave: the kernel for x and W
 // 16-byte aligned.  A lane takes pieces lane, lane + 64, ... of a row -- a piece
-// is one load, 16 codes of 8 bits, 32 of 4 or 2 -- of RW rows at a time, the
-// next pieces' loads in flight while these are computed; each value of x read
-// from LDS and each conversion of a code serve RW rows and MR rows of x.  Codes become f32 by
-// v_cvt_f32_ubyte, and per piece (inside one group)
+// is one load, 16 codes of 8 bits, 32 of 4 or 2 -- of RW rows at a time; each
+// value of x read from LDS and each conversion of a code serve RW rows and MR
+// rows of x.  Codes become f32 by v_cvt_f32_ubyte, and per piece (inside one group)
 //   y += scale * sum(x * q) + bias * sum(x),
 // all in f32, sum(x) of a piece once per workgroup.
+// Two steps of loads are in flight over the wave's whole stream of rows, the
+// first ones across the barriers of the staging of x (LDS only).  They are
+// unconditional: behind a branch the compiler waits for every load in flight
+// before each step (f16 8-bit 1000 x 8192 one row 5.4 -> 7.4 us; four or eight
+// steps in flight, whose loads wait in line before the first: 5.5 / 6.5).
 // What bounds it: one row of x, the stream of W; from two rows on VALU issue
-// (per code ~(4.9 + 2.5 MR) cycles of a SIMD).  Against the
-// kernels it replaced (x from global memory; one row of W per wave with x in
-// LDS; f16 4-bit dot instructions), us: bf16 8-bit 9728 x 2560 1 row 9.9 -> 6.0
-// (4.4 TB/s), 4 rows 16.8 -> 11.6, 12 rows 43 -> 26; f16 8-bit 17408 x 5120 1 row
-// 22.8 -> 18.1, 12 rows 149 -> 71; f16 4-bit the same shape 1 row 17.3 both, 4
-// rows 42 -> 34; f32 4-bit 2560 x 9728 1 row 11.4 -> 9.4, 4 rows 48 -> 16.5.
+// (per code ~(4.9 + 2.5 MR) cycles of a SIMD).  us: bf16 8-bit 9728 x 2560 1 row
+// 5.9 (4.4 TB/s); 2560 x 9728 1 row 8.1, 2 rows 11.3; f16 8-bit 17408 x 5120 1
+// row 19, 12 rows 70; 5120 x 17408 12 rows 90; f32 4-bit 17408 x 5120 1 row 17.
 // x in LDS: planes of 16 bytes, plane q of every piece side by side (a wave's
 // reads of a plane are contiguous), then the sums.
 template <int DT, int BITS>
@@ -148,24 +149,89 @@ __device__ __forceinline__ void for_planes(F&& f, std::integer_sequence<int, Q..
   (f(std::integral_constant<int, Q>{}), ...);
 }
 
+// Workgroup barrier over LDS only: loads from global memory stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 template <int DT, int BITS, int GS, int MR, int RW>
 __global__ __launch_bounds__(256) void qmv_typed_rows_kernel(const void* x, const uint32_t* w, const void* s,
                                                              const void* b, void* y, int M, int N, int K) {
   using Pc = Piece<DT, BITS>;
   typedef uint32_t wv_t __attribute__((ext_vector_type(Pc::WORDS)));
+  constexpr int D = 2;
   extern __shared__ __attribute__((aligned(16))) unsigned char xsm[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int C = K / Pc::P, G = K / GS;
   const int64_t wstride = K / (32 / BITS);
   const int m0 = blockIdx.y * MR, mr = M - m0 < MR ? M - m0 : MR;
   float* const xsum = reinterpret_cast<float*>(xsm + (size_t)MR * K * Pc::SZ);  // [MR][C]
-  for (int m = 0; m < MR; ++m) {  // (rows past M: copies of the last, never stored)
-    const u32x4* src = reinterpret_cast<const u32x4*>(static_cast<const unsigned char*>(x) +
-                                                      (int64_t)(m0 + (m < mr ? m : mr - 1)) * K * Pc::SZ);
-    u32x4* dst = reinterpret_cast<u32x4*>(xsm + (size_t)m * K * Pc::SZ);
-    for (int e = tid; e < C * Pc::PL; e += 256) dst[(e % Pc::PL) * C + e / Pc::PL] = src[e];
+  // the wave's stream: steps 0 .. S - 1 of rows n0, of rows n0 + stride, ...; loads
+  // are unconditional (clamped past a row's pieces and past the last row), so
+  // that the waits count them
+  struct Row {
+    wv_t w[RW];
+    float s[RW], b[RW];
+  };
+  const int S = (C + 63) / 64, stride = gridDim.x * 4 * RW;
+  int ln = (blockIdx.x * 4 + wave) * RW, lt = 0;  // next step to load: rows, step
+  // (wave-uniform bases: a load then has one 32-bit offset per lane)
+  const uint32_t* wp[RW];
+  const unsigned char *sp[RW], *bp[RW];
+  auto set_rows = [&]() {
+#pragma unroll
+    for (int r = 0; r < RW; ++r) {
+      const int64_t n = ln + r < N ? ln + r : N - 1;
+      wp[r] = w + n * wstride;
+      sp[r] = static_cast<const unsigned char*>(s) + n * G * Pc::SZ;
+      bp[r] = static_cast<const unsigned char*>(b) + n * G * Pc::SZ;
+    }
+  };
+  set_rows();
+  auto load = [&](Row& o) {
+    const int c = lt * 64 + lane, cc = c < C ? c : C - 1, g = cc * Pc::P / GS;
+#pragma unroll
+    for (int r = 0; r < RW; ++r) {
+      o.w[r] = reinterpret_cast<const wv_t*>(wp[r])[cc];
+      o.s[r] = ld<DT>(sp[r], g);
+      o.b[r] = ld<DT>(bp[r], g);
+    }
+    if (++lt == S) {
+      lt = 0;
+      if (ln < N) ln += stride;
+      set_rows();
+    }
+  };
+  int n0 = ln, t = 0;
+  Row ring[D];
+
+  // x to LDS, U units per thread and turn with their loads together, then the
+  // ring's first loads (rows past M: copies of the last, never stored)
+  constexpr int U = MR >= 4 ? 1 : 4 / MR;
+  const int units = C * Pc::PL;
+  for (int e0 = tid; e0 < units; e0 += 256 * U) {
+    u32x4 v[U][MR];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int m = 0; m < MR; ++m)
+        v[u][m] = reinterpret_cast<const u32x4*>(static_cast<const unsigned char*>(x) +
+                                                 (int64_t)(m0 + (m < mr ? m : mr - 1)) * K * Pc::SZ)
+            [e0 + 256 * u < units ? e0 + 256 * u : units - 1];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int e = e0 + 256 * u;
+      if (e >= units) break;
+#pragma unroll
+      for (int m = 0; m < MR; ++m)
+        reinterpret_cast<u32x4*>(xsm + (size_t)m * K * Pc::SZ)[(e % Pc::PL) * C + e / Pc::PL] = v[u][m];
+    }
   }
-  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < D; ++i) load(ring[i]);
+  lds_barrier();
   // plane q of piece c of row m as f32
   auto plane = [&](int m, int q, int c, float* v) {
     const u32x4 a = reinterpret_cast<const u32x4*>(xsm + (size_t)m * K * Pc::SZ)[q * C + c];
@@ -183,84 +249,121 @@ __global__ __launch_bounds__(256) void qmv_typed_rows_kernel(const void* x, cons
       }
     }
   };
-  for (int i = tid; i < MR * C; i += 256) {
-    float t = 0.f;
+  auto piece_sum = [&](int m, int c) {
+    float sum = 0.f;
 #pragma unroll
     for (int q = 0; q < Pc::PL; ++q) {
       float v[Pc::V];
-      plane(i / C, q, i % C, v);
+      plane(m, q, c, v);
 #pragma unroll
-      for (int e = 0; e < Pc::V; ++e) t += v[e];
+      for (int e = 0; e < Pc::V; ++e) sum += v[e];
     }
-    xsum[i] = t;
-  }
-  __syncthreads();
-
-  struct Row {
-    wv_t w[RW];
-    float s[RW], b[RW];
+    return sum;
   };
-  for (int n0 = (blockIdx.x * 4 + wave) * RW; n0 < N; n0 += gridDim.x * 4 * RW) {  // (wave-uniform)
-    auto load = [&](int c, Row& o) {  // piece c (clamped: the last one, never used) of the RW rows
-      const int cc = c < C ? c : C - 1, g = cc * Pc::P / GS;
+  for (int i = tid; i < MR * C; i += 256) xsum[i] = piece_sum(i / C, i % C);
+  lds_barrier();
+
+  float part[RW][MR] = {};
+  auto piece = [&](int c, const Row& o) {
+    if (c >= C) return;
+    float dot[RW][MR] = {};
+    auto one = [&](auto qi) {
+      constexpr int q = decltype(qi)::value;
+      float xv[MR][Pc::V];
+#pragma unroll
+      for (int m = 0; m < MR; ++m) plane(m, q, c, xv[m]);
 #pragma unroll
       for (int r = 0; r < RW; ++r) {
-        const int64_t n = n0 + r < N ? n0 + r : N - 1;
-        o.w[r] = *reinterpret_cast<const wv_t*>(w + n * wstride + cc * Pc::WORDS);
-        o.s[r] = ld<DT>(s, n * G + g);
-        o.b[r] = ld<DT>(b, n * G + g);
+        uint32_t wd[Pc::WORDS];
+#pragma unroll
+        for (int e = 0; e < Pc::WORDS; ++e) wd[e] = o.w[r][e];
+        float cv[Pc::V];
+        piece_codes<BITS, Pc::V, q>(wd, cv);
+#pragma unroll
+        for (int e = 0; e < Pc::V; ++e)
+#pragma unroll
+          for (int m = 0; m < MR; ++m) dot[r][m] = fmaf(xv[m][e], cv[e], dot[r][m]);
       }
     };
-    float part[RW][MR] = {};
-    auto piece = [&](int c, const Row& o) {
-      if (c >= C) return;
-      float dot[RW][MR] = {};
-      auto one = [&](auto qi) {
-        constexpr int q = decltype(qi)::value;
-        float xv[MR][Pc::V];
+    for_planes(one, std::make_integer_sequence<int, Pc::PL>{});
 #pragma unroll
-        for (int m = 0; m < MR; ++m) plane(m, q, c, xv[m]);
+    for (int m = 0; m < MR; ++m) {
+      const float xs = xsum[m * C + c];
 #pragma unroll
-        for (int r = 0; r < RW; ++r) {
-          uint32_t wd[Pc::WORDS];
-#pragma unroll
-          for (int e = 0; e < Pc::WORDS; ++e) wd[e] = o.w[r][e];
-          float cv[Pc::V];
-          piece_codes<BITS, Pc::V, q>(wd, cv);
-#pragma unroll
-          for (int e = 0; e < Pc::V; ++e)
-#pragma unroll
-            for (int m = 0; m < MR; ++m) dot[r][m] = fmaf(xv[m][e], cv[e], dot[r][m]);
-        }
-      };
-      for_planes(one, std::make_integer_sequence<int, Pc::PL>{});
-#pragma unroll
-      for (int m = 0; m < MR; ++m) {
-        const float xs = xsum[m * C + c];
-#pragma unroll
-        for (int r = 0; r < RW; ++r) part[r][m] = fmaf(o.s[r], dot[r][m], fmaf(o.b[r], xs, part[r][m]));
-      }
-    };
-    Row ra, rb;
-    load(lane, ra);
-    int c = lane;
-    for (int j = 0; j < C; j += 128, c += 128) {  // (uniform)
-      if (j + 64 < C) load(c + 64, rb);
-      piece(c, ra);
-      if (j + 128 < C) load(c + 128, ra);
-      if (j + 64 < C) piece(c + 64, rb);
+      for (int r = 0; r < RW; ++r) part[r][m] = fmaf(o.s[r], dot[r][m], fmaf(o.b[r], xs, part[r][m]));
     }
+  };
+  // rows n0 .. done: their sums over the wave, stored, and the next rows
+  auto finish = [&]() {
     float out = 0.f;
 #pragma unroll
     for (int r = 0; r < RW; ++r)
 #pragma unroll
       for (int m = 0; m < MR; ++m) {
-        const float t = qmvdev::wave_sum(part[r][m]);
-        out = lane == r * MR + m ? t : out;
+        const float v = qmvdev::wave_sum(part[r][m]);
+        out = lane == r * MR + m ? v : out;
+        part[r][m] = 0.f;
       }
     const int r = lane / MR, m = lane % MR;
     if (lane < RW * MR && n0 + r < N && m < mr) st<DT>(y, (int64_t)(m0 + m) * N + n0 + r, out);
+    t = 0;
+    n0 += stride;
+  };
+  while (n0 < N) {
+#pragma unroll
+    for (int i = 0; i < D; ++i) {
+      if (n0 < N) {  // (wave-uniform)
+        piece(t * 64 + lane, ring[i]);
+        if (++t == S) finish();
+      }
+      load(ring[i]);
+    }
   }
+}
+
+// One row of f16 x and 4-bit codes of at most 4096 rows: a wave per output row on
+// dot instructions, x from global memory (cached).  A code becomes the f16
+// 1024 + q (bits 0x6400 | q), and q itself by a packed subtraction, both exact, so
+// v_dot2_f32_f16 takes the pairs (q_j, q_j+4) of a word against (x_j, x_j+4);
+// sum(x) of a piece by dots against (1, 1).  Short streams that the kernel
+// above starts too late, staging x first (us, there / here): 2560 x 9728 8.4 /
+// 7.1, 300 x 512 3.5 / 3.1, 1000 x 8192 4.9 / 4.8; 17408 x 5120 17.4 / 18.6.
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+
+template <int GS>
+__global__ __launch_bounds__(256) void qmv_f16_dot_kernel(const void* x, const uint32_t* w, const void* s,
+                                                          const void* b, void* y, int M, int N, int K) {
+  const int lane = threadIdx.x & 63;
+  const int n = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (n >= N) return;
+  const int C = K / 32, G = K / GS;
+  const uint32_t* wrow = w + (int64_t)n * (K / 8);
+  const u32x4* xq = static_cast<const u32x4*>(x);
+  const f16x2 k1024 = {(_Float16)1024.f, (_Float16)1024.f}, one = {(_Float16)1.f, (_Float16)1.f};
+  float part = 0.f;
+  for (int c = lane; c < C; c += 64) {
+    const u32x4 wv = *reinterpret_cast<const u32x4*>(wrow + c * 4);
+    const int g = c * 32 / GS;
+    const float sc = ld<2>(s, (int64_t)n * G + g), bi = ld<2>(b, (int64_t)n * G + g);
+    float dot = 0.f, xs = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const u32x4 v = xq[c * 4 + i];  // values 32 c + 8 i .. + 7
+      const uint32_t pr[4] = {__builtin_amdgcn_perm(v[2], v[0], 0x05040100u), __builtin_amdgcn_perm(v[2], v[0], 0x07060302u),
+                              __builtin_amdgcn_perm(v[3], v[1], 0x05040100u), __builtin_amdgcn_perm(v[3], v[1], 0x07060302u)};
+      const uint32_t wd = wv[i];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t q = ((wd >> (4 * j)) & 0x000F000Fu) | 0x64006400u;
+        const f16x2 xp = __builtin_bit_cast(f16x2, pr[j]);
+        dot = __builtin_amdgcn_fdot2(xp, __builtin_bit_cast(f16x2, q) - k1024, dot, false);
+        xs = __builtin_amdgcn_fdot2(xp, one, xs, false);
+      }
+    }
+    part = fmaf(sc, dot, fmaf(bi, xs, part));
+  }
+  const float t = wsum64(part);
+  if (lane == 0) st<2>(y, n, t);
 }
 
 // Matmul: 64 x 64 output tile per workgroup, K in steps of 32 through LDS (x
@@ -571,6 +674,7 @@ TypedRows pick_rows_mr(int MR, int RW) {
   if (MR == 1 && RW == 1) return {qmv_typed_rows_kernel<DT, BITS, GS, 1, 1>, 1};
   if (MR == 1 && RW == 2) return {qmv_typed_rows_kernel<DT, BITS, GS, 1, 2>, 2};
   if (MR == 1 && RW == 4) return {qmv_typed_rows_kernel<DT, BITS, GS, 1, 4>, 4};
+  if (MR == 2 && RW == 1) return {qmv_typed_rows_kernel<DT, BITS, GS, 2, 1>, 1};
   if (MR == 2 && RW == 2) return {qmv_typed_rows_kernel<DT, BITS, GS, 2, 2>, 2};
   if (MR == 2 && RW == 4) return {qmv_typed_rows_kernel<DT, BITS, GS, 2, 4>, 4};
   if (MR == 4 && RW == 2) return {qmv_typed_rows_kernel<DT, BITS, GS, 4, 2>, 2};
@@ -695,23 +799,35 @@ int launch_typed_mm(hipStream_t st, bool matvec, const void* x, const uint32_t* 
   // Matvec, x and W 16-byte aligned and a row of x fits the LDS: the rows
   // kernel.  Rows of x per workgroup (MR): four save re-reading a large W where
   // they take at most 48 KB of LDS (f16 8-bit 17408 x 5120 4 rows 30.5 us, two
-  // at a time 37.2; 12 rows 71 / 90), two otherwise (bf16 8-bit 9728 x 2560 4 rows
-  // 11.6 us, 15.3 four at a time; 12 rows 26 / 31), one where two pass that
-  // (bf16 8-bit 5120 x 17408 4 rows 42 us, 62 / 48 at four / two).  Rows of W per
-  // wave (RW): one row of x two, one below 4096 rows (f32 1000 x 8192 RW 2 6.0 us,
-  // RW 4 7.6); several rows of x one at a time four; else four, two where that
-  // leaves a compute unit without a workgroup.
+  // at a time 37.2; 12 rows 71 / 90), else two up to 48 KB, and of 16-bit types up
+  // to 80 KB (bf16 8-bit 5120 x 17408 4 rows 38 us, one at a time 51; 12 rows 86 /
+  // 147; but 4-bit 3 rows 38.7 / 35.4; f32 4-bit 2560 x 9728 3 rows 18.9 / 14.6), else one.
+  // Rows of W per wave (RW): one row of x two, one below 4096 rows (f32 1000 x
+  // 8192 RW 2 6.0 us, RW 4 7.6); else four where that makes a workgroup per
+  // compute unit, of 16-bit pairs of rows 400 (bf16 8-bit 2 rows of 4096 x 4096, 256
+  // with four rows, 8.2 us, with two 6.5; 6 rows of 2560 x 9728, 480, 15.0 / 18.9), and
+  // one where two leave compute units without a workgroup.
+  const bool al16 = reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0;
+  if (matvec && M == 1 && dtype == LISAQ_DTYPE_F16 && bits == 4 && al16 && N <= 4096) {
+    const typed_fn dot = gs == 32 ? qmv_f16_dot_kernel<32> : gs == 64 ? qmv_f16_dot_kernel<64> : qmv_f16_dot_kernel<128>;
+    hipLaunchKernelGGL(dot, dim3((unsigned)((N + 3) / 4)), dim3(256), 0, st, x, w, s, b, y, 1, (int)N, (int)K);
+    return check_launch("quantized_matmul_typed");
+  }
   const int P = bits == 8 ? 16 : 32;
   const int64_t per_row = K * (dtype == LISAQ_DTYPE_F32 ? 4 : 2) + K / P * 4;
-  if (matvec && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0 &&
-      per_row <= 160 * 1024) {
+  if (matvec && al16 && per_row <= 160 * 1024) {
     const int64_t room = 48 * 1024;
+    const bool half = dtype != LISAQ_DTYPE_F32;
     const int MR = M >= 3 && N * K * bits / 8 >= ((int64_t)32 << 20) && 4 * per_row <= room ? 4
-                   : M >= 2 && 2 * per_row <= room                                          ? 2
+                   : M >= 2 && 2 * per_row <= (half && M != 3 ? 80 * 1024 : room)           ? 2
                                                                                             : 1;
     const int64_t groups = (M + MR - 1) / MR;
-    const int RW = M == 1 ? (N >= 4096 ? 2 : 1) : (N + 15) / 16 * groups >= 256 ? 4 : 2;
-    const TypedRows k = pick_rows(dtype, bits, gs, MR, MR == 1 && M > 1 ? 4 : RW);
+    const auto blocks_of = [&](int rw) { return (N + 4 * rw - 1) / (4 * rw) * groups; };
+    const int RW = M == 1                                              ? (N >= 4096 ? 2 : 1)
+                   : blocks_of(4) >= (MR == 2 && half ? 400 : 256)     ? 4
+                   : blocks_of(2) >= 256 || MR == 4                    ? 2
+                                                                       : 1;
+    const TypedRows k = pick_rows(dtype, bits, gs, MR, RW);
     if (k.fn) {
       const int lds = (int)(MR * per_row);
       if (int rc = allow_dyn_lds((const void*)k.fn, lds, "quantized_matmul_typed")) return rc;

@@ -296,3 +296,46 @@ def test_typed_matmul_unaligned_x(dev, oracle, dtype, bits, M, N, K, gs):
     _close(run(off(x), wd, sd, bd), ref, dtype, "unaligned x")
     _close(run(x, off(wd), sd, bd), ref, dtype, "unaligned w")
     _close(run(x, wd, off(sd), off(bd)), ref, dtype, "unaligned scales")
+
+
+@pytest.mark.parametrize("scale", [1.0, 2.0**-21])
+@pytest.mark.parametrize("N,K,gs", [(1, 32, 32), (7, 128, 128), (4095, 2080, 32), (4096, 1024, 64), (2560, 9728, 128)])
+def test_f16_one_row_dot(dev, oracle, N, K, gs, scale):
+    """One f16 row and 4-bit codes of at most 4096 rows (dot instructions) at the edges of its pieces and rows, against
+    the oracle; scale 2^-21: values of x below the smallest normal f16, which count like any other."""
+    rng = np.random.default_rng(N + K)
+    w, s, b = np_linear(rng, N, K, 4, gs)
+    up = np.float32(2.0**10 if scale < 1 else 1.0)
+    sf = oracle._round_to(bf16_bits_to_f32(s) * up, "f16")
+    bf = oracle._round_to(bf16_bits_to_f32(b) * up, "f16")
+    xf = oracle._round_to(rng.standard_normal((1, K)).astype(np.float32) * np.float32(scale), "f16")
+    y = ops.quantized_matmul(_tensor(xf, "f16", dev), to_dev_u32(w, dev), _tensor(sf, "f16", dev),
+                             _tensor(bf, "f16", dev), True, gs, 4).float().cpu().numpy()
+    ref = oracle.qmv_typed(xf, w, sf, bf, gs, 4)
+    # one rounding to f16 (2^-11 relative, 2^-25 below its normal range) and f32 sums
+    mag = oracle.qmv_typed(np.abs(xf), w, np.abs(sf), np.abs(bf), gs, 4)
+    assert (np.abs(y - ref) <= 2.0**-10 * np.abs(ref) + 2.0**-24 + K * 2.0**-24 * mag).all()
+
+
+@pytest.mark.parametrize("dtype,bits", [("bf16", 8), ("f16", 2), ("f16", 4), ("f16", 8), ("f32", 4), ("f32", 8)])
+@pytest.mark.parametrize("M,N,K,gs", [
+    (2, 9, 2048, 64),        # pairs of rows of x, one row of W per wave, most workgroups' waves without rows
+    (2, 3001, 1056, 32),     # a wave's stream of several rows, its last piece's lanes partly past the row
+    (4, 700, 17408, 64),     # 16 bits: pairs of long rows (80 KB); f32: one at a time, one row of W per wave
+    (3, 2600, 12288, 128),   # three long rows one at a time, four rows of W
+    (1, 33000, 96, 32),      # short rows: every step ends one, more rows than the chip holds at once
+    (12, 33000, 64, 64),
+])
+def test_typed_matvec_streams(dev, oracle, dtype, bits, M, N, K, gs):
+    """The matvec's streams of rows: steps that cross from one row to the next, clamped ends, long and short rows."""
+    rng = np.random.default_rng(M + N + K + bits)
+    w, s, b = np_linear(rng, N, K, bits, gs, s_std=0.02 if bits < 8 else 0.002)
+    sf = oracle._round_to(bf16_bits_to_f32(s), dtype)
+    bf = oracle._round_to(bf16_bits_to_f32(b), dtype)
+    xf = oracle._round_to(rng.standard_normal((M, K)).astype(np.float32), dtype)
+    assert M < ops.qmv_batch_limit(K, N)
+    y = ops.quantized_matmul(_tensor(xf, dtype, dev), to_dev_u32(w, dev), _tensor(sf, dtype, dev),
+                             _tensor(bf, dtype, dev), True, gs, bits).float().cpu().numpy()
+    q = oracle.unpack(w, K, bits).astype(np.float64)
+    wd = np.repeat(sf.astype(np.float64), gs, 1) * q + np.repeat(bf.astype(np.float64), gs, 1)
+    _close(y, xf.astype(np.float64) @ wd.T, dtype, f"{dtype} bits={bits} {M}x{N}x{K}")
