@@ -204,7 +204,7 @@ constexpr int kGatherMvRows = 16;
 // knows one (moe_forward: a token picks an expert at most once, so T);
 // otherwise R.  It only sizes the matvec rows and decides if matmul tiles can
 // occur; the tables still follow the actual runs.
-// tall: matmul tiles of kTallBM rows (runs known to average >= kTallAvg rows).
+// tall: matmul tiles of kTallBM rows (runs known to average >= qmm_tall_avg rows).
 // gu: tables for gate|up + SwiGLU (N = I): matvec entries of half a block's
 // rows (the other half of its waves take the up weights), matmul tiles of the
 // gate|up matmul kernel.
@@ -283,7 +283,7 @@ static GatherLayout gather_layout(int64_t R, int64_t N, int64_t K, int E, int gs
     }
   }
   if (gu) {
-    L.mc.BM = qmm_gu_rows(R, E);
+    L.mc.BM = qmm_gu_rows(R, E, N);
     L.mc.BN = kGuBN;
   }
   // A run's last tile of at most kShortBM rows goes to a kernel of short
@@ -911,13 +911,13 @@ int lisaq_gather_rows(void* stream, const void* x, const int32_t* rows, void* ou
 // table (see gather_layout)
 static int64_t gu_cap(int64_t R, int64_t I, int E) {
   const int64_t runs = R < E ? R : E;
-  const int BM = qmm_gu_rows(R, E);
+  const int BM = qmm_gu_rows(R, E, I);
   return ((R + BM - 1) / BM + runs) * ((I + kGuBN - 1) / kGuBN);
 }
 static int64_t gu_short_cap(int64_t R, int64_t I, int E) {
   const int64_t runs = R < E ? R : E;
   constexpr int sbn = kShortBN / 2;  // output columns of a short gate|up tile
-  return qmm_gu_rows(R, E) > kShortBM && path_int("LISAQ_GATHER_SHORT", 1) != 0 ? runs * ((I + sbn - 1) / sbn) : 0;
+  return qmm_gu_rows(R, E, I) > kShortBM && path_int("LISAQ_GATHER_SHORT", 1) != 0 ? runs * ((I + sbn - 1) / sbn) : 0;
 }
 // workspace of the gate|up tables: [counts 256 B][tiles][short tiles]
 static size_t gu_ws_bytes(int64_t R, int64_t I, int E) {
@@ -942,7 +942,7 @@ static TileTableJob gu_job(int64_t R, int64_t I, int E, void* ws) {
   j.N = (int)I;
   j.limit = 1;  // every run as matmul tiles
   j.MV = 1;
-  j.BM = qmm_gu_rows(R, E);
+  j.BM = qmm_gu_rows(R, E, I);
   j.BN = kGuBN;
   j.mv_vr[0] = j.mv_vr[1] = 16;
   j.qmm_tab = (int4*)(gb + 256);
@@ -990,7 +990,7 @@ static int gate_up_swiglu(hipStream_t st, const void* x, const int32_t* xrows, i
   p.K = (int)H;
   p.G = (int)(H / gs);
   p.ksplit = 1;
-  if (int rc = qmm_gu_launch(st, p, bits, gs, (int)cap, qmm_gu_rows(R, E))) return rc;
+  if (int rc = qmm_gu_launch(st, p, bits, gs, (int)cap, qmm_gu_rows(R, E, I))) return rc;
   if (scap == 0) return LISAQ_OK;
   p.tiles = (const int4*)(gb + 256 + up256((size_t)cap * 16));
   return qmm_gu_launch(st, p, bits, gs, (int)scap, kShortBM);
@@ -1074,10 +1074,10 @@ struct MoeLayout {
 };
 
 // The down projection of the fused-gate|up prefill takes kTallBM-row matmul
-// tiles when runs average >= kTallAvg rows (as the gate|up matmul does).
+// tiles when runs average >= qmm_tall_avg rows (as the gate|up matmul does).
 static bool moe_down_tall(int64_t T, int64_t H, int64_t I, int E, int k, int gs, int bits) {
   return moe_gu_path(T, H, I, E, k, gs, bits) && tune_int("LISAQ_MOE_DOWN_TALL", 1) != 0 &&
-         T * k >= kTallAvg * (int64_t)E;
+         T * k >= qmm_tall_avg(E, I) * (int64_t)E;
 }
 
 static MoeLayout moe_layout(int64_t T, int64_t H, int64_t I, int E, int k, int gs, int bits) {

@@ -44,10 +44,10 @@ int qmm_launch(hipStream_t stream, const QmmConfig& c, QmmParams p, int bits, in
 // Gate|up matmul of the MoE prefill: tile-table launch of `grid` workgroups,
 // y = SwiGLU(x . gate^T, x . up^T) over 128-column output tiles of 128 rows,
 // x rows gathered through p.xrows (qmm_gu.hip).
-// rows: the row tile, qmm_gu_rows(R, E) (the tile table's BM).
+// rows: the row tile, qmm_gu_rows(R, E, I) (the tile table's BM).
 int qmm_gu_launch(hipStream_t stream, const QmmParams& p, int bits, int gs, int grid, int rows);
 constexpr int kGuBN = 128;          // output-column tile of qmm_gu_launch
-int qmm_gu_rows(int64_t R, int E);  // its row tile for R sorted rows over E experts
+int qmm_gu_rows(int64_t R, int E, int64_t I);  // its row tile for R sorted rows over E experts of I columns
 // Gather (tile-table) launch of `rows`-row tiles (256, or 64 for the short
 // last tiles of runs).
 int qmm_gather_launch(hipStream_t stream, const QmmParams& p, int bits, int gs, int grid, int rows);
@@ -55,10 +55,10 @@ int qmm_gather_launch(hipStream_t stream, const QmmParams& p, int bits, int gs, 
 // at most this many rows.  Its rows are bitwise equal to the same rows in a
 // taller tile (the accumulation order does not depend on the tile height).
 constexpr int kShortBM = 64;
-// Row tile of the tall gather launches (runs averaging >= kTallAvg rows:
+// Row tile of the tall gather launches (runs averaging >= qmm_tall_avg rows:
 // gate|up and down of the MoE prefill): 288 rows, nine 32-row blocks
 constexpr int kTallBM = 288;
-constexpr int kTallAvg = 120;  // (the crossover lies between 112 and 125 rows a run, see qmm_gu_rows)
+int qmm_tall_avg(int E, int64_t I);  // (see qmm_gu.hip)
 // (four waves, 128 columns: MoE T = 4096 471 -> 476 us, T = 512 173 -> 180 us)
 constexpr int kShortWN = 8;  // waves of a short-tile workgroup (32 columns each)
 constexpr int kShortBN = 32 * kShortWN;   // output columns of a short tile (gate|up: half of them)

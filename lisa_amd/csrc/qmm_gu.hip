@@ -20,17 +20,27 @@ namespace lisaq {
 constexpr bool kSkip(int mt) { return mt <= 2 || mt == 9; }
 
 
-// Row tile: 288 rows when the average expert run is at least kTallAvg rows,
+// Row tile: 288 rows when the average expert run is at least qmm_tall_avg rows,
 // else 128 rows.  A K-step of a tile costs about 0.55 us + 6 ns per active row
 // (dequantization, copies and the barrier do not depend on the rows), so one
 // tall tile per run, its empty 32-row blocks skipped, beats a 128-row tile
-// and a second one or a short one as soon as runs pass 128 rows.  Whole block,
-// 128 -> 288 rows (E = 128, k = 8, H = 2048, I = 768): T = 1800 (112 rows a
-// run) 291 -> 303 us, T = 2100 338 -> 316, T = 2500 386 -> 337, T = 3000 442 ->
-// 358; E = 32: T = 500 (125 rows) 120 -> 103; E = 64, H = 1024, I = 512: T =
-// 1500 (187 rows) 130 -> 97.
-int qmm_gu_rows(int64_t R, int E) {
-  return R >= kTallAvg * (int64_t)E ? kTallBM : 128;
+// and a second one or a short one as soon as runs pass 128 rows -- where the
+// tiles of a launch make two rounds of workgroups and more, however the tokens
+// are spread over the experts.  With fewer tiles the launch ends with its longest,
+// and uneven runs want low ones.  Whole block, us, 128- / 288-row tiles, router
+// logits N(0, 1) and the same plus a ramp of 1 over the experts:
+//   E = 128, k = 8, H = 2048, I = 768 (768 workgroups): T = 1800 (112 rows a run)
+//     291 / 303; T = 2200 347 / 309, ramp 367 / 355; T = 2600 404 / 330, ramp 373 / 360
+//   E = 64, k = 8, the same H, I (384): T = 960 (120 rows) 173 / 174, ramp 172 / 209;
+//     T = 1200 207 / 189, ramp 203 / 227; T = 1400 (175) 228 / 202, ramp 232 / 233
+//   E = 32, k = 4, H = 1024, I = 512 (128): T = 1200 (150) 82 / 74, ramp 83 / 103
+//   E = 16, k = 2, H = 2048, I = 1024 (128): T = 1200 113 / 101, ramp 115 / 148
+int qmm_tall_avg(int E, int64_t I) {
+  const int64_t wg = E * ((I + kGuBN - 1) / kGuBN);
+  return wg >= 512 ? 120 : wg >= 320 ? 170 : 192;
+}
+int qmm_gu_rows(int64_t R, int E, int64_t I) {
+  return R >= qmm_tall_avg(E, I) * (int64_t)E ? kTallBM : 128;
 }
 
 template <int MT, int WN = 8, int NB = 3>
@@ -70,7 +80,7 @@ int qmm_gu_launch(hipStream_t stream, const QmmParams& p, int bits, int gs, int 
 }
 
 // Gather launches of 288-row tiles (the MoE prefill's down projection when
-// runs average >= kTallAvg rows) and of 64-row tiles (the short last tile of a
+// runs average >= qmm_tall_avg rows) and of 64-row tiles (the short last tile of a
 // run, skipping the matrix instructions of an empty 32-row block).
 int qmm_gather_launch(hipStream_t stream, const QmmParams& p, int bits, int gs, int grid, int rows) {
   qmm_fn fn = nullptr;

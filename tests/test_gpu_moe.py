@@ -551,8 +551,8 @@ def test_gather_short_last_tiles(dev, oracle, force_path, runs):
 @pytest.mark.parametrize("T,bits,I", [(479, 4, 320), (480, 4, 320), (480, 2, 320), (700, 4, 320), (479, 4, 384),
                                       (480, 4, 384), (480, 2, 384), (700, 4, 384)])
 def test_moe_forward_tile_height_rule(dev, oracle, T, bits, I):
-    """Runs averaging just below and from 120 rows on (128- and 288-row tiles; 175 rows: a run's second tile too), an
-    odd and an even number of groups in the down projection: moe_forward bitwise equal to the composition over
+    """Runs averaging 120 to 175 rows (a run's second tile too; the tile-height rule by the number of workgroups:
+    test_moe_forward_uneven_runs), an odd and an even number of groups in the down projection: moe_forward bitwise equal to the composition over
     128-row gather tiles, whose gate, up and down of the longest and the shortest run agree with the oracle."""
     import torch
 
@@ -611,3 +611,37 @@ def test_gather_odd_group_counts(dev, oracle, runs, N, K, gs, bits):
         ref = bf16_bits_to_f32(oracle.swiglu(oracle.f32_to_bf16(g), u))
         assert_close_bf16(act[a:b], ref, rtol=2e-2, what=f"gather_qmm_swiglu expert {e} ({n} rows)")
         a = b
+
+
+@pytest.mark.parametrize("E,k,T,H,I,skew", [(16, 2, 1535, 128, 128, 3.0),    # 191 rows a run: 128-row tiles
+                                            (16, 2, 1536, 128, 128, 3.0),    # 192: tall ones
+                                            (40, 4, 1699, 128, 1024, 1.0),   # 320 workgroups: 169 rows
+                                            (40, 4, 1700, 128, 1024, 1.0),   # and 170
+                                            (128, 8, 1919, 128, 512, 1.0),   # 512 workgroups: 119 rows
+                                            (128, 8, 1920, 128, 512, 1.0),   # and 120
+                                            (8, 4, 2000, 128, 192, 6.0),     # a run of almost every token
+                                            (1, 1, 700, 128, 256, 0.0)])     # one run
+def test_moe_forward_uneven_runs(dev, E, k, T, H, I, skew):
+    """Both sides of the tile-height rule, by the number of workgroups, with uneven runs: moe_forward bitwise equal to
+    the composition over 128-row gather tiles."""
+    import torch
+
+    rng = np.random.default_rng(E + T)
+    G, U, D = (_expert_stack(rng, E, n, m) for n, m in ((I, H), (I, H), (H, I)))
+    x = to_dev_bf16(np_x(rng, T, H), dev)
+    lg = rng.standard_normal((T, E)) + np.linspace(0.0, skew, E)[None]
+    lg = to_dev(lg.astype(np.float32), dev)
+    dv = [tuple(to_dev_u32(a, dev) if i == 0 else to_dev_bf16(a, dev) for i, a in enumerate(st)) for st in (G, U, D)]
+    out = ops.moe_forward(x, lg, dv[0], dv[1], dv[2], k)
+    ridx, rw = ops.moe_route(lg, k)
+    srt, order, rows, inv, offs = ops.moe_sort(ridx.reshape(-1), E, k)
+    act = ops.gather_qmm_swiglu(x, rows, dv[0], dv[1], srt)
+    xs = ops.gather_rows(x, rows)
+    g, u = (ops.gather_qmm(xs, *dv[i], rhs_indices=srt) for i in (0, 1))
+    comp = ops.swiglu(g, u)
+    o, lim = offs.cpu().numpy(), ops.qmv_batch_limit(H, I)
+    long = torch.from_numpy(np.repeat(np.diff(o) >= lim, np.diff(o))).to(dev)  # (rows with the matmul arithmetic)
+    assert long.any() and torch.equal(act[long].view(torch.int16), comp[long].view(torch.int16))
+    d = ops.gather_qmm(act, *dv[2], rhs_indices=srt)
+    ref = ops.moe_combine(d, rw.reshape(-1), inv, T, k)
+    assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
