@@ -42,7 +42,7 @@ METRIC = "4-bit qmv GB/s (% HBM peak) @M=1; qmm TFLOP/s (% bf16 MFMA peak) @M=20
 QMV_TRAFFIC_BYTES = round((24576.5 * 1.9993 + 136.0) * 1024)
 QMM_TRAFFIC_BYTES = round((243697.5 * 1.9993 + 131780.5) * 1024)
 QMV_KERNEL = "lisaq::qmvp_kernel<4, 64, 3, 2, 16, 1, false>"
-QMM_KERNEL = "lisaq::qmm_kernel<4, 64, 8, 1, 8, true, false, 3, false, 0>"  # M=2048: 256-row tiles, last round split over K (+ qmm_hybrid_reduce_kernel)
+QMM_KERNEL = "lisaq::qmm_kernel<4, 64, 8, 1, 8, true, false, 3, false, 0, false>"  # M=2048: 256-row tiles, last round split over K (+ qmm_hybrid_reduce_kernel)
 
 
 def qmv_bytes(M, N, K, bits=4, gs=64):

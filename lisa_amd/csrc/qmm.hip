@@ -218,15 +218,15 @@ static qmm_fn rows_pick(const QmmConfig& c, int bits, int gs, int ct, int* lds) 
 }
 
 template <bool SPLIT>
-static qmm_fn qmm_pick(const QmmConfig& c, int bits, int gs, int ct, int* lds) {
+static qmm_fn qmm_pick(const QmmConfig& c, int bits, int gs, int ct, bool odd, int* lds) {
   if (ct == kCtBf16) {
-    if (bits == 4) return qmm_get<4, SPLIT>(gs, c.MT, lds);
-    if (bits == 2) return qmm_get<2, SPLIT>(gs, c.MT, lds);
-    if (bits == 8) return qmm_get<8, SPLIT>(gs, c.MT, lds);
+    if (bits == 4) return qmm_get<4, SPLIT>(gs, c.MT, odd, lds);
+    if (bits == 2) return qmm_get<2, SPLIT>(gs, c.MT, odd, lds);
+    if (bits == 8) return qmm_get<8, SPLIT>(gs, c.MT, odd, lds);
   } else if (ct == kCtF16) {
-    if (bits == 4) return qmm_get<4, SPLIT, kCtF16>(gs, c.MT, lds);
-    if (bits == 2) return qmm_get<2, SPLIT, kCtF16>(gs, c.MT, lds);
-    if (bits == 8) return qmm_get<8, SPLIT, kCtF16>(gs, c.MT, lds);
+    if (bits == 4) return qmm_get<4, SPLIT, kCtF16>(gs, c.MT, odd, lds);
+    if (bits == 2) return qmm_get<2, SPLIT, kCtF16>(gs, c.MT, odd, lds);
+    if (bits == 8) return qmm_get<8, SPLIT, kCtF16>(gs, c.MT, odd, lds);
   }
   return nullptr;
 }
@@ -249,7 +249,10 @@ int qmm_launch(hipStream_t stream, const QmmConfig& c, QmmParams p, int bits, in
     return set_error(LISAQ_EUNSUPPORTED, "qmm: split over K with %d-row tiles (%s layout) is not built", 32 * c.MT,
                      c.full_tiles > 0 ? "hybrid" : "per-part");
   int lds = 0;
-  qmm_fn fn = c.rows ? rows_pick(c, bits, gs, ct, &lds) : split ? qmm_pick<true>(c, bits, gs, ct, &lds) : qmm_pick<false>(c, bits, gs, ct, &lds);
+  const bool odd = p.G & 1;
+  qmm_fn fn = c.rows  ? rows_pick(c, bits, gs, ct, &lds)
+              : split ? qmm_pick<true>(c, bits, gs, ct, odd, &lds)
+                      : qmm_pick<false>(c, bits, gs, ct, odd, &lds);
   if (!fn) return set_error(LISAQ_EUNSUPPORTED, "qmm: bits=%d group_size=%d not supported", bits, gs);
   if (int rc = allow_dyn_lds((const void*)fn, lds, "qmm")) return rc;
   p.ksplit = split ? c.S : 1;

@@ -43,14 +43,21 @@ int qmm_gu_rows(int64_t R, int E, int64_t I) {
   return R >= qmm_tall_avg(E, I) * (int64_t)E ? kTallBM : 128;
 }
 
+// the kernel for rows of G groups, an even or an odd number
+template <int B, int GS, int MT, int WN, bool GU, int NB>
+static qmm_fn pick_odd(int G) {
+  if (G & 1) return qmm_kernel<B, GS, MT, 1, WN, false, GU, NB, kSkip(MT), kCtBf16, true>;
+  return qmm_kernel<B, GS, MT, 1, WN, false, GU, NB, kSkip(MT)>;
+}
+
 template <int MT, int WN = 8, int NB = 3>
 static int gu_launch(hipStream_t stream, const QmmParams& p, int bits, int gs, int grid) {
   qmm_fn fn = nullptr;
   auto pick = [&](auto bt) {
     constexpr int B = decltype(bt)::value;
     if (gs == 32) fn = qmm_kernel<B, 32, MT, 1, WN, false, true, NB, kSkip(MT)>;
-    if (gs == 64) fn = qmm_kernel<B, 64, MT, 1, WN, false, true, NB, kSkip(MT)>;
-    if (gs == 128) fn = qmm_kernel<B, 128, MT, 1, WN, false, true, NB, kSkip(MT)>;
+    if (gs == 64) fn = pick_odd<B, 64, MT, WN, true, NB>(p.G);
+    if (gs == 128) fn = pick_odd<B, 128, MT, WN, true, NB>(p.G);
   };
   if (bits == 4) pick(std::integral_constant<int, 4>{});
   if (bits == 2) pick(std::integral_constant<int, 2>{});
@@ -92,8 +99,8 @@ int qmm_gather_launch(hipStream_t stream, const QmmParams& p, int bits, int gs, 
     lds = QmmLds<B, 64, MT, 1, WN, NB>::TOTAL;
     threads = 64 * WN;
     if (gs == 32) fn = qmm_kernel<B, 32, MT, 1, WN, false, false, NB, kSkip(MT)>;
-    if (gs == 64) fn = qmm_kernel<B, 64, MT, 1, WN, false, false, NB, kSkip(MT)>;
-    if (gs == 128) fn = qmm_kernel<B, 128, MT, 1, WN, false, false, NB, kSkip(MT)>;
+    if (gs == 64) fn = pick_odd<B, 64, MT, WN, false, NB>(p.G);
+    if (gs == 128) fn = pick_odd<B, 128, MT, WN, false, NB>(p.G);
   };
   LISAQ_REQUIRE(rows == 64 || rows == kTallBM, LISAQ_EUNSUPPORTED, "qmm gather: row tile %d not built", rows);
   auto pick_mt = [&](auto bt) {

@@ -5,8 +5,8 @@
 namespace lisaq {
 
 template <>
-qmm_fn qmm_get<2, true>(int gs, int MT, int* lds) {
-  return qmm_get_impl<2, true>(gs, MT, lds);
+qmm_fn qmm_get<2, true>(int gs, int MT, bool odd, int* lds) {
+  return qmm_get_impl<2, true>(gs, MT, odd, lds);
 }
 
 }  // namespace lisaq

@@ -258,14 +258,17 @@ struct QmmLds {
 //
 // SKIP (tile-table launches; implied by GU): 32-row blocks past the tile's rows
 // skip their matrix instructions.
+//
+// OG: rows of an odd number of groups (see pad).
 template <int BITS, int GS, int MT, int NT, int WN, bool SPLIT, bool GU = false, int NB = 3, bool SKIP = GU,
-          int CT = kCtBf16>
+          int CT = kCtBf16, bool OG = false>
 __global__ __launch_bounds__(64 * WN) void qmm_kernel(QmmParams p) {
   using G = MGeo<BITS>;
   using C = Ct<CT>;
   using L = QmmLds<BITS, GS, MT, NT, WN, NB>;
   static_assert(!GU || CT == kCtBf16, "SwiGLU epilogue: bf16 only");
   static_assert(NB == 3, "ring depth");
+  static_assert(!OG || GS > 32, "K is a multiple of 64: an even number of groups of 32");
   constexpr int BM = L::BM;
   constexpr int BN = L::BN;
   constexpr int NWV = WN;  // waves per workgroup
@@ -463,11 +466,11 @@ __global__ __launch_bounds__(64 * WN) void qmm_kernel(QmmParams p) {
   // end, which the descriptor's range check returns as zero.  So such rows are
   // cut into blocks from their end: block 0 starts `pad` groups before the row
   // and every dword of a row's blocks ends with the row.  Steps count from
-  // kbs where scales and biases are meant, and the loop does the same work either
-  // way (a two-byte shift of the last block alone cost it three scalar
-  // instructions a step, 500 x 5120 x 5120 42.1 -> 42.5 us).  Nothing before row 0
-  // is read: the first rows' block 0 is put together in the prologue.
-  const int pad = GS > 32 && (p.G & 1) ? 8 - (p.G & 7) : 0;
+  // kbs where scales and biases are meant.  Nothing before row 0 is read: the first
+  // rows' block 0 is put together in the prologue.  (Kernels of their own: one
+  // kernel for both kinds took 1% more time for the MoE prefill's even rows,
+  // T = 3000 356 -> 360 us.)
+  const int pad = OG ? 8 - (p.G & 7) : 0;
   const int kbs = kb + pad * (GS / BK);
   // scale/bias block sb (groups 8 sb - pad .. 8 sb - pad + 7 of every row; past
   // its ends: other rows' groups or zeros, never used) into block buffer sb % 2
@@ -573,7 +576,7 @@ __global__ __launch_bounds__(64 * WN) void qmm_kernel(QmmParams p) {
   // an odd number of groups: the lanes whose row starts fewer than `pad` groups
   // into the array (and was copied from its start) put block 0's groups in
   // their places (the copy has landed)
-  if (pad > 0 && kbs / SBK == 0) {
+  if (OG && kbs / SBK == 0) {
 #pragma unroll
     for (int q = 0; q < SBI; ++q) {
       const int idx = wave + NWV * q;
@@ -897,14 +900,20 @@ typedef void (*qmm_fn)(QmmParams);
 // qmm_t<type><bits>.hip instantiate the
 // tile heights MT = 4, 6, 8 and group sizes 32, 64, 128 (eight waves, NT = 1),
 // so the units compile in parallel.  *lds = dynamic LDS bytes.
+// odd: an odd number of groups a row (bf16 with 2 and 4 bits; never in groups of 32).
 template <int BITS, bool SPLIT, int CT = kCtBf16>
-qmm_fn qmm_get(int gs, int MT, int* lds);
+qmm_fn qmm_get(int gs, int MT, bool odd, int* lds);
 
 template <int BITS, bool SPLIT, int CT = kCtBf16>
-qmm_fn qmm_get_impl(int gs, int MT, int* lds) {
+qmm_fn qmm_get_impl(int gs, int MT, bool odd, int* lds) {
   auto one = [&](auto mt) -> qmm_fn {
     constexpr int M_ = decltype(mt)::value;
     *lds = QmmLds<BITS, 64, M_, 1, 8>::TOTAL;  // (group-size independent)
+    if constexpr (CT == kCtBf16 && BITS != 8) {
+      if (odd && gs == 64) return qmm_kernel<BITS, 64, M_, 1, 8, SPLIT, false, 3, false, CT, true>;
+      if (odd && gs == 128) return qmm_kernel<BITS, 128, M_, 1, 8, SPLIT, false, 3, false, CT, true>;
+    }
+    if (odd) return nullptr;
     if (gs == 32) return qmm_kernel<BITS, 32, M_, 1, 8, SPLIT, false, 3, false, CT>;
     if (gs == 64) return qmm_kernel<BITS, 64, M_, 1, 8, SPLIT, false, 3, false, CT>;
     if (gs == 128) return qmm_kernel<BITS, 128, M_, 1, 8, SPLIT, false, 3, false, CT>;

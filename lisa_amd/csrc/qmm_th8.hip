@@ -5,13 +5,13 @@
 namespace lisaq {
 
 template <>
-qmm_fn qmm_get<8, false, kCtF16>(int gs, int MT, int* lds) {
-  return qmm_get_impl<8, false, kCtF16>(gs, MT, lds);
+qmm_fn qmm_get<8, false, kCtF16>(int gs, int MT, bool odd, int* lds) {
+  return qmm_get_impl<8, false, kCtF16>(gs, MT, odd, lds);
 }
 
 template <>
-qmm_fn qmm_get<8, true, kCtF16>(int gs, int MT, int* lds) {
-  return qmm_get_impl<8, true, kCtF16>(gs, MT, lds);
+qmm_fn qmm_get<8, true, kCtF16>(int gs, int MT, bool odd, int* lds) {
+  return qmm_get_impl<8, true, kCtF16>(gs, MT, odd, lds);
 }
 
 }  // namespace lisaq
