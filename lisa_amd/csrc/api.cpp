@@ -605,7 +605,7 @@ int lisaq_quantized_matmul(void* stream, const void* x, const uint32_t* w, const
 static bool typed_tiles_faster(int64_t M, int64_t N, int64_t K) {
   const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64);
   if (M <= 64 && K > (M <= 32 ? 256 : 512)) return false;
-  if (K > 768) return K <= 1024 && M >= 128 && M <= 1024 && tiles >= 48 && tiles <= 512;
+  if (K > 768) return K <= 1024 && M >= 128 && M <= 1536 && tiles >= 48 && tiles <= 512;
   return K * tiles <= 768 * 256;
 }
 

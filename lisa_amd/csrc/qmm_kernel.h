@@ -585,8 +585,14 @@ __global__ __launch_bounds__(64 * WN) void qmm_kernel(QmmParams p) {
       const bool up = GU && blk >= SI / 2;
       const uint16_t* base = is_b ? (up ? bi2 : bi) : (up ? sc2 : sc);
       uint16_t* st = reinterpret_cast<uint16_t*>(smem + L::SB0 + (is_b ? L::SBA : 0) + (blk * 64 + lane) * 16);
-      if (sbrow[q] < (uint32_t)pad)
-        for (int g = 0; g < 8 - pad; ++g) st[pad + g] = base[sbrow[q] + g];
+      if (sbrow[q] < (uint32_t)pad) {
+        uint16_t v[7];  // (every load before the first store)
+#pragma unroll
+        for (int g = 0; g < 7; ++g) v[g] = base[sbrow[q] + (g < 8 - pad ? g : 7 - pad)];
+#pragma unroll
+        for (int g = 0; g < 7; ++g)
+          if (g < 8 - pad) st[pad + g] = v[g];
+      }
     }
     wait_lgkm0();
   }
