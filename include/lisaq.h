@@ -113,8 +113,8 @@ LISAQ_API int lisaq_quantized_matmul(void* stream, const void* x, const uint32_t
  * once.  The matvec: x staged in LDS, one to four output rows per wave (x or w
  * off 16 bytes: one wave per output row).  The matmul: the bf16 2/4-bit
  * matmul's kernel for bf16 and f16 where K is a multiple of 64 and of two
- * groups and the tensors are aligned for it (x and w 16 bytes, the others 4),
- * which splits K in a workspace of lisaq_quantized_matmul_workspace bytes
+ * groups, not a short one over few tiles (K <= 1024), and the tensors are
+ * aligned for it (x and w 16 bytes, the others 4), which splits K in a workspace of lisaq_quantized_matmul_workspace bytes
  * (256-byte aligned; without it the call runs unsplit).  Else, without a
  * workspace: matrix-core tiles of 64 x 64 or 128 x 128, for f32 of 64 x 64 or
  * 32 x 32, and 64 x 64 f32-FMA tiles for an x off 16 bytes. */
